@@ -125,7 +125,7 @@ class ImportanceArgs(ctypes.Structure):
 EXPORTS = (
     "akv_abi_version", "akv_last_error", "akv_struct_size",
     "akv_decode_workspace_bytes", "akv_decode_counter_bytes", "akv_decode_attn", "akv_decode_attn_noalloc",
-    "akv_quant_pack", "akv_dequant_unpack",
+    "akv_quant_pack", "akv_quant_workspace_bytes", "akv_quant_pack_ws", "akv_dequant_unpack",
     "akv_bitpack", "akv_bitunpack", "akv_importance_update",
     "akv_prefill_workspace_bytes", "akv_prefill_attn", "akv_select_demote", "akv_stream_read",
     "akv_timeline_words", "akv_timeline_fetch", "akv_timeline_clear",
@@ -159,6 +159,10 @@ def load() -> ctypes.CDLL:
     lib.akv_decode_attn_noalloc.argtypes = [ctypes.POINTER(DecodeArgs), _vp]
     lib.akv_quant_pack.restype = ctypes.c_int
     lib.akv_quant_pack.argtypes = [ctypes.POINTER(QuantArgs), _vp]
+    lib.akv_quant_workspace_bytes.restype = _i64
+    lib.akv_quant_workspace_bytes.argtypes = [ctypes.POINTER(QuantArgs)]
+    lib.akv_quant_pack_ws.restype = ctypes.c_int
+    lib.akv_quant_pack_ws.argtypes = [ctypes.POINTER(QuantArgs), _vp, _i64, _vp]
     lib.akv_dequant_unpack.restype = ctypes.c_int
     lib.akv_dequant_unpack.argtypes = [ctypes.POINTER(DequantArgs), _vp]
     lib.akv_bitpack.restype = ctypes.c_int
@@ -251,6 +255,18 @@ def workspace(nbytes: int, device, zero_prefix: int = 0) -> torch.Tensor:
     if zero_prefix > 0:
         ws[: min(int(zero_prefix), n)].zero_()
     return ws
+
+
+def quant_pack(a: QuantArgs, like: torch.Tensor, what: str) -> None:
+    """``akv_quant_pack_ws`` on the current stream of ``like``'s device, with scratch for the
+    forms that ask for some (long K blocks)."""
+    lib = load()
+    ref = ctypes.byref(a)
+    nbytes = lib.akv_quant_workspace_bytes(ref)
+    if nbytes < 0:
+        check(lib.akv_quant_pack(ref, None), what)
+    ws = workspace(nbytes, like.device) if nbytes > 0 else None
+    check(lib.akv_quant_pack_ws(ref, ptr(ws), nbytes if ws is not None else 0, stream_of(like)), what)
 
 
 class DecodeWorkspace:

@@ -45,7 +45,6 @@ class AffineQuantizer:
         nat.require_device(x)
         if bits not in (2, 3, 4, 8):
             raise NotImplementedError(f"the MI355X quantizer takes 2/3/4-bit (packed) or 8-bit (raw) codes, got {bits}")
-        lib = nat.load()
         if x.dim() != 3:
             raise ValueError("expected (H, N, D)")
         H, N, D = x.shape
@@ -81,7 +80,7 @@ class AffineQuantizer:
             a.v_codes, a.v_scale, a.v_zero = codes.data_ptr(), sc.data_ptr(), ze.data_ptr()
             if n_out:
                 a.v_oidx, a.v_odata = oidx.data_ptr(), odata.data_ptr()
-        nat.check(lib.akv_quant_pack(ctypes.byref(a), nat.stream_of(x)), "quantize")
+        nat.quant_pack(a, x, "quantize")
         res = {
             "scale": sc[0],
             "zero": ze[0],

@@ -108,7 +108,6 @@ def quantize_kv(k: torch.Tensor, v: torch.Tensor, bits_k: int = 3, bits_v: int =
 
     k, v: (B, Hkv, N, D) float16 / bfloat16 / float32 on the device."""
     nat.require_device(k, v, sel)
-    lib = nat.load()
     if k.shape != v.shape or k.dim() != 4:
         raise ValueError("k and v must both be (B, H, N, D)")
     k = nat.dev_contig(k)
@@ -150,7 +149,7 @@ def quantize_kv(k: torch.Tensor, v: torch.Tensor, bits_k: int = 3, bits_v: int =
     if n_out:
         a.k_oidx, a.v_oidx = koi.data_ptr(), voi.data_ptr()
         a.k_odata, a.v_odata = kod.data_ptr(), vod.data_ptr()
-    nat.check(lib.akv_quant_pack(ctypes.byref(a), nat.stream_of(k)), "quantize_kv")
+    nat.quant_pack(a, k, "quantize_kv")
     return WarmTier(kc, ks, kz, vc, vs, vz, bits_k, bits_v, block_t, group_v, D, koi, voi, kod, vod)
 
 

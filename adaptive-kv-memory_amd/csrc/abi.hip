@@ -504,13 +504,22 @@ int akv_decode_attn_noalloc(const akv_decode_args *a, void *stream) {
     return decode_run(a, pl, base, base + kScratchCtrBytes, stream);
 }
 
-int akv_quant_pack(const akv_quant_args *a, void *stream) {
+}  // extern "C"
+
+namespace {
+
+// Validation and the kernels' parameter block; *empty is set when there is nothing to do.
+int quant_params(const akv_quant_args *a, akv::QuantParams &p, bool *empty) {
+    *empty = false;
     if (!a) return fail(AKV_E_INVALID, "args is NULL");
     if (a->abi_version != AKV_ABI_VERSION) return fail(AKV_E_ABI, "ABI mismatch");
     if (a->D != 64 && a->D != 128) return fail(AKV_E_SHAPE, "head_dim %d unsupported (64 or 128)", a->D);
     if (a->B < 1 || a->H < 1 || a->n_src < 0 || a->n_sel < 0) return fail(AKV_E_SHAPE, "bad sizes");
     if (a->in_dtype < 0 || a->in_dtype > 2) return fail(AKV_E_DTYPE, "bad input dtype");
-    if (a->n_sel == 0) return ok();
+    if (a->n_sel == 0) {
+        *empty = true;
+        return ok();
+    }
     if (!a->sel && a->n_sel > a->n_src) return fail(AKV_E_SHAPE, "n_sel > n_src without indices");
     const bool affine = a->layout == AKV_QUANT_AFFINE;
     const bool kvq = a->layout == AKV_QUANT_KVQ;
@@ -532,7 +541,7 @@ int akv_quant_pack(const akv_quant_args *a, void *stream) {
         return fail(AKV_E_INVALID, "outlier outputs missing");
     for (const void *ptr : {(const void *)a->k_codes, (const void *)a->v_codes})
         if (ptr && !aligned16(ptr)) return fail(AKV_E_ALIGN, "code outputs must be 16-byte aligned");
-    akv::QuantParams p{};
+    p = akv::QuantParams{};
     p.B = a->B; p.H = a->H; p.D = a->D;
     p.in_dt = a->in_dtype;
     // arithmetic dtype and the scale clamp as that dtype rounds it
@@ -570,10 +579,39 @@ int akv_quant_pack(const akv_quant_args *a, void *stream) {
     p.k_row = p.pD * p.sbits_k / 8;
     p.v_row = p.pD * p.sbits_v / 8;
     p.nblk = (a->n_sel + p.T - 1) / p.T;
+    return AKV_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int64_t akv_quant_workspace_bytes(const akv_quant_args *a) {
+    akv::QuantParams p;
+    bool empty;
+    if (quant_params(a, p, &empty) != AKV_OK) return -1;
+    return empty ? 0 : align256(akv::quant_plan_ws(p) * 4);
+}
+
+int akv_quant_pack_ws(const akv_quant_args *a, void *workspace, int64_t workspace_bytes, void *stream) {
+    akv::QuantParams p;
+    bool empty;
+    const int rc = quant_params(a, p, &empty);
+    if (rc != AKV_OK || empty) return rc;
+    const int64_t need = akv::quant_plan_ws(p) * 4;
+    if (workspace && need > 0) {
+        if (workspace_bytes < need) return fail(AKV_E_WORKSPACE, "workspace of %lld bytes needed", (long long)need);
+        if (!aligned16(workspace)) return fail(AKV_E_ALIGN, "workspace must be 16-byte aligned");
+        p.ws = (float *)workspace;
+    } else {
+        p.nchunk = 0;
+    }
     hipError_t e = akv::quant_launch(p, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "quant launch");
     return ok();
 }
+
+int akv_quant_pack(const akv_quant_args *a, void *stream) { return akv_quant_pack_ws(a, nullptr, 0, stream); }
 
 int akv_dequant_unpack(const akv_dequant_args *a, void *stream) {
     if (!a) return fail(AKV_E_INVALID, "args is NULL");

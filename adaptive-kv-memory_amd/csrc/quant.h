@@ -28,8 +28,21 @@ struct QuantParams {
     void *v_codes, *v_scale, *v_zero;
     int64_t *k_oidx, *v_oidx;
     void *k_odata, *v_odata;
+    float *ws;                   // optional scratch: statistics partials, then outlier norms
+    int nchunk, chunk_tokens;    // long-block statistics chunks in ws (0: none)
+    int64_t norm_off;            // floats before the norms [B][nblk][2][H][D] in ws
 };
 
+// Scratch floats that let the long-block forms spread over the GPU (0: none needed);
+// fills nchunk, chunk_tokens and norm_off.
+int64_t quant_plan_ws(QuantParams &p);
 hipError_t quant_launch(const QuantParams &p, hipStream_t s);
+
+// quant_tile.hip
+bool quant_fast_eligible(const QuantParams &p);  // quant.hip
+bool quant_tile_eligible(const QuantParams &p);
+int quant_stat_chunks(const QuantParams &p, int *tokens);
+bool quant_norms_in_ws(const QuantParams &p);
+hipError_t quant_tile_launch(const QuantParams &p, hipStream_t s);
 
 }  // namespace akv

@@ -530,7 +530,7 @@ __global__ __launch_bounds__(256) void quant_fast_kernel(const QuantParams p) {
     }
 }
 
-static bool quant_fast_eligible(const QuantParams &p) {
+bool quant_fast_eligible(const QuantParams &p) {
     const bool al = (((uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.k_codes | (uintptr_t)p.v_codes |
                       (uintptr_t)p.k_scale | (uintptr_t)p.k_zero) & 15u) == 0;
     return al && p.in_dt == AKV_DT_F16 && p.ar_dt == AKV_DT_F16 && p.D == 128 && p.pD == 128 && p.T == 32 &&
@@ -546,13 +546,16 @@ static void launch_quant_fast(const QuantParams &p, dim3 grid, hipStream_t s) {
     else hipLaunchKernelGGL((quant_fast_kernel<BK, BV, 1>), grid, dim3(256), 0, s, p);
 }
 
+int64_t quant_plan_ws(QuantParams &p) {
+    p.nchunk = p.chunk_tokens = 0;
+    p.norm_off = 0;
+    if (quant_fast_eligible(p) || !quant_tile_eligible(p)) return 0;
+    p.nchunk = quant_stat_chunks(p, &p.chunk_tokens);
+    p.norm_off = (int64_t)p.B * p.H * p.nblk * p.nchunk * 2 * p.D;
+    return p.norm_off + (quant_norms_in_ws(p) ? (int64_t)p.B * p.nblk * 2 * p.H * p.D : 0);
+}
+
 hipError_t quant_launch(const QuantParams &p, hipStream_t s) {
-    hipError_t e;
-    if (p.n_out > 0) {
-        dim3 g((unsigned)p.nblk, p.B);
-        hipLaunchKernelGGL(outlier_select_kernel<AKV_DT_F32>, g, dim3(256), 0, s, p);
-        if ((e = hipGetLastError()) != hipSuccess) return e;
-    }
     dim3 grid((unsigned)((p.nblk + 3) / 4), p.H, p.B);
     if (quant_fast_eligible(p)) {
 #define AKV_QKV(a, c) \
@@ -561,6 +564,15 @@ hipError_t quant_launch(const QuantParams &p, hipStream_t s) {
         AKV_QKV(4, 3) AKV_QKV(4, 4)
 #undef AKV_QKV
         return hipGetLastError();
+    }
+    // inputs on 16-byte boundaries in the arithmetic's own dtype: whole tiles in registers;
+    // the rest (KVQuantizer's float32 arithmetic on 16-bit inputs or its symmetric branch,
+    // unaligned pointers) element by element
+    if (quant_tile_eligible(p)) return quant_tile_launch(p, s);
+    if (p.n_out > 0) {
+        hipLaunchKernelGGL(outlier_select_kernel<AKV_DT_F32>, dim3((unsigned)p.nblk, p.B), dim3(256), 0, s, p);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
     }
     if (p.ar_dt == AKV_DT_F16) hipLaunchKernelGGL(quant_kernel<AKV_DT_F16>, grid, dim3(256), 0, s, p);
     else if (p.ar_dt == AKV_DT_BF16) hipLaunchKernelGGL(quant_kernel<AKV_DT_BF16>, grid, dim3(256), 0, s, p);

@@ -212,6 +212,14 @@ typedef struct akv_quant_args {
  * step of triton_kernels.fused_quantize_evict (akv/triton_kernels.py:464-507). */
 int akv_quant_pack(const akv_quant_args *args, void *stream);
 
+/* The same call with device scratch: one K block of thousands of tokens (a prompt's
+ * demotion event) then spreads over the GPU instead of one workgroup per (batch, head),
+ * and so do its outlier norms.  akv_quant_workspace_bytes gives the bytes (0: none used; -1:
+ * invalid args); workspace NULL is akv_quant_pack.  The workspace needs no initial value
+ * and holds nothing between calls; calls that share one must not overlap. */
+int64_t akv_quant_workspace_bytes(const akv_quant_args *args);
+int akv_quant_pack_ws(const akv_quant_args *args, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* ------------------------------------------------------------- dequant */
 
 typedef struct akv_dequant_args {
