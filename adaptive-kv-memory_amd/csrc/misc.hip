@@ -75,6 +75,146 @@ __global__ __launch_bounds__(256) void dequant_kernel(const DequantParams p) {
     }
 }
 
+// ------------------------------------------------------- dequant, whole chunks
+// The same arithmetic for tiers whose rows, meta and outputs lie on vector boundaries
+// (head_dim a multiple of 32, groups of a multiple of 8): a thread owns 8 channels of
+// kDqTok tokens of one (batch, head) and one of K / V, with one load for the codes, one for
+// the scales and zeros (K: 16 bytes each; V and legacy: one value of the chunk's group) and
+// 16-byte stores; all its tokens' loads are in flight together.  HBM-bound: it writes what
+// the view holds and reads a fraction of that.  Before, each code, scale and zero was a load
+// of its own behind three 64-bit divisions per thread (dequant_kernel): 16,255 tokens x 8
+// heads of K and V at 3 bits 101 -> 32 us (2.5 TB/s, scattered to their positions); 3,969
+// tokens x 32 heads of legacy 2-bit rows 52 -> 12.8 us (2.9 TB/s).
+namespace {
+constexpr int kDqTok = 4;
+
+// the 8 codes of chunk ch8 of a packed row whose start is 4-byte aligned (8 with 8 bits)
+__device__ __forceinline__ void chunk_codes(const unsigned char *row, int ch8, int bits, uint32_t (&c)[8]) {
+    if (bits == 4) {
+        const uint32_t w = *(const uint32_t *)(row + 4 * ch8);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[i] = (w >> (8 * (i / 2) + ((i & 1) ? 0 : 4))) & 15u;
+    } else if (bits == 2) {
+        const uint32_t w = *(const uint16_t *)(row + 2 * ch8);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[i] = (w >> (8 * (i / 4) + 6 - 2 * (i & 3))) & 3u;
+    } else if (bits == 3) {  // 3 bytes, in one or two aligned words of the row
+        const int o = 3 * ch8;
+        const uint32_t *w = (const uint32_t *)row + o / 4;
+        const uint32_t lo = w[0], hi = (o & 3) > 1 ? w[1] : 0u;
+        const uint32_t x = (uint32_t)((((uint64_t)hi << 32) | lo) >> (8 * (o & 3)));
+        const uint32_t W = ((x & 0xFFu) << 16) | (x & 0xFF00u) | ((x >> 16) & 0xFFu);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[i] = (W >> (21 - 3 * i)) & 7u;
+    } else {
+        const u2 w = *(const u2 *)(row + 8 * ch8);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) c[i] = (w[i / 4] >> (8 * (i & 3))) & 0xFFu;
+    }
+}
+template <int OUT>
+__device__ __forceinline__ void store_chunk(void *out, int64_t o, const float (&v)[8]) {
+    if (OUT == AKV_DT_F32) {
+        *(f4 *)((float *)out + o) = (f4){v[0], v[1], v[2], v[3]};
+        *(f4 *)((float *)out + o + 4) = (f4){v[4], v[5], v[6], v[7]};
+    } else if (OUT == AKV_DT_F16) {
+        h8 x;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) x[i] = (_Float16)v[i];
+        *(h8 *)((_Float16 *)out + o) = x;
+    } else {
+        u4 x;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            x[i] = (uint32_t)f32_to_bf16_rne(v[2 * i]) | ((uint32_t)f32_to_bf16_rne(v[2 * i + 1]) << 16);
+        *(u4 *)((uint16_t *)out + o) = x;
+    }
+}
+}  // namespace
+
+template <bool AFFINE, int OUT>
+__global__ __launch_bounds__(256) void dequant_chunk_kernel(const DequantParams p) {
+    const int nch = p.D / 8, per = 256 / nch;  // tokens of one pass of the workgroup
+    const int ch8 = threadIdx.x % nch, tr = threadIdx.x / nch;
+    const bool is_k = p.k_out && blockIdx.z == 0;
+    void *out = is_k ? p.k_out : p.v_out;
+    const int bits = is_k ? p.bits_k : p.bits_v, row_bytes = is_k ? p.kc_row : p.vc_row;
+    const unsigned char *codes = (const unsigned char *)(is_k ? p.kc : p.vc);
+    const void *sc = is_k ? p.ks : p.vs, *ze = is_k ? p.kz : p.vz;
+    const int64_t bh = blockIdx.y, t0 = (int64_t)blockIdx.x * per * kDqTok + tr;
+    if (tr >= per) return;
+    const int sym = AFFINE ? 0 : p.sym_flags ? p.sym_flags[is_k ? 0 : 1] : p.legacy_sym;
+    const float half_max = (float)(((1 << bits) - 1) / 2);
+    uint32_t c[kDqTok][8];
+    h8 s8[kDqTok], z8[kDqTok];
+    float sf[kDqTok], zf[kDqTok];
+    int64_t orow[kDqTok], blk[kDqTok];
+#pragma unroll
+    for (int i = 0; i < kDqTok; ++i) {
+        const int64_t t = min(t0 + (int64_t)i * per, p.n_warm - 1), row = bh * p.tok_stride + t;
+        orow[i] = p.out_slot ? bh * p.out_tokens + p.out_slot[t] : bh * p.n_warm + t;
+        chunk_codes(codes + row * row_bytes, ch8, bits, c[i]);
+        if (AFFINE) {
+            blk[i] = p.blk_of ? (int64_t)p.blk_of[t] : (int64_t)((uint32_t)t / (uint32_t)p.T);
+            if (is_k) {
+                const int64_t mi = (bh * p.nblk + blk[i]) * p.D + 8 * ch8;
+                s8[i] = *(const h8 *)((const _Float16 *)sc + mi);
+                z8[i] = *(const h8 *)((const _Float16 *)ze + mi);
+            } else {
+                const int64_t mi = row * (p.D / p.Gv) + 8 * ch8 / p.Gv;
+                const _Float16 s = ((const _Float16 *)sc)[mi], z = ((const _Float16 *)ze)[mi];
+                s8[i] = (h8){s, s, s, s, s, s, s, s};
+                z8[i] = (h8){z, z, z, z, z, z, z, z};
+            }
+        } else {
+            const int64_t mi = row * p.lg + 8 * ch8 / p.gs;
+            sf[i] = load_as_f32(sc, mi, p.meta_dt);
+            zf[i] = sym ? 0.f : load_as_f32(ze, mi, p.meta_dt);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < kDqTok; ++i) {
+        const int64_t t = t0 + (int64_t)i * per;
+        if (t >= p.n_warm) break;
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            if (AFFINE) {
+                _Float16 x = (_Float16)(uint16_t)c[i][e] * s8[i][e];
+                x = x + z8[i][e];
+                v[e] = (float)x;
+            } else if (sym) {
+                v[e] = ((float)c[i][e] - half_max) * sf[i];
+            } else {
+                const float x = (float)c[i][e] * sf[i];
+                v[e] = x + zf[i];
+            }
+        }
+        if (AFFINE && p.n_out > 0) {
+            const int64_t *oi = (is_k ? p.k_oidx : p.v_oidx) + ((bh / p.Hkv) * p.nblk + blk[i]) * p.n_out;
+            const _Float16 *od = (const _Float16 *)(is_k ? p.k_odata : p.v_odata) + (bh * p.tok_stride + t) * p.n_out;
+            for (int j = 0; j < p.n_out; ++j) {
+                const int d = (int)oi[j];
+                if (d / 8 != ch8) continue;
+                const float x = (float)od[j];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (d % 8 == e) v[e] = x;
+            }
+        }
+        store_chunk<OUT>(out, orow[i] * p.D + 8 * ch8, v);
+    }
+}
+
+// Vector boundaries everywhere, a chunk inside one group, 32-bit token arithmetic.
+static bool dequant_chunk_eligible(const DequantParams &p) {
+    const uintptr_t al = (uintptr_t)p.kc | (uintptr_t)p.vc | (uintptr_t)p.ks | (uintptr_t)p.kz | (uintptr_t)p.k_out |
+                         (uintptr_t)p.v_out;
+    const int g = p.kind == AKV_WARM_AFFINE ? p.Gv : p.gs;
+    return (al & 15u) == 0 && p.D % 32 == 0 && p.D <= 2048 && g % 8 == 0 && p.kc_row % 8 == 0 && p.vc_row % 8 == 0 &&
+           p.nbh <= 65535 && p.n_warm < ((int64_t)1 << 31);
+}
+
 // ------------------------------------------------------------------ bitpack
 // One thread per (row, group of 8 codes); bytes past the packed row are not written.
 __global__ __launch_bounds__(256) void bitpack_kernel(const unsigned char *codes, unsigned char *packed, int64_t rows,
@@ -486,7 +626,20 @@ hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t
 
 hipError_t dequant_launch(const DequantParams &p, hipStream_t s) {
     const int64_t tasks = (int64_t)p.nbh * p.n_warm * (p.D / 8);
-    if (tasks == 0) return hipSuccess;
+    if (tasks == 0 || (!p.k_out && !p.v_out)) return hipSuccess;
+    if (dequant_chunk_eligible(p)) {
+        const int per = 256 / (p.D / 8) * kDqTok;
+        const dim3 grid((unsigned)((p.n_warm + per - 1) / per), (unsigned)p.nbh, (p.k_out != nullptr) + (p.v_out != nullptr));
+#define AKV_DQ(aff, dt) hipLaunchKernelGGL((dequant_chunk_kernel<aff, dt>), grid, dim3(256), 0, s, p)
+        if (p.kind == AKV_WARM_AFFINE) {
+            if (p.out_dt == AKV_DT_F16) AKV_DQ(true, AKV_DT_F16);
+            else AKV_DQ(true, AKV_DT_F32);
+        } else if (p.out_dt == AKV_DT_F16) AKV_DQ(false, AKV_DT_F16);
+        else if (p.out_dt == AKV_DT_BF16) AKV_DQ(false, AKV_DT_BF16);
+        else AKV_DQ(false, AKV_DT_F32);
+#undef AKV_DQ
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(dequant_kernel, dim3((unsigned)((tasks + 255) / 256)), dim3(256), 0, s, p);
     return hipGetLastError();
 }
