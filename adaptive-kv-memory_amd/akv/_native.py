@@ -127,6 +127,7 @@ EXPORTS = (
     "akv_decode_workspace_bytes", "akv_decode_counter_bytes", "akv_decode_attn", "akv_decode_attn_noalloc",
     "akv_quant_pack", "akv_quant_workspace_bytes", "akv_quant_pack_ws", "akv_dequant_unpack",
     "akv_bitpack", "akv_bitunpack", "akv_importance_update",
+    "akv_importance_workspace_bytes", "akv_importance_update_ws",
     "akv_prefill_workspace_bytes", "akv_prefill_attn", "akv_select_demote", "akv_stream_read",
     "akv_timeline_words", "akv_timeline_fetch", "akv_timeline_clear",
 )
@@ -171,6 +172,10 @@ def load() -> ctypes.CDLL:
     lib.akv_bitunpack.argtypes = [_vp, _vp, _i64, _i32, _i32, _i32, _vp]
     lib.akv_importance_update.restype = ctypes.c_int
     lib.akv_importance_update.argtypes = [ctypes.POINTER(ImportanceArgs), _vp]
+    lib.akv_importance_workspace_bytes.restype = _i64
+    lib.akv_importance_workspace_bytes.argtypes = [ctypes.POINTER(ImportanceArgs)]
+    lib.akv_importance_update_ws.restype = ctypes.c_int
+    lib.akv_importance_update_ws.argtypes = [ctypes.POINTER(ImportanceArgs), _vp, _i64, _vp]
     lib.akv_prefill_workspace_bytes.restype = _i64
     lib.akv_prefill_workspace_bytes.argtypes = [ctypes.POINTER(PrefillArgs)]
     lib.akv_prefill_attn.restype = ctypes.c_int
@@ -267,6 +272,16 @@ def quant_pack(a: QuantArgs, like: torch.Tensor, what: str) -> None:
         check(lib.akv_quant_pack(ref, None), what)
     ws = workspace(nbytes, like.device) if nbytes > 0 else None
     check(lib.akv_quant_pack_ws(ref, ptr(ws), nbytes if ws is not None else 0, stream_of(like)), what)
+
+
+def importance_update(a: ImportanceArgs, like: torch.Tensor, what: str) -> None:
+    """``akv_importance_update_ws`` on the current stream of ``like``'s device, with scratch for
+    the calls that ask for some (many query rows)."""
+    lib = load()
+    ref = ctypes.byref(a)
+    nbytes = max(0, lib.akv_importance_workspace_bytes(ref))  # < 0: the call itself reports it
+    ws = workspace(nbytes, like.device) if nbytes > 0 else None
+    check(lib.akv_importance_update_ws(ref, ptr(ws), nbytes, stream_of(like)), what)
 
 
 class DecodeWorkspace:

@@ -15,7 +15,6 @@ with zeros when the context grows (akv/importance.py:117-123).
 """
 from __future__ import annotations
 
-import ctypes
 import logging
 from dataclasses import dataclass
 from enum import Enum
@@ -61,7 +60,6 @@ def accumulate(scores: torch.Tensor, attention_weights: torch.Tensor, decay: flo
     (truncated / zero-padded to n); q_window > 0 sums only the last q_window queries and
     pool_kernel > 1 average-pools the per-key sum first (OBSERVATION_WINDOW)."""
     nat.require_device(scores, attention_weights)
-    lib = nat.load()
     B, H, M, N = attention_weights.shape
     attn = attention_weights
     if attn.dtype not in (torch.float16, torch.bfloat16, torch.float32):
@@ -77,7 +75,7 @@ def accumulate(scores: torch.Tensor, attention_weights: torch.Tensor, decay: flo
     a.decay = float(decay)
     a.q_window = int(q_window)
     a.pool_kernel = int(pool_kernel)
-    nat.check(lib.akv_importance_update(ctypes.byref(a), nat.stream_of(scores)), "importance update")
+    nat.importance_update(a, scores, "importance update")
     return scores
 
 

@@ -80,7 +80,6 @@ def fused_importance_update(
     weights, truncated / zero-padded to len(scores); in place, returned
     (akv/triton_ops.py:604-650, torch-path semantics)."""
     nat.require_device(attention_weights, scores)
-    lib = nat.load()
     B, H, M, N = attention_weights.shape
     attn = attention_weights
     if attn.dtype not in (torch.float16, torch.bfloat16, torch.float32):
@@ -96,7 +95,7 @@ def fused_importance_update(
     a.scores = buf.data_ptr()
     a.n_scores = buf.numel()
     a.decay = float(decay)
-    nat.check(lib.akv_importance_update(ctypes.byref(a), nat.stream_of(buf)), "fused_importance_update")
+    nat.importance_update(a, buf, "fused_importance_update")
     if not direct:
         scores.copy_(buf.view_as(scores))
     return scores

@@ -789,24 +789,44 @@ int akv_select_demote(const float *scores, int64_t rows, int64_t len, int64_t n_
     return ok();
 }
 
-int akv_importance_update(const akv_importance_args *a, void *stream) {
+static int importance_params(const akv_importance_args *a, akv::ImportanceParams *p) {
     if (!a) return fail(AKV_E_INVALID, "args is NULL");
     if (a->abi_version != AKV_ABI_VERSION) return fail(AKV_E_ABI, "ABI mismatch");
     if (a->attn_dtype < 0 || a->attn_dtype > 2) return fail(AKV_E_DTYPE, "bad attention dtype");
     if (a->B < 1 || a->H < 1 || a->M < 1 || a->N < 0 || a->n_scores < 0) return fail(AKV_E_SHAPE, "bad sizes");
     if ((a->n_scores > 0 && !a->scores) || (a->N > 0 && !a->attn)) return fail(AKV_E_INVALID, "null pointer");
-    akv::ImportanceParams p{};
-    p.attn = a->attn; p.attn_dt = a->attn_dtype;
-    p.B = a->B; p.H = a->H; p.M = a->M; p.N = a->N;
-    p.scores = a->scores; p.n_scores = a->n_scores; p.decay = a->decay;
     if (a->q_window < 0 || a->pool_kernel < 0 || a->pool_kernel > 64)
         return fail(AKV_E_SHAPE, "q_window must be >= 0 and pool_kernel in [0, 64]");
-    p.m0 = (a->q_window > 0 && a->q_window < a->M) ? a->M - a->q_window : 0;
+    *p = akv::ImportanceParams{};
+    p->attn = a->attn; p->attn_dt = a->attn_dtype;
+    p->B = a->B; p->H = a->H; p->M = a->M; p->N = a->N;
+    p->scores = a->scores; p->n_scores = a->n_scores; p->decay = a->decay;
+    p->m0 = (a->q_window > 0 && a->q_window < a->M) ? a->M - a->q_window : 0;
     // the reference pools only when kv_len > kernel (akv/importance.py:111)
-    p.pool = (a->pool_kernel > 1 && a->N > a->pool_kernel) ? a->pool_kernel : 1;
-    hipError_t e = akv::importance_launch(p, (hipStream_t)stream);
+    p->pool = (a->pool_kernel > 1 && a->N > a->pool_kernel) ? a->pool_kernel : 1;
+    return AKV_OK;
+}
+
+int64_t akv_importance_workspace_bytes(const akv_importance_args *a) {
+    akv::ImportanceParams p;
+    return importance_params(a, &p) == AKV_OK ? akv::importance_workspace_bytes(p) : -1;
+}
+
+int akv_importance_update_ws(const akv_importance_args *a, void *workspace, int64_t workspace_bytes, void *stream) {
+    akv::ImportanceParams p;
+    int rc = importance_params(a, &p);
+    if (rc != AKV_OK) return rc;
+    const int64_t need = akv::importance_workspace_bytes(p);
+    if (workspace && workspace_bytes < need)
+        return fail(AKV_E_WORKSPACE, "workspace of %lld bytes needed", (long long)need);
+    if (workspace && !aligned16(workspace)) return fail(AKV_E_ALIGN, "workspace must be 16-byte aligned");
+    hipError_t e = akv::importance_launch(p, (float *)workspace, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "importance launch");
     return ok();
+}
+
+int akv_importance_update(const akv_importance_args *a, void *stream) {
+    return akv_importance_update_ws(a, nullptr, 0, stream);
 }
 
 }  // extern "C"

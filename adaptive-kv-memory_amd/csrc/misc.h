@@ -44,7 +44,9 @@ hipError_t dequant_launch(const DequantParams &p, hipStream_t s);
 hipError_t stream_read_launch(const void *p, int64_t bytes, uint32_t *sink, hipStream_t s);
 hipError_t bitpack_launch(const void *codes, void *packed, int64_t rows, int dim, int bits, int prow, hipStream_t s);
 hipError_t bitunpack_launch(const void *packed, void *codes, int64_t rows, int prow, int dim, int bits, hipStream_t s);
-hipError_t importance_launch(const ImportanceParams &p, hipStream_t s);
+// part: importance_workspace_bytes() bytes for calls that split the query sum, or NULL.
+int64_t importance_workspace_bytes(const ImportanceParams &p);
+hipError_t importance_launch(const ImportanceParams &p, float *part, hipStream_t s);
 // bytes (a multiple of 16) of device memory at p set to zero by a kernel on s.
 hipError_t zero_fill_launch(void *p, int64_t bytes, hipStream_t s);
 // Demote selection: per row, the n smallest of `len` fp32 scores with positions [0, pf) and

@@ -346,6 +346,128 @@ __global__ __launch_bounds__(64 * RG) void importance_rows_kernel(const Importan
     p.scores[n] = sc;
 }
 
+// Many query rows (a prefill's weights): the sum over queries is split across workgroups.
+// HBM-bound: B*H*M*N weights are read once and everything else is small.  A wave owns
+// 64 x kV consecutive keys of every 4th query of its workgroup's range, each lane one
+// 16-byte load (kV keys) per (batch, head) row, 8 rows in flight; the four waves' sums and
+// one partial row per workgroup go to a workspace that importance_finish_kernel adds,
+// pools and folds into the scores.  Rows of odd length put the loads off 16 bytes, which
+// global loads allow; the lane across the row's end loads the row's last kV keys instead and
+// keeps those that are its own.  Per query the (batch, head) rows go to two accumulators
+// in turn, then the mean, then the queries in blocks: the association of
+// importance_rows_kernel with the query sum split.  32 heads x 256 queries x 8,191 keys in
+// bf16 (134 MB): 299 -> 26.6 us (5.0 TB/s); with 7-key pooling 4,888 -> 28.4 us.
+typedef u4 u4_any __attribute__((aligned(2)));
+template <int DT>
+struct ImpVec {
+    static constexpr int kV = DT == AKV_DT_F32 ? 4 : 8;
+    static __device__ __forceinline__ void add(u4 w, float (&acc)[kV]) {
+        if constexpr (DT == AKV_DT_F32) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t e = w[i];  // a copy: __builtin_bit_cast of a vector's element reads element 0
+                acc[i] += __builtin_bit_cast(float, e);
+            }
+        } else if constexpr (DT == AKV_DT_BF16) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                acc[2 * i] += __builtin_bit_cast(float, w[i] << 16);
+                acc[2 * i + 1] += __builtin_bit_cast(float, w[i] & 0xFFFF0000u);
+            }
+        } else {
+            const h8 x = __builtin_bit_cast(h8, w);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) acc[i] += (float)x[i];
+        }
+    }
+};
+constexpr int kImpWaves = 4, kImpMinQueries = 8;
+template <int DT>
+__global__ __launch_bounds__(64 * kImpWaves) void importance_part_kernel(const ImportanceParams p, float *part,
+                                                                         int64_t q_per) {
+    constexpr int kV = ImpVec<DT>::kV, kTile = 64 * kV, kSize = DT == AKV_DT_F32 ? 4 : 2;
+    __shared__ float red[kImpWaves][kTile];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t n0 = (int64_t)blockIdx.x * kTile + lane * kV, base = min(n0, p.N - kV);
+    const int64_t bhn = p.B * p.H, bh_bytes = p.M * p.N * kSize;
+    const int64_t q0 = p.m0 + (int64_t)blockIdx.y * q_per, q1 = min(p.M, q0 + q_per);
+    float imp[kV];
+#pragma unroll
+    for (int i = 0; i < kV; ++i) imp[i] = 0.f;
+    for (int64_t m = q0 + w; m < q1; m += kImpWaves) {
+        const char *row = (const char *)p.attn + (m * p.N + base) * kSize;
+        float a0[kV], a1[kV];
+#pragma unroll
+        for (int i = 0; i < kV; ++i) a0[i] = a1[i] = 0.f;
+        int64_t bh = 0;
+        for (; bh + 8 <= bhn; bh += 8) {
+            u4 x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = *(const u4_any *)(row + (bh + j) * bh_bytes);
+#pragma unroll
+            for (int j = 0; j < 8; j += 2) {
+                ImpVec<DT>::add(x[j], a0);
+                ImpVec<DT>::add(x[j + 1], a1);
+            }
+        }
+        for (; bh < bhn; ++bh) ImpVec<DT>::add(*(const u4_any *)(row + bh * bh_bytes), a0);
+#pragma unroll
+        for (int i = 0; i < kV; ++i) imp[i] += (a0[i] + a1[i]) / (float)bhn;
+    }
+#pragma unroll
+    for (int i = 0; i < kV; ++i) red[w][lane * kV + i] = imp[i];
+    __syncthreads();
+    // entry (lane, i) is key base + i; a key two lanes hold is written by its owner
+    for (int t = threadIdx.x; t < kTile; t += 64 * kImpWaves) {
+        float s = red[0][t];
+#pragma unroll
+        for (int r = 1; r < kImpWaves; ++r) s += red[r][t];
+        const int64_t own = (int64_t)blockIdx.x * kTile + t / kV * kV;
+        const int64_t n = min(own, p.N - kV) + t % kV;
+        if (own < p.N && n >= own) part[(int64_t)blockIdx.y * p.N + n] = s;
+    }
+}
+// One workgroup per 64 scores: its 4 waves add the partials of a quarter of the query blocks
+// each (8 loads in flight), over the tile and the pooling halo.
+__global__ __launch_bounds__(256) void importance_finish_kernel(const ImportanceParams p, const float *part, int nq) {
+    __shared__ float red[4][64 + kImpMaxPool];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t n0 = (int64_t)blockIdx.x * 64;
+    const int pad = p.pool / 2, width = 64 + p.pool - 1, per = (nq + 3) / 4;
+    const int c0 = min(nq, per * w), c1 = min(nq, c0 + per);
+    for (int i = lane; i < width; i += 64) {
+        const int64_t n = n0 - pad + i;
+        float s = 0.f;
+        if (n >= 0 && n < p.N) {
+            int c = c0;
+            for (; c + 8 <= c1; c += 8) {
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = part[(int64_t)(c + j) * p.N + n];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) s += x[j];
+            }
+            for (; c < c1; ++c) s += part[(int64_t)c * p.N + n];
+        }
+        red[w][i] = s;
+    }
+    __syncthreads();
+    const int64_t n = n0 + lane;
+    if (w != 0 || n >= p.n_scores) return;
+    float imp = 0.f;
+    for (int j = 0; j < p.pool; ++j) {
+        float s = red[0][lane + j];
+#pragma unroll
+        for (int r = 1; r < 4; ++r) s += red[r][lane + j];
+        imp += s;
+    }
+    if (p.pool > 1) imp = imp / (float)p.pool;
+    if (n >= p.N) imp = 0.f;
+    float sc = p.scores[n] * p.decay;
+    sc = sc + imp;
+    p.scores[n] = sc;
+}
+
 // ------------------------------------------------------------ demote selection
 // One workgroup (1024 threads) per row.  Scores become order-preserving 32-bit
 // keys (-0 as +0, NaN above +inf, protected positions = +inf); a 4-pass radix
@@ -685,8 +807,40 @@ hipError_t stream_read_launch(const void *p, int64_t bytes, uint32_t *sink, hipS
     hipLaunchKernelGGL(stream_read_kernel, dim3(2048), dim3(256), 0, s, (const u4 *)p, n16, sink);
     return hipGetLastError();
 }
-hipError_t importance_launch(const ImportanceParams &p, hipStream_t s) {
+// Query blocks of importance_part_kernel (0: the one-launch kernels); about four workgroups
+// per compute unit, each wave at least one query.  The second launch has to pay: without
+// pooling one launch takes 4.1-5.6 us at 4 query rows and 6.5-8.7 us at 8 (700 to 8,191 keys,
+// 8 to 32 heads) against 5.8-7.1 us split at any count up to 16; with pooling 4.1-10.8 us at
+// one row and 6.3-20.7 us at two against 5.8-6.9 us.
+static int64_t importance_q_blocks(const ImportanceParams &p, int64_t *q_per) {
+    const int64_t q = p.M - p.m0, kv = p.attn_dt == AKV_DT_F32 ? 4 : 8;
+    if (q < (p.pool > 1 ? 2 : kImpMinQueries) || p.N < kv || p.n_scores == 0) return 0;
+    const int64_t tiles = (p.N + 64 * kv - 1) / (64 * kv);
+    const int64_t want = max((int64_t)1, min((q + kImpWaves - 1) / kImpWaves, 1024 / tiles));
+    *q_per = ((q + want - 1) / want + kImpWaves - 1) / kImpWaves * kImpWaves;
+    const int64_t nq = (q + *q_per - 1) / *q_per;
+    return nq <= 65535 ? nq : 0;
+}
+int64_t importance_workspace_bytes(const ImportanceParams &p) {
+    int64_t q_per;
+    return importance_q_blocks(p, &q_per) * p.N * 4;
+}
+hipError_t importance_launch(const ImportanceParams &p, float *part, hipStream_t s) {
     if (p.n_scores == 0) return hipSuccess;
+    int64_t q_per = 0;
+    const int64_t nq = part ? importance_q_blocks(p, &q_per) : 0;
+    if (nq > 0) {
+        const int64_t kv = p.attn_dt == AKV_DT_F32 ? 4 : 8;
+        const dim3 grid((unsigned)((p.N + 64 * kv - 1) / (64 * kv)), (unsigned)nq);
+#define AKV_IMP(dt) hipLaunchKernelGGL(importance_part_kernel<dt>, grid, dim3(64 * kImpWaves), 0, s, p, part, q_per)
+        if (p.attn_dt == AKV_DT_F32) AKV_IMP(AKV_DT_F32);
+        else if (p.attn_dt == AKV_DT_F16) AKV_IMP(AKV_DT_F16);
+        else AKV_IMP(AKV_DT_BF16);
+#undef AKV_IMP
+        hipLaunchKernelGGL(importance_finish_kernel, dim3((unsigned)((p.n_scores + 63) / 64)), dim3(256), 0, s, p,
+                           part, (int)nq);
+        return hipGetLastError();
+    }
     if (p.pool <= 1) {
         const unsigned tiles = (unsigned)((p.n_scores + kImpKeys - 1) / kImpKeys);
         const int64_t rows = p.B * p.H * (p.M - p.m0);

@@ -283,6 +283,13 @@ typedef struct akv_importance_args {
  * the last q_window queries summed, then avg_pool1d(kernel, stride 1, padding kernel // 2). */
 int akv_importance_update(const akv_importance_args *args, void *stream);
 
+/* The same with device scratch (16-byte aligned) for calls of many query rows, whose sum over
+ * queries is then split over workgroups.  akv_importance_workspace_bytes gives the bytes (0:
+ * none used; -1: invalid args); workspace NULL is akv_importance_update.  The workspace needs
+ * no initial value. */
+int64_t akv_importance_workspace_bytes(const akv_importance_args *args);
+int akv_importance_update_ws(const akv_importance_args *args, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* --------------------------------------------------------------- prefill */
 
 typedef struct akv_prefill_args {
