@@ -469,12 +469,24 @@ __global__ __launch_bounds__(256) void importance_finish_kernel(const Importance
 }
 
 // ------------------------------------------------------------ demote selection
-// One workgroup (1024 threads) per row.  Scores become order-preserving 32-bit
-// keys (-0 as +0, NaN above +inf, protected positions = +inf); a 4-pass radix
-// select (8 bits per pass, per-wave LDS histograms) finds the key tau of the
-// n-th smallest and how many tau-valued elements to take; a block-wide scan of
-// per-thread counts over contiguous chunks then writes the selected indices in
-// ascending order (equal keys: lowest index first).
+// One workgroup (1024 threads) per row; latency-bound, so few passes over the keys.  Scores
+// become order-preserving 32-bit keys (-0 as +0, NaN above +inf, protected positions =
+// +inf).  Wave w owns the contiguous elements [w seg, (w + 1) seg), 64 per slot; its keys
+// are read once and kept on chip: slots 0-31 in registers, slots 32-63 in LDS (128 KiB;
+// 64 registers of keys spill at 1024 threads).  Rows past 65,536 re-read the row.
+//   1. smallest and largest finite key, finite and +inf counts (a selection that reaches
+//      past the finite keys is settled here: the keys left are +inf and NaN alone);
+//   2. a histogram of 2048 equal bins over that range finds the bin of the n-th smallest --
+//      bins of the range, not of the leading bits, so that scores of one magnitude spread
+//      over many bins instead of colliding on a few LDS addresses, and a row of equal
+//      scores needs no histogram; lanes that share the first lane's bin add once;
+//   3. at most 2048 keys of that bin go to a list, on which the remaining bits are refined;
+//   4. the selected indices are written in ascending order (equal keys: lowest index
+//      first) from per-wave counts and ballots.
+// The radix select before it made four histogram passes over 64 slots whatever the row's
+// length, with one LDS address per lane: uniform scores, 1 x 140 45 -> 7.5 us, 1 x 2,049
+// 46 -> 9.0, 1 x 16,383 49 -> 19.7, 16 x 65,536 67 -> 53, 1 x 131,071 371 -> 150; equal
+// scores (a prompt's, all new) 1 x 16,383 87 -> 11.7 us.
 namespace {
 __device__ __forceinline__ uint32_t order_key(float f) {
     uint32_t u = __builtin_bit_cast(uint32_t, f);
@@ -483,95 +495,13 @@ __device__ __forceinline__ uint32_t order_key(float f) {
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 constexpr uint32_t kKeyInf = 0xFF800000u;  // order_key(+inf)
-}  // namespace
-
-__global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64_t len, int64_t n, int64_t pf,
-                                                      int64_t pl, int64_t *out) {
-    __shared__ uint32_t hist[16][256];
-    __shared__ uint32_t tot[256];
-    __shared__ uint32_t cnt_lt[1024], cnt_eq[1024];
-    __shared__ uint32_t s_prefix, s_k;
-    const int tid = threadIdx.x, wave = tid >> 6;
-    const float *srow = scores + (int64_t)blockIdx.x * len;
-    int64_t *orow = out + (int64_t)blockIdx.x * n;
-    const int64_t rec = len - pl > 0 ? len - pl : 0;
-    auto key = [&](int64_t i) -> uint32_t { return (i < pf || i >= rec) ? kKeyInf : order_key(srow[i]); };
-    if (tid == 0) {
-        s_prefix = 0u;
-        s_k = (uint32_t)n;  // rank (1-based) of the key to find among the remaining candidates
-    }
-    for (int pass = 0; pass < 4; ++pass) {
-        const int shift = 24 - 8 * pass;
-        for (int i = tid; i < 16 * 256; i += 1024) (&hist[0][0])[i] = 0u;
-        __syncthreads();
-        const uint32_t prefix = s_prefix;
-        const uint32_t hmask = pass == 0 ? 0u : (0xFFFFFFFFu << (shift + 8));
-        for (int64_t i = tid; i < len; i += 1024) {
-            const uint32_t k = key(i);
-            if ((k & hmask) == prefix) atomicAdd(&hist[wave][(k >> shift) & 255u], 1u);
-        }
-        __syncthreads();
-        if (tid < 256) {
-            uint32_t t = 0;
-#pragma unroll
-            for (int w = 0; w < 16; ++w) t += hist[w][tid];
-            tot[tid] = t;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            uint32_t k = s_k, cum = 0;
-            int b = 0;
-            for (; b < 255; ++b) {
-                if (cum + tot[b] >= k) break;
-                cum += tot[b];
-            }
-            s_k = k - cum;
-            s_prefix = prefix | ((uint32_t)b << shift);
-        }
-        __syncthreads();
-    }
-    const uint32_t tau = s_prefix, take_eq = s_k;  // take the first take_eq elements equal to tau
-    // per-thread contiguous chunk counts, then exclusive scans
-    const int64_t chunk = (len + 1023) / 1024;
-    const int64_t c0 = (int64_t)tid * chunk, c1 = c0 + chunk < len ? c0 + chunk : len;
-    uint32_t lt = 0, eq = 0;
-    for (int64_t i = c0; i < c1; ++i) {
-        const uint32_t k = key(i);
-        lt += k < tau;
-        eq += k == tau;
-    }
-    cnt_lt[tid] = lt;
-    cnt_eq[tid] = eq;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {  // inclusive scans (Hillis-Steele)
-        const uint32_t a = tid >= off ? cnt_lt[tid - off] : 0u, e = tid >= off ? cnt_eq[tid - off] : 0u;
-        __syncthreads();
-        cnt_lt[tid] += a;
-        cnt_eq[tid] += e;
-        __syncthreads();
-    }
-    uint32_t lt_before = cnt_lt[tid] - lt, eq_before = cnt_eq[tid] - eq;
-    for (int64_t i = c0; i < c1; ++i) {
-        const uint32_t k = key(i);
-        if (k < tau) {
-            const uint32_t pos = lt_before + (eq_before < take_eq ? eq_before : take_eq);
-            orow[pos] = i;
-            ++lt_before;
-        } else if (k == tau) {
-            if (eq_before < take_eq) orow[lt_before + eq_before] = i;
-            ++eq_before;
-        }
-    }
+constexpr int kSelRegSlots = 32, kSelBins = 2048, kSelList = 2048;
+// LDS words: bins, list, per-wave scratch of the reductions and scans (5 x 16), then the LDS slots
+constexpr int kSelHeadWords = kSelBins + kSelList + 5 * 16;
+constexpr int sel_lds_bytes(int slots) {
+    return 4 * (kSelHeadWords + (slots > kSelRegSlots ? (slots - kSelRegSlots) * 1024 : 0));
 }
-
-// Rows of up to 65536 scores: the same selection with the keys read once and
-// kept on chip (element tid + 1024 j in slot j of thread tid): slots 0-31 in
-// registers, slots 32-63 in LDS (128 KiB, one 4 KiB row per slot, so a slot's
-// reads are conflict-free) -- all 64 in registers spilled 30 VGPRs to scratch at
-// 1024 threads.  In the first pass (sign and exponent bits, which cluster) the two
-// most common digits of a wave are added as groups (one LDS atomic each) before the
-// per-lane atomics; the digit searches and the output positions use wave scans (the
-// positions from per-(slot, wave) counts scanned in element order).
+static_assert(sel_lds_bytes(64) <= 160 * 1024, "select keys exceed the LDS");
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, int lane) {
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
@@ -580,151 +510,214 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x, int lane) {
     }
     return x;
 }
-constexpr int kSelSlots = 64, kSelRegSlots = 32;
-// dynamic LDS of select_reg_kernel: hist[16][256], tot[256], cnt_lt[1024], cnt_eq[1024],
-// s_prefix, s_k (padded to 16 bytes), then the LDS key slots [32][1024]
-constexpr int kSelLdsWords = 16 * 256 + 256 + 2 * 1024 + 4 + (kSelSlots - kSelRegSlots) * 1024;
-constexpr int kSelLdsBytes = kSelLdsWords * 4;
-static_assert(kSelLdsBytes <= 160 * 1024, "select keys exceed the LDS");
-__global__ __launch_bounds__(1024) void select_reg_kernel(const float *scores, int64_t len, int64_t n, int64_t pf,
-                                                          int64_t pl, int64_t *out) {
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+}  // namespace
+
+// SLOTS 0: the row stays in memory.
+template <int SLOTS>
+__global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64_t len, int64_t n, int64_t pf,
+                                                      int64_t pl, int64_t *out) {
     extern __shared__ __align__(16) uint32_t sel_lds[];
-    uint32_t(*hist)[256] = (uint32_t(*)[256])sel_lds;
-    uint32_t *tot = sel_lds + 16 * 256;
-    uint32_t *cnt_lt = tot + 256, *cnt_eq = cnt_lt + 1024;
-    uint32_t &s_prefix = cnt_eq[1024], &s_k = cnt_eq[1025];
-    uint32_t *key_lds = cnt_eq + 1024 + 4;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    uint32_t *hist = sel_lds, *list = hist + kSelBins, *red = list + kSelList, *key_lds = red + 5 * 16;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const float *srow = scores + (int64_t)blockIdx.x * len;
     int64_t *orow = out + (int64_t)blockIdx.x * n;
-    const int64_t rec = len - pl > 0 ? len - pl : 0;
-    uint32_t key_reg[kSelRegSlots];
-    // buffer loads: the slot offset is a constant, so no per-slot address registers
-    const __amdgpu_buffer_rsrc_t rs = make_rsrc(srow, (uint32_t)(len * 4));
-    // 32-bit position arithmetic against per-thread limits (len <= 65536), so that no
-    // per-slot index stays live in a register
-    const int lim = (int)len - tid, lim_pf = (int)pf - tid, lim_rec = (int)rec - tid;
-    auto to_key = [&](int j, uint32_t raw) {
-        const bool prot = 1024 * j < lim_pf || 1024 * j >= lim_rec;
-        return 1024 * j < lim ? (prot ? kKeyInf : order_key(__builtin_bit_cast(float, raw))) : 0u;
+    // len < 2^31: positions in 32 bits
+    const uint32_t L = (uint32_t)len, rec = (uint32_t)(len - pl > 0 ? len - pl : 0);
+    const uint32_t first = (uint32_t)(pf < len ? pf : len);
+    const int nslot = (int)((L + 1023u) / 1024u);
+    const uint32_t i0 = (uint32_t)wave * 64u * (uint32_t)nslot + (uint32_t)lane;  // slot 0 of this lane
+    auto raw_at = [&](int j) { return srow[min(i0 + 64u * (uint32_t)j, L - 1u)]; };
+    auto to_key = [&](int j, float x) -> uint32_t {
+        const uint32_t i = i0 + 64u * (uint32_t)j;
+        if (i >= L) return 0xFFFFFFFFu;
+        return (i < first || i >= rec) ? kKeyInf : order_key(x);
     };
+    uint32_t key_reg[SLOTS > 0 ? (SLOTS < kSelRegSlots ? SLOTS : kSelRegSlots) : 1];
+    // f(slot, key) over this wave's slots
+    auto each = [&](auto &&f) {
+        if constexpr (SLOTS > 0) {
 #pragma unroll
-    for (int j = 0; j < kSelRegSlots; ++j)
-        key_reg[j] = __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)tid * 4u, 4096 * j, 0);
+            for (int j = 0; j < (SLOTS < kSelRegSlots ? SLOTS : kSelRegSlots); ++j)
+                if (j < nslot) f(j, key_reg[j]);
+            if constexpr (SLOTS > kSelRegSlots)
+                for (int j = kSelRegSlots; j < nslot; j += 8) {  // 8 reads in flight
+                    uint32_t k[8];
 #pragma unroll
-    for (int j0 = kSelRegSlots; j0 < kSelSlots; j0 += 8) {  // LDS slots, 8 loads in flight at a time
-        uint32_t raw[8];
+                    for (int e = 0; e < 8; ++e) k[e] = key_lds[(min(j + e, nslot - 1) - kSelRegSlots) * 1024 + tid];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) raw[i] = __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)tid * 4u, 4096 * (j0 + i), 0);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) key_lds[(j0 + i - kSelRegSlots) * 1024 + tid] = to_key(j0 + i, raw[i]);
-    }
-#pragma unroll
-    for (int j = 0; j < kSelRegSlots; ++j) key_reg[j] = to_key(j, key_reg[j]);
-    // slot j of this thread (j a compile-time constant after unrolling); a thread reads
-    // only its own LDS slots, so they need no barrier
-    auto key = [&](int j) -> uint32_t { return j < kSelRegSlots ? key_reg[j] : key_lds[(j - kSelRegSlots) * 1024 + tid]; };
-    auto valid = [&](int j) { return 1024 * j < lim; };
-    if (tid == 0) {
-        s_prefix = 0u;
-        s_k = (uint32_t)n;
-    }
-    for (int pass = 0; pass < 4; ++pass) {
-        const int shift = 24 - 8 * pass;
-        for (int i = tid; i < 16 * 256; i += 1024) (&hist[0][0])[i] = 0u;
-        __syncthreads();
-        const uint32_t prefix = s_prefix;
-        const uint32_t hmask = pass == 0 ? 0u : (0xFFFFFFFFu << (shift + 8));
-#pragma unroll
-        for (int j = 0; j < kSelSlots; ++j) {
-            const uint32_t d = (key(j) >> shift) & 255u;
-            bool pend = valid(j) && (key(j) & hmask) == prefix;
-            if (pass == 0) {  // the sign / exponent digit clusters: add the two most common
-                              // digits of the wave as groups, the rest per lane
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    const uint64_t act = __builtin_amdgcn_ballot_w64(pend);
-                    if (!act) break;
-                    const int first = (int)__builtin_ctzll(act);
-                    const uint32_t db = (uint32_t)__builtin_amdgcn_readlane((int)d, first);
-                    const uint64_t m = __builtin_amdgcn_ballot_w64(pend && d == db);
-                    if (lane == first) atomicAdd(&hist[wave][db], (uint32_t)__builtin_popcountll(m));
-                    pend = pend && d != db;
+                    for (int e = 0; e < 8; ++e)
+                        if (j + e < nslot) f(j + e, k[e]);
                 }
-            }
-            if (pend) atomicAdd(&hist[wave][d], 1u);
-            asm volatile("" ::: "memory");
-        }
-        __syncthreads();
-        // digit of the k-th key: scan of the 256 bin totals (4 waves), then the one
-        // bin with excl < k <= incl (the last bin also when the keys run out)
-        const uint32_t k = s_k;
-        uint32_t t = 0, incl = 0;
-        if (tid < 256) {
+        } else {
+            for (int j = 0; j < nslot; j += 8) {  // 8 loads in flight; slots past the last hold no element
+                float x[8];
 #pragma unroll
-            for (int w = 0; w < 16; ++w) t += hist[w][tid];
-            incl = wave_incl_scan(t, lane);
-            if (lane == 63) tot[wave] = incl;
-        }
-        __syncthreads();
-        if (tid < 256) {
-            for (int w = 0; w < wave; ++w) incl += tot[w];
-            const uint32_t excl = incl - t;
-            if (excl < k && (k <= incl || tid == 255)) {
-                s_k = k - excl;
-                s_prefix = prefix | ((uint32_t)tid << shift);
+                for (int e = 0; e < 8; ++e) x[e] = raw_at(min(j + e, nslot - 1));
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (j + e < nslot) f(j + e, to_key(j + e, x[e]));
             }
         }
-        __syncthreads();
-    }
-    const uint32_t tau = s_prefix, take_eq = s_k;  // take the first take_eq elements equal to tau
-    // counts of (slot j, wave w) at entry 16 j + w: element order
+    };
+    if constexpr (SLOTS > 0) {
+        constexpr int kR = SLOTS < kSelRegSlots ? SLOTS : kSelRegSlots;
+        float x[kR];
 #pragma unroll
-    for (int j = 0; j < kSelSlots; ++j) {
-        const uint64_t ml = __builtin_amdgcn_ballot_w64(valid(j) && key(j) < tau);
-        const uint64_t me = __builtin_amdgcn_ballot_w64(valid(j) && key(j) == tau);
-        if (lane == 0) {
-            cnt_lt[16 * j + wave] = (uint32_t)__builtin_popcountll(ml);
-            cnt_eq[16 * j + wave] = (uint32_t)__builtin_popcountll(me);
+        for (int j = 0; j < kR; ++j) x[j] = raw_at(min(j, nslot - 1));
+#pragma unroll
+        for (int j = 0; j < kR; ++j) key_reg[j] = to_key(j, x[j]);
+        if constexpr (SLOTS > kSelRegSlots) {
+            for (int j = kSelRegSlots; j < nslot; j += 8) {
+                float y[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) y[e] = raw_at(min(j + e, nslot - 1));
+#pragma unroll
+                for (int e = 0; e < 8; ++e)  // a thread reads only its own LDS slots: no barrier
+                    if (j + e < nslot) key_lds[(j + e - kSelRegSlots) * 1024 + tid] = to_key(j + e, y[e]);
+            }
         }
-        asm volatile("" ::: "memory");
+    }
+    uint32_t kmin = 0xFFFFFFFFu, kmax = 0u, n_fin = 0u, n_inf = 0u;
+    each([&](int, uint32_t k) {
+        const bool fin = k < kKeyInf;
+        kmin = min(kmin, k);
+        kmax = max(kmax, fin ? k : 0u);
+        n_fin += fin;
+        n_inf += k == kKeyInf;
+    });
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        kmin = min(kmin, (uint32_t)__shfl_xor((int)kmin, o));
+        kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o));
+        n_fin += (uint32_t)__shfl_xor((int)n_fin, o);
+        n_inf += (uint32_t)__shfl_xor((int)n_inf, o);
+    }
+    if (lane == 0) {
+        red[wave] = kmin;
+        red[16 + wave] = kmax;
+        red[32 + wave] = n_fin;
+        red[48 + wave] = n_inf;
     }
     __syncthreads();
-    {  // exclusive scans of the 1024 counts: in each wave, then across the 16 waves
-        const uint32_t own_lt = cnt_lt[tid], own_eq = cnt_eq[tid];
-        uint32_t il = wave_incl_scan(own_lt, lane), ie = wave_incl_scan(own_eq, lane);
-        if (lane == 63) {
-            hist[0][wave] = il;
-            hist[1][wave] = ie;
+    n_fin = n_inf = 0u;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        kmin = min(kmin, red[w]);
+        kmax = max(kmax, red[16 + w]);
+        n_fin += red[32 + w];
+        n_inf += red[48 + w];
+    }
+    const uint32_t want = (uint32_t)n;
+    uint32_t tau, take_eq;  // the n-th smallest key; how many elements equal to it to take
+    if (want > n_fin) {
+        tau = want <= n_fin + n_inf ? kKeyInf : 0xFFFFFFFFu;
+        take_eq = want - n_fin - (tau == kKeyInf ? 0u : n_inf);
+    } else {
+        // the key of rank k among those in [lo, lo + maxd], maxd < 2^bits
+        uint32_t lo = kmin, maxd = kmax - kmin, k = want, n_list = 0;
+        int bits = maxd ? 32 - __builtin_clz(maxd) : 0;
+        bool listed = false;
+        while (bits > 0) {
+            const int shift = bits > 11 ? bits - 11 : 0;
+            hist[tid] = 0u;
+            hist[tid + 1024] = 0u;
+            __syncthreads();
+            auto add = [&](uint32_t key) {
+                const uint32_t d = key - lo, bin = d >> shift;
+                const bool in = d <= maxd;
+                const uint64_t act = __builtin_amdgcn_ballot_w64(in);
+                if (!act) return;
+                const int l0 = (int)__builtin_ctzll(act);
+                const bool same = in && bin == (uint32_t)__builtin_amdgcn_readlane((int)bin, l0);
+                const uint64_t m = __builtin_amdgcn_ballot_w64(same);
+                if (in && (!same || lane == l0)) atomicAdd(&hist[bin], same ? (uint32_t)__builtin_popcountll(m) : 1u);
+            };
+            if (listed) {
+                for (uint32_t i = 0; i < n_list; i += 1024u)
+                    add(i + (uint32_t)tid < n_list ? list[i + (uint32_t)tid] : lo - 1u);
+            } else {
+                each([&](int, uint32_t key) { add(key); });
+            }
+            __syncthreads();
+            const uint32_t a = hist[2 * tid], b = hist[2 * tid + 1];
+            uint32_t incl = wave_incl_scan(a + b, lane);
+            if (lane == 63) red[wave] = incl;
+            __syncthreads();
+            for (int w = 0; w < wave; ++w) incl += red[w];
+            const uint32_t excl = incl - a - b;
+            if (excl < k && k <= incl) {  // one thread
+                const bool hi = k > excl + a;
+                red[64] = 2u * (uint32_t)tid + (hi ? 1u : 0u);
+                red[65] = k - excl - (hi ? a : 0u);
+                red[66] = hi ? b : a;
+                red[67] = 0u;  // the list's length
+            }
+            __syncthreads();
+            const uint32_t off = red[64] << shift, cnt = red[66];
+            k = red[65];
+            maxd = min(maxd - off, (1u << shift) - 1u);
+            lo += off;
+            bits = shift;
+            if (bits > 0 && !listed && cnt <= (uint32_t)kSelList) {
+                each([&](int, uint32_t key) {
+                    const bool in = key - lo <= maxd;
+                    const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+                    if (!m) return;
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(&red[67], (uint32_t)__builtin_popcountll(m));
+                    base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+                    if (in) list[base + lanes_below(m)] = key;
+                });
+                listed = true;
+                n_list = cnt;
+            }
+            __syncthreads();  // the list is written; red and hist may be written again
         }
-        __syncthreads();
-        for (int w = 0; w < wave; ++w) {
-            il += hist[0][w];
-            ie += hist[1][w];
-        }
-        cnt_lt[tid] = il - own_lt;
-        cnt_eq[tid] = ie - own_eq;
+        tau = lo;
+        take_eq = k;
     }
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kSelSlots; ++j) {
-        const bool lt = valid(j) && key(j) < tau, eq = valid(j) && key(j) == tau;
+    uint32_t lt_run = 0, eq_run = 0;  // of this wave, then before its current slot
+    auto is_eq = [&](int j, uint32_t key) { return key == tau && i0 + 64u * (uint32_t)j < L; };
+    each([&](int j, uint32_t key) {
+        lt_run += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key < tau));
+        eq_run += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(is_eq(j, key)));
+    });
+    if (lane == 0) {
+        red[wave] = lt_run;
+        red[16 + wave] = eq_run;
+    }
+    __syncthreads();
+    lt_run = eq_run = 0;
+    for (int w = 0; w < wave; ++w) {
+        lt_run += red[w];
+        eq_run += red[16 + w];
+    }
+    each([&](int j, uint32_t key) {
+        const bool lt = key < tau, eq = is_eq(j, key);
         const uint64_t ml = __builtin_amdgcn_ballot_w64(lt), me = __builtin_amdgcn_ballot_w64(eq);
-        const uint32_t lt_before = cnt_lt[16 * j + wave] + __builtin_amdgcn_mbcnt_hi((uint32_t)(ml >> 32),
-                                       __builtin_amdgcn_mbcnt_lo((uint32_t)ml, 0u));
-        const uint32_t eq_before = cnt_eq[16 * j + wave] + __builtin_amdgcn_mbcnt_hi((uint32_t)(me >> 32),
-                                       __builtin_amdgcn_mbcnt_lo((uint32_t)me, 0u));
-        const int64_t i = (int64_t)(tid + 1024 * j);
-        if (lt) orow[lt_before + (eq_before < take_eq ? eq_before : take_eq)] = i;
-        else if (eq && eq_before < take_eq) orow[lt_before + eq_before] = i;
-        asm volatile("" ::: "memory");  // one slot at a time (keeps the live ranges short)
-    }
+        const uint32_t lt_before = lt_run + lanes_below(ml), eq_before = eq_run + lanes_below(me);
+        if (lt || (eq && eq_before < take_eq))
+            orow[lt_before + min(eq_before, take_eq)] = (int64_t)(i0 + 64u * (uint32_t)j);
+        lt_run += (uint32_t)__builtin_popcountll(ml);
+        eq_run += (uint32_t)__builtin_popcountll(me);
+    });
 }
 
 hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t n, int64_t pf, int64_t pl,
                          int64_t *out, hipStream_t s) {
     if (rows <= 0 || n <= 0) return hipSuccess;
-    if (len <= 1024 * kSelSlots) {
+#define AKV_SEL(slots)                                                                                          \
+    hipLaunchKernelGGL(select_kernel<slots>, dim3((unsigned)rows), dim3(1024), sel_lds_bytes(slots), s, scores, len, \
+                       n, pf, pl, out)
+    if (len <= 2 * 1024) AKV_SEL(2);
+    else if (len <= 8 * 1024) AKV_SEL(8);
+    else if (len <= 32 * 1024) AKV_SEL(32);
+    else if (len <= 64 * 1024) {
         // raise the dynamic LDS cap above 64 KiB once per device (a bit per device index;
         // host threads that race here both set it, which is harmless)
         static std::atomic<uint64_t> attr_devs{0};
@@ -733,16 +726,14 @@ hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t
         if (e != hipSuccess) return e;
         const uint64_t bit = (dev >= 0 && dev < 64) ? 1ull << dev : 0ull;
         if (!bit || !(attr_devs.load(std::memory_order_acquire) & bit)) {
-            e = hipFuncSetAttribute((const void *)select_reg_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    kSelLdsBytes);
+            e = hipFuncSetAttribute((const void *)select_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    sel_lds_bytes(64));
             if (e != hipSuccess) return e;
             attr_devs.fetch_or(bit, std::memory_order_release);
         }
-        hipLaunchKernelGGL(select_reg_kernel, dim3((unsigned)rows), dim3(1024), kSelLdsBytes, s, scores, len, n, pf,
-                           pl, out);
-    }
-    else
-        hipLaunchKernelGGL(select_kernel, dim3((unsigned)rows), dim3(1024), 0, s, scores, len, n, pf, pl, out);
+        AKV_SEL(64);
+    } else AKV_SEL(0);
+#undef AKV_SEL
     return hipGetLastError();
 }
 
