@@ -122,6 +122,17 @@ class ImportanceArgs(ctypes.Structure):
     ]
 
 
+class RowsJob(ctypes.Structure):
+    _fields_ = [
+        ("src", _vp), ("dst", _vp),
+        ("src_b", _i64), ("src_h", _i64), ("src_t", _i64),
+        ("dst_b", _i64), ("dst_h", _i64), ("dst_t", _i64),
+        ("n", _i64), ("limit", _i64), ("start", _i64), ("step", _i64),
+        ("B", _i32), ("H", _i32), ("row", _i32), ("elem", _i32),
+        ("kind", _i32), ("map", _i32), ("src_dt", _i32), ("value", ctypes.c_float),
+    ]
+
+
 EXPORTS = (
     "akv_abi_version", "akv_last_error", "akv_struct_size",
     "akv_decode_workspace_bytes", "akv_decode_counter_bytes", "akv_decode_attn", "akv_decode_attn_noalloc",
@@ -129,9 +140,10 @@ EXPORTS = (
     "akv_bitpack", "akv_bitunpack", "akv_importance_update",
     "akv_importance_workspace_bytes", "akv_importance_update_ws",
     "akv_prefill_workspace_bytes", "akv_prefill_attn", "akv_select_demote", "akv_stream_read",
+    "akv_rows_move", "akv_promote_select",
     "akv_timeline_words", "akv_timeline_fetch", "akv_timeline_clear",
 )
-STRUCTS = (WarmDesc, DecodeArgs, QuantArgs, DequantArgs, ImportanceArgs, PrefillArgs)
+STRUCTS = (WarmDesc, DecodeArgs, QuantArgs, DequantArgs, ImportanceArgs, PrefillArgs, RowsJob)
 
 _lib: Optional[ctypes.CDLL] = None
 
@@ -182,6 +194,10 @@ def load() -> ctypes.CDLL:
     lib.akv_prefill_attn.argtypes = [ctypes.POINTER(PrefillArgs), _vp]
     lib.akv_select_demote.restype = ctypes.c_int
     lib.akv_select_demote.argtypes = [_vp, _i64, _i64, _i64, _i32, _i32, _vp, _vp]
+    lib.akv_rows_move.restype = ctypes.c_int
+    lib.akv_rows_move.argtypes = [ctypes.POINTER(RowsJob), _i32, _vp, _i64, _vp]
+    lib.akv_promote_select.restype = ctypes.c_int
+    lib.akv_promote_select.argtypes = [_vp, _vp, _vp, _i64, ctypes.c_float, ctypes.c_float, ctypes.c_float, _i64, _vp, _vp]
     lib.akv_stream_read.restype = ctypes.c_int
     lib.akv_stream_read.argtypes = [_vp, _i64, _vp, _vp]
     lib.akv_timeline_words.restype = _i64

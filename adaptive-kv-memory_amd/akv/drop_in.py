@@ -20,6 +20,7 @@ from typing import Optional
 import torch
 
 from . import _native as nat
+from .row_moves import GATHER, KEEP, SCATTER, RowMoves, movable
 from .warm_tier import WarmTier, packed_row_bytes, quantize_kv
 
 _PRESETS = {
@@ -164,37 +165,45 @@ class _EventTier:
 
     _TOKEN_AXIS = {"kc": 2, "vc": 2, "vs": 2, "vz": 2, "kod": 2, "vod": 2, "blk": 0, "pos": 0}
 
+    @staticmethod
+    def _rows4(name, x):
+        """A tier tensor as (B, H, rows, C): the outlier indices have no head axis."""
+        return x.unsqueeze(1) if name in ("koi", "voi") else x
+
     def _grow(self, cap, ecap):
         t = self._alloc(cap, ecap)
+        mv = RowMoves()
         for name, old in self.t.items():
-            if name in self._TOKEN_AXIS:
-                t[name].narrow(self._TOKEN_AXIS[name], 0, self.n).copy_(old.narrow(self._TOKEN_AXIS[name], 0, self.n))
-            else:
-                ax = 2 if name in ("ks", "kz") else 1
-                t[name].narrow(ax, 0, self.n_events).copy_(old.narrow(ax, 0, self.n_events))
+            mv.copy(self._rows4(name, t[name]), self._rows4(name, old),
+                    self.n if name in self._TOKEN_AXIS else self.n_events)
+        mv.run()
         self.t, self.cap, self.ecap = t, cap, ecap
 
-    def append(self, w: WarmTier, positions: torch.Tensor):
-        """One demotion event: ``w`` holds its n tokens as a single K block."""
+    def append(self, w: WarmTier, positions: torch.Tensor, idx: torch.Tensor):
+        """One demotion event: ``w`` holds its n tokens as a single K block; their positions
+        are ``positions[idx]``."""
         n = w.n_warm
         if self.n + n > self.cap or self.n_events + 1 > self.ecap:
             self._grow(max(self.cap, 2 * (self.n + n)), max(self.ecap, 2 * (self.n_events + 1)))
         t, a, e = self.t, self.n, self.n_events
-        t["kc"][:, :, a:a + n] = w.k_codes
-        t["vc"][:, :, a:a + n] = w.v_codes
-        t["vs"][:, :, a:a + n] = w.v_scale
-        t["vz"][:, :, a:a + n] = w.v_zero
-        t["ks"][:, :, e:e + 1] = w.k_scale
-        t["kz"][:, :, e:e + 1] = w.k_zero
+        mv = RowMoves()
+        for name, x in (("kc", w.k_codes), ("vc", w.v_codes), ("vs", w.v_scale), ("vz", w.v_zero)):
+            mv.copy(t[name], x, n, at=a)
+        mv.copy(t["ks"], w.k_scale, 1, at=e)
+        mv.copy(t["kz"], w.k_zero, 1, at=e)
         if self.n_out:
-            t["kod"][:, :, a:a + n] = w.k_odata
-            t["vod"][:, :, a:a + n] = w.v_odata
-            t["koi"][:, e:e + 1] = w.k_oidx
-            t["voi"][:, e:e + 1] = w.v_oidx
-        t["blk"][a:a + n] = e
-        t["pos"][a:a + n] = positions
+            mv.copy(t["kod"], w.k_odata, n, at=a)
+            mv.copy(t["vod"], w.v_odata, n, at=a)
+            mv.copy(t["koi"].unsqueeze(1), w.k_oidx.unsqueeze(1), 1, at=e)
+            mv.copy(t["voi"].unsqueeze(1), w.v_oidx.unsqueeze(1), 1, at=e)
+        mv.count(t["blk"], n, e, 0, at=a)
+        mv.copy(t["pos"], positions, n, GATHER, at=a)
+        mv.run(idx, n)
         self.n += n
         self.n_events += 1
+
+    def positions(self) -> torch.Tensor:
+        return self.t["pos"][: self.n]
 
     def resident_bytes(self) -> int:
         """Bytes of the used extents (codes, meta, outliers, event map, positions)."""
@@ -247,25 +256,40 @@ class _EventTier:
         sub = _EventTier.__new__(_EventTier)
         sub.__dict__.update({k: v for k, v in self.__dict__.items() if k != "t"})
         sub.t = {}
+        mv = RowMoves()
         for name, x in self.t.items():
             if name in self._TOKEN_AXIS:
-                sub.t[name] = x.narrow(self._TOKEN_AXIS[name], 0, self.n).index_select(self._TOKEN_AXIS[name], idx)
+                shape = list(x.shape)
+                shape[self._TOKEN_AXIS[name]] = n
+                sub.t[name] = torch.empty(shape, dtype=x.dtype, device=x.device)
+                mv.copy(sub.t[name], x, n, GATHER)
             else:
                 sub.t[name] = x
+        mv.run(idx, n)
         sub.n, sub.cap = n, n
         k = torch.empty(self.B, self.H, n, self.D, dtype=torch.float16, device=self.dev)
         v = torch.empty_like(k)
         sub.dequantize_into(k, v, slots=False)
         return k, v
 
-    def keep(self, keep_mask: torch.Tensor):
-        """Drop the warm tokens where ``keep_mask`` is False (their events' K meta rows stay)."""
-        kept = keep_mask.nonzero().flatten()
-        for name, x in self.t.items():
-            if name in self._TOKEN_AXIS:
-                ax = self._TOKEN_AXIS[name]
-                x.narrow(ax, 0, kept.numel()).copy_(x.narrow(ax, 0, self.n).index_select(ax, kept))
-        self.n = kept.numel()
+    def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+        """Drop the ``n`` warm tokens of the ascending list ``idx`` (their events' K meta rows
+        stay); ``vector`` (one float32 per warm token) is returned without theirs.  The kept
+        rows go to fresh tensors: rows shift by up to n, so a move in place would race."""
+        kept = self.n - n
+        mv = RowMoves()
+        for name in self._TOKEN_AXIS:
+            if name in self.t:
+                x = self.t[name]
+                self.t[name] = torch.empty_like(x)
+                mv.copy(self.t[name], x, kept, KEEP)
+        out = None
+        if vector is not None:
+            out = torch.empty(kept, dtype=vector.dtype, device=vector.device)
+            mv.copy(out, vector, kept, KEEP)
+        mv.run(idx, n)
+        self.n = kept
+        return out
 
     def index_batch(self, beam_idx: torch.Tensor):
         for name in list(self.t):
@@ -291,7 +315,7 @@ class _HeadBitsTier:
             self.groups.append([bits, torch.tensor(heads, dtype=torch.long, device=dev), None])
 
     def demote(self, hk, hv, idx, outlier_fraction, positions) -> int:
-        """Quantize hot tokens ``idx`` of every head with its width as one event; returns
+        """Quantize hot tokens ``idx`` (at ``positions[idx]``) of every head with its width as one event; returns
         the measured packed bytes (codes + scale + zero of K and V, per head)."""
         B, _, _, D = hk.shape
         n = idx.numel()
@@ -304,7 +328,7 @@ class _HeadBitsTier:
             w = quantize_kv(k, v, bits, bits, block_t=max(n, 1), group_v=D, outlier_fraction=outlier_fraction)
             if tier is None:
                 g[2] = tier = _EventTier(B * hs, 1, D, bits, bits, w.n_out, self.dev)
-            tier.append(w, positions)
+            tier.append(w, positions, idx)
             packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
                        + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
         self.n += n
@@ -334,10 +358,16 @@ class _HeadBitsTier:
             v.index_copy_(1, heads, tv.view(self.B, heads.numel(), n, self.D))
         return k, v
 
-    def keep(self, keep_mask: torch.Tensor):
-        for g in self.groups:
-            g[2].keep(keep_mask)
-        self.n = int(keep_mask.sum())
+    def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+        out = None
+        for i, g in enumerate(self.groups):
+            kept = g[2].remove(idx, n, vector if i == 0 else None)
+            out = kept if i == 0 else out
+        self.n -= n
+        return out
+
+    def positions(self) -> torch.Tensor:
+        return self.groups[0][2].positions()
 
     def index_batch(self, beam_idx: torch.Tensor):
         beam_idx = beam_idx.to(self.dev)
@@ -402,9 +432,8 @@ class AKVLayer:
         self.per_head_bits = list(per_head_bits) if per_head_bits is not None else None
         self._hot_keys: Optional[torch.Tensor] = None
         self._hot_values: Optional[torch.Tensor] = None
-        self._hot_positions: Optional[torch.Tensor] = None   # (N_hot,) int64, host
+        self._hot_positions: Optional[torch.Tensor] = None   # (N_hot,) int64, device
         self._warm: Optional[_EventTier] = None
-        self._warm_positions: Optional[torch.Tensor] = None  # (N_warm,) int64, host
         self._warm_len = 0
         self._total_len = 0
         self._warm_bytes_packed = 0
@@ -417,135 +446,192 @@ class AKVLayer:
     def get_seq_length(self) -> int:
         return self._total_len
 
-    def _append_hot(self, k, v, pos):
-        if self._hot_keys is None:
-            self._hot_keys, self._hot_values, self._hot_positions = k, v, pos
-        else:
-            self._hot_keys = torch.cat([self._hot_keys, k], dim=2)
-            self._hot_values = torch.cat([self._hot_values, v], dim=2)
-            self._hot_positions = torch.cat([self._hot_positions, pos])
+    @property
+    def _warm_positions(self) -> Optional[torch.Tensor]:
+        """(N_warm,) int64, device: the warm tokens' positions in demotion order."""
+        return None if self._warm is None else self._warm.positions()
 
-    def _update_importance(self, n_new: int, hot_len: int, device):
-        """akv/drop_in.py:375-389 (recency decay, on the device)."""
-        if self._importance is None or self._importance.shape[0] != hot_len - n_new:
-            self._importance = torch.ones(hot_len, dtype=torch.float32, device=device)
-        else:
-            self._importance = torch.cat([self._importance * self._decay,
-                                          torch.ones(n_new, dtype=torch.float32, device=device)])
+    @staticmethod
+    def _join(mv: RowMoves, parts: list) -> torch.Tensor:
+        """torch.cat(parts, dim=2) as jobs of ``mv`` (one part: itself), torch's own where the
+        parts do not fit each other or row moves do not do them."""
+        if len(parts) == 1:
+            return parts[0]
+        first, dt = parts[0], parts[0].dtype
+        for x in parts[1:]:
+            dt = torch.promote_types(dt, x.dtype)
+        if not movable(dt, *parts) or any(x.dim() != 4 or x.device != first.device or x.shape[:2] != first.shape[:2]
+                                          or x.shape[3] != first.shape[3] for x in parts):
+            return torch.cat(parts, dim=2)
+        out = torch.empty(first.shape[0], first.shape[1], sum(x.shape[2] for x in parts), first.shape[3], dtype=dt,
+                          device=first.device)
+        at = 0
+        for x in parts:
+            n = x.shape[2]
+            mv.copy(out, x if x.stride(3) == 1 or x.shape[3] <= 1 else x.contiguous(), n, at=at)
+            at += n
+        return out
 
-    def _update_proxy_score(self, key_states: torch.Tensor):
-        """akv/drop_in.py:486-525 over the packed tier: only its keys are dequantized (one
-        launch, warm-tier order, no copy of the packed arrays)."""
+    def _append_hot(self, k, v, promoted=None):
+        """The hot tier with the promoted tokens in front and the new ones (k, v) behind, their
+        positions, and the importance: 2 for the promoted, decayed for the old, 1 for the new
+        (akv/drop_in.py:375-389, :433-484); one launch.  ``promoted``: (K, V, the warm tier's
+        positions, their indices among them)."""
+        dev = k.device
+        old = 0 if self._hot_keys is None else self._hot_keys.shape[2]
+        new = k.shape[2]
+        front = 0 if promoted is None else promoted[0].shape[2]
+        mv = RowMoves()
+        parts_k = ([] if promoted is None else [promoted[0]]) + ([] if self._hot_keys is None else [self._hot_keys]) + [k]
+        parts_v = ([] if promoted is None else [promoted[1]]) + ([] if self._hot_keys is None else [self._hot_values]) + [v]
+        keys, values = self._join(mv, parts_k), self._join(mv, parts_v)
+        pos = torch.empty(front + old + new, dtype=torch.int64, device=dev)
+        if front:
+            mv.copy(pos, promoted[2], front, GATHER)
+        if old:
+            mv.copy(pos, self._hot_positions, old, at=front)
+        mv.count(pos, new, self._total_len, at=front + old)
+        imp = None
+        if not self.protect:
+            imp = torch.empty(front + old + new, dtype=torch.float32, device=dev)
+            mv.fill(imp, front, 2.0)
+            if self._importance is not None and self._importance.shape[0] == old:
+                mv.copy(imp, self._importance, old, at=front, value=self._decay)
+            else:
+                mv.fill(imp, old, 1.0, at=front)
+            mv.fill(imp, new, 1.0, at=front + old)
+        mv.run(None if promoted is None else promoted[3], front)
+        self._hot_keys, self._hot_values, self._hot_positions, self._importance = keys, values, pos, imp
+        self._total_len += new
+
+    def _proxy_similarity(self, key_states: torch.Tensor) -> Optional[torch.Tensor]:
+        """akv/drop_in.py:486-525 over the packed tier: the cosine of every warm token's key
+        with the mean new key; only the keys are dequantized (one launch, warm-tier order, no
+        copy of the packed arrays), to float32."""
         if self._warm is None or self._warm.n == 0:
             self._proxy_score = None
-            return
+            return None
         probe = key_states.detach().float().mean(dim=(0, 1, 2))
         probe = probe / (probe.norm() + 1e-6)
         w = self._warm
-        wk = torch.empty(w.B, w.H, w.n, w.D, dtype=torch.float16, device=w.dev)
+        wk = torch.empty(w.B, w.H, w.n, w.D, dtype=torch.float32, device=w.dev)
         w.dequantize_into(wk, None, slots=False)
-        wk_flat = wk.float().mean(dim=(0, 1))
+        wk_flat = wk.mean(dim=(0, 1))
         wk_norm = wk_flat / (wk_flat.norm(dim=-1, keepdim=True) + 1e-6)
-        sim = wk_norm @ probe
-        if self._proxy_score is None or self._proxy_score.shape[0] != sim.shape[0]:
-            self._proxy_score = sim.abs()
-        else:
-            d = self.proxy_decay
-            self._proxy_score = d * self._proxy_score + (1 - d) * sim.abs()
+        return wk_norm @ probe
 
-    def _promote(self, scores: torch.Tensor, use_proxy: bool):
-        """akv/drop_in.py:433-484 / :543-589: move the warm tokens above the threshold
-        (at most max(1, hot_budget // 8), the top ones) to the front of the hot tier."""
-        warm_len = self._warm.n
-        mask = scores > self.promotion_threshold
-        n = int(mask.sum().item())
+    def _choose(self, scores: torch.Tensor, proxy: bool) -> torch.Tensor:
+        """The promotion choice of ``akv_promote_select``: (1 + cap,) int64, how many, then the
+        warm indices.  ``proxy``: ``scores`` are similarities that first go into the running
+        proxy scores (their EMA where the tokens are the same)."""
+        n = scores.shape[0]
+        cap = min(n, max(1, self.hot_budget // 8))
+        scores = nat.dev_contig(scores, torch.float32)
+        out = torch.empty(1 + cap, dtype=torch.int64, device=scores.device)
+        prev = new = None
+        if proxy:
+            if self._proxy_score is not None and self._proxy_score.shape[0] == n:
+                prev = nat.dev_contig(self._proxy_score)
+            new = torch.empty(n, dtype=torch.float32, device=scores.device)
+        d = self.proxy_decay
+        nat.check(nat.load().akv_promote_select(scores.data_ptr(), nat.ptr(prev), nat.ptr(new), n, d, 1 - d,
+                                                self.promotion_threshold, cap, out.data_ptr(), nat.stream_of(scores)),
+                  "promotion choice")
+        if proxy:
+            self._proxy_score = new
+        return out
+
+    def _take_promoted(self, chosen: torch.Tensor, use_proxy: bool):
+        """akv/drop_in.py:433-484 / :543-589: the chosen warm tokens leave the packed tier;
+        returns what ``_append_hot`` puts in front of the hot tier, or None.  The count is the
+        one value an update waits for: the shapes that follow depend on it."""
+        n = int(chosen[0])
         if n == 0:
-            return
-        cap = max(1, self.hot_budget // 8)
-        if n > cap:
-            _, top = scores.topk(cap)
-            mask = torch.zeros_like(mask)
-            mask[top] = True
-            n = cap
-        idx = mask.nonzero().flatten()
+            return None
+        idx = chosen[1:1 + n]
+        warm_len = self._warm.n
+        positions = self._warm.positions()
         pk, pv = self._warm.take(idx)
-        idx_host = idx.cpu()
-        positions = self._warm_positions[idx_host]
-        keep = ~mask
-        self._warm.keep(keep)
-        self._warm_positions = self._warm_positions[keep.cpu()]
+        kept = self._warm.remove(idx, n, self._proxy_score if use_proxy else None)
         if use_proxy:
-            self._proxy_score = self._proxy_score[keep]
+            self._proxy_score = kept
         self._warm_bytes_packed = int(self._warm_bytes_packed * (max(0, warm_len - n) / warm_len))
         self._warm_len -= n
-        self._hot_keys = torch.cat([pk, self._hot_keys], dim=2)
-        self._hot_values = torch.cat([pv, self._hot_values], dim=2)
-        self._hot_positions = torch.cat([positions, self._hot_positions])
-        if self._importance is not None:
-            self._importance = torch.cat([torch.full((n,), 2.0, device=self._importance.device), self._importance])
+        return pk, pv, positions, idx
 
     def _demote(self, n_demote: int, hot_len: int):
         hk, hv = self._hot_keys, self._hot_values
         dev = hk.device
         B, H, _, D = hk.shape
         idx = select_demote_indices(self._importance, n_demote, hot_len, self.hot_budget, device=dev)
-        idx_host = idx.cpu()
-        positions = self._hot_positions[idx_host]
         if self.per_head_bits and len(self.per_head_bits) == H:
             if self._warm is None:
                 self._warm = _HeadBitsTier(B, H, D, self.per_head_bits, dev)
-            self._warm_bytes_packed += self._warm.demote(hk, hv, idx, self.outlier_fraction, positions.to(dev))
+            self._warm_bytes_packed += self._warm.demote(hk, hv, idx, self.outlier_fraction, self._hot_positions)
         else:
             w = quantize_kv(hk, hv, self.warm_key_bits, self.warm_value_bits, block_t=max(n_demote, 1), group_v=D,
                             outlier_fraction=self.outlier_fraction, sel=idx.unsqueeze(0).expand(B, n_demote))
             if self._warm is None:
                 self._warm = _EventTier(B, H, D, self.warm_key_bits, self.warm_value_bits, w.n_out, dev)
-            self._warm.append(w, positions.to(dev))
+            self._warm.append(w, self._hot_positions, idx)
             # measure_packed_bytes per batch element: packed codes + fp16 scale and zero, K and V
             self._warm_bytes_packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
                                         + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
-        self._warm_positions = positions if self._warm_positions is None else torch.cat([self._warm_positions,
-                                                                                         positions])
         self._warm_len += n_demote
+        mv = RowMoves()
         if self._proxy_score is not None:  # new warm tokens start with no evidence
-            self._proxy_score = torch.cat([self._proxy_score,
-                                           torch.zeros(n_demote, dtype=self._proxy_score.dtype, device=dev)])
-        keep = torch.ones(hot_len, dtype=torch.bool)
-        keep[idx_host] = False
-        keep_dev = keep.to(dev)
-        self._hot_keys = hk[:, :, keep_dev]
-        self._hot_values = hv[:, :, keep_dev]
-        self._hot_positions = self._hot_positions[keep]
-        self._importance = self._importance[keep_dev]
+            old = self._proxy_score
+            self._proxy_score = torch.empty(old.shape[0] + n_demote, dtype=torch.float32, device=dev)
+            mv.copy(self._proxy_score, old, old.shape[0])
+            mv.fill(self._proxy_score, n_demote, 0.0, at=old.shape[0])
+        kept = hot_len - n_demote
+        pos, imp = self._hot_positions, self._importance
+        self._hot_positions = torch.empty(kept, dtype=torch.int64, device=dev)
+        self._importance = torch.empty(kept, dtype=torch.float32, device=dev)
+        mv.copy(self._hot_positions, pos, kept, KEEP)
+        mv.copy(self._importance, imp, kept, KEEP)
+        if movable(hk.dtype, hk) and movable(hv.dtype, hv):
+            tiers = []
+            for x in (hk, hv):
+                x = x if x.stride(3) == 1 or D <= 1 else x.contiguous()
+                tiers.append(torch.empty(B, H, kept, D, dtype=x.dtype, device=dev))
+                mv.copy(tiers[-1], x, kept, KEEP)
+            self._hot_keys, self._hot_values = tiers
+        else:
+            keep = torch.ones(hot_len, dtype=torch.bool, device=dev)
+            keep[idx] = False
+            self._hot_keys, self._hot_values = hk[:, :, keep], hv[:, :, keep]
+        mv.run(idx, n_demote)
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor,
                cache_kwargs: Optional[dict] = None) -> tuple[torch.Tensor, torch.Tensor]:
         """Append new KV, demote past the budget, return the chronological view."""
         nat.require_device(key_states, value_states)
         B, H, N, D = key_states.shape
-        new_positions = torch.arange(self._total_len, self._total_len + N, dtype=torch.long)
         if self.protect:
-            self._append_hot(key_states, value_states, new_positions)
-            self._total_len += N
+            self._append_hot(key_states, value_states)
             self.keys, self.values = self._hot_keys, self._hot_values
             return self._hot_keys, self._hot_values
-        self._append_hot(key_states, value_states, new_positions)
-        self._total_len += N
+        for hot, x in ((self._hot_keys, key_states), (self._hot_values, value_states)):
+            if hot is not None and (x.shape[:2] != hot.shape[:2] or x.shape[3] != hot.shape[3]):
+                torch.cat([hot, x], dim=2)  # raises, before any tier changes
         self._step += 1
-        hot_len = self._hot_keys.shape[2]
-        self._update_importance(N, hot_len, key_states.device)
+        chosen, use_proxy = None, False
         if self.enable_promotion_proxy:
-            self._update_proxy_score(key_states)
-        if self.enable_promotion and cache_kwargs and "attention_weights" in cache_kwargs:
+            sim = self._proxy_similarity(key_states)
+            if sim is not None:
+                chosen, use_proxy = self._choose(sim, proxy=True), True
+        if not self.enable_promotion:
+            chosen = None
+        elif cache_kwargs and "attention_weights" in cache_kwargs:
+            chosen, use_proxy = None, False
             aw = cache_kwargs["attention_weights"]
+            hot_len = N + (0 if self._hot_keys is None else self._hot_keys.shape[2])
             if self._warm is not None and self._warm.n and aw.dim() == 4 and aw.shape[-1] >= self._warm.n + hot_len:
-                self._promote(aw[:, :, :, : self._warm.n].float().mean(dim=(0, 1, 2)), use_proxy=False)
-            hot_len = self._hot_keys.shape[2]
-        elif self.enable_promotion and self.enable_promotion_proxy:
-            if (self._proxy_score is not None and self._warm is not None and self._warm.n
-                    and self._proxy_score.shape[0] == self._warm.n):
-                self._promote(self._proxy_score, use_proxy=True)
-            hot_len = self._hot_keys.shape[2]
+                chosen = self._choose(aw[:, :, :, : self._warm.n].float().mean(dim=(0, 1, 2)), proxy=False)
+        self._append_hot(key_states, value_states,
+                         None if chosen is None else self._take_promoted(chosen, use_proxy))
+        hot_len = self._hot_keys.shape[2]
         budget = self.hot_budget
         if self.adaptive_hot_frac > 0.0:
             budget = max(self.hot_budget, int(self.adaptive_hot_frac * self._total_len))
@@ -559,9 +645,15 @@ class AKVLayer:
         fk = torch.empty(B, H, self._total_len, D, dtype=out_dt, device=hk.device)
         fv = torch.empty_like(fk)
         self._warm.dequantize_into(fk, fv)
-        hp = self._hot_positions.to(hk.device)
-        fk.index_copy_(2, hp, hk.to(out_dt))
-        fv.index_copy_(2, hp, hv.to(out_dt))
+        hp = self._hot_positions
+        if movable(out_dt, hk) and movable(out_dt, hv):
+            mv = RowMoves()
+            mv.copy(fk, hk, hk.shape[2], SCATTER)
+            mv.copy(fv, hv, hv.shape[2], SCATTER)
+            mv.run(hp, hp.shape[0])
+        else:
+            fk.index_copy_(2, hp, hk.to(out_dt))
+            fv.index_copy_(2, hp, hv.to(out_dt))
         self.keys, self.values = fk, fv
         return fk, fv
 
@@ -574,21 +666,21 @@ class AKVLayer:
         if self._hot_keys is not None:
             keep = self._hot_positions < max_length
             if not bool(keep.all()):
-                kd = keep.to(self._hot_keys.device)
-                self._hot_keys = self._hot_keys[:, :, kd]
-                self._hot_values = self._hot_values[:, :, kd]
+                self._hot_keys = self._hot_keys[:, :, keep]
+                self._hot_values = self._hot_values[:, :, keep]
                 self._hot_positions = self._hot_positions[keep]
                 if self._importance is not None and self._importance.shape[0] == keep.shape[0]:
-                    self._importance = self._importance[kd]
-        if self._warm is not None and self._warm_positions is not None:
-            wkeep = self._warm_positions < max_length
-            n_drop = int((~wkeep).sum())
+                    self._importance = self._importance[keep]
+        if self._warm is not None and self._warm.n:
+            warm_len = self._warm.n
+            drop = (self._warm.positions() >= max_length).nonzero().flatten()
+            n_drop = drop.numel()
             if n_drop:
-                warm_len = int(wkeep.shape[0])
-                self._warm.keep(wkeep.to(self._warm.dev))
-                self._warm_positions = self._warm_positions[wkeep]
-                if self._proxy_score is not None and self._proxy_score.shape[0] == warm_len:
-                    self._proxy_score = self._proxy_score[wkeep.to(self._proxy_score.device)]
+                proxy = self._proxy_score
+                fits = proxy is not None and proxy.shape[0] == warm_len
+                kept = self._warm.remove(drop, n_drop, proxy if fits else None)
+                if fits:
+                    self._proxy_score = kept
                 self._warm_bytes_packed = int(self._warm_bytes_packed * ((warm_len - n_drop) / warm_len))
                 self._warm_len -= n_drop
         self._total_len = max_length

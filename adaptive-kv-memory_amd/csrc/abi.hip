@@ -11,6 +11,7 @@
 #include "prefill.h"
 #include "misc.h"
 #include "quant.h"
+#include "rows.h"
 
 namespace {
 
@@ -309,6 +310,7 @@ int64_t akv_struct_size(int32_t which) {
         case 3: return (int64_t)sizeof(akv_dequant_args);
         case 4: return (int64_t)sizeof(akv_importance_args);
         case 5: return (int64_t)sizeof(akv_prefill_args);
+        case 6: return (int64_t)sizeof(akv_rows_job);
         default: return -1;
     }
 }
@@ -827,6 +829,41 @@ int akv_importance_update_ws(const akv_importance_args *a, void *workspace, int6
 
 int akv_importance_update(const akv_importance_args *a, void *stream) {
     return akv_importance_update_ws(a, nullptr, 0, stream);
+}
+
+int akv_rows_move(const akv_rows_job *jobs, int32_t n_jobs, const int64_t *idx, int64_t n_idx, void *stream) {
+    if (n_jobs < 0 || n_jobs > akv::kRowsMaxJobs) return fail(AKV_E_SHAPE, "at most %d jobs", akv::kRowsMaxJobs);
+    if (n_jobs > 0 && !jobs) return fail(AKV_E_INVALID, "jobs is NULL");
+    if (n_idx < 0 || (n_idx > 0 && !idx)) return fail(AKV_E_INVALID, "bad index list");
+    for (int i = 0; i < n_jobs; ++i) {
+        const akv_rows_job &j = jobs[i];
+        if (j.kind < AKV_ROWS_COPY || j.kind > AKV_ROWS_COUNT || j.map < AKV_ROWS_SAME || j.map > AKV_ROWS_SCATTER)
+            return fail(AKV_E_INVALID, "unknown job kind or map");
+        if (j.n < 0 || j.B < 0 || j.H < 0 || j.row < 1 || j.row > (1 << 20) || j.limit < 0)
+            return fail(AKV_E_SHAPE, "bad job sizes");
+        if (j.n >= ((int64_t)1 << 31)) return fail(AKV_E_SHAPE, "too many rows");
+        if (j.n == 0 || j.B == 0 || j.H == 0) continue;
+        const bool reads = j.kind == AKV_ROWS_COPY || j.kind == AKV_ROWS_WIDEN;
+        if (!j.dst || (reads && !j.src)) return fail(AKV_E_INVALID, "null pointer");
+        if (!reads && j.map != AKV_ROWS_SAME) return fail(AKV_E_INVALID, "FILL and COUNT take the SAME map");
+        if ((j.map == AKV_ROWS_GATHER || j.map == AKV_ROWS_SCATTER) && n_idx < j.n)
+            return fail(AKV_E_SHAPE, "index list shorter than the job");
+        if (j.kind == AKV_ROWS_COPY && (j.elem < 1 || j.elem > 8)) return fail(AKV_E_DTYPE, "bad element size");
+        if (j.kind == AKV_ROWS_COUNT && j.elem != 4 && j.elem != 8) return fail(AKV_E_DTYPE, "bad element size");
+        if (j.kind == AKV_ROWS_WIDEN && (j.src_dt < 0 || j.src_dt > 2)) return fail(AKV_E_DTYPE, "bad source dtype");
+    }
+    hipError_t e = akv::rows_move_launch(jobs, n_jobs, idx, n_idx, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "row move launch");
+    return ok();
+}
+
+int akv_promote_select(const float *scores, const float *previous, float *proxy, int64_t n, float decay, float fresh,
+                       float threshold, int64_t cap, int64_t *out, void *stream) {
+    if (n < 1 || n >= ((int64_t)1 << 31) || cap < 1) return fail(AKV_E_SHAPE, "bad sizes");
+    if (!scores || !out || (previous && !proxy)) return fail(AKV_E_INVALID, "null pointer");
+    hipError_t e = akv::promote_launch(scores, previous, proxy, n, decay, fresh, threshold, cap, out, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "promote launch");
+    return ok();
 }
 
 }  // extern "C"

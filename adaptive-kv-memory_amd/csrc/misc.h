@@ -54,4 +54,8 @@ hipError_t zero_fill_launch(void *p, int64_t bytes, hipStream_t s);
 hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t n, int64_t pf, int64_t pl,
                          int64_t *out, hipStream_t s);
 
+// Promotion choice over one row of warm scores (akv_promote_select).
+hipError_t promote_launch(const float *scores, const float *previous, float *proxy, int64_t n, float decay, float fresh,
+                          float threshold, int64_t cap, int64_t *out, hipStream_t s);
+
 }  // namespace akv

@@ -515,16 +515,29 @@ __device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
 }
 }  // namespace
 
-// SLOTS 0: the row stays in memory.
-template <int SLOTS>
-__global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64_t len, int64_t n, int64_t pf,
-                                                      int64_t pl, int64_t *out) {
+// What a selection takes besides the row: of a demotion the protected ends, of a promotion
+// the score update, the threshold and the most rows it may take.
+struct SelectParams {
+    const float *scores;
+    int64_t len, n, pf, pl;
+    int64_t *out;
+    const float *previous;  // promotion: scores before this step (or NULL)
+    float *proxy;           // promotion: updated scores (or NULL: `scores` as they are)
+    float decay, fresh, threshold;
+};
+
+// SLOTS 0: the row stays in memory.  PROMOTE: the keys are inverted (the largest scores are
+// the smallest keys, NaN smallest), n is the smaller of p.n and the scores above the
+// threshold, and out starts with that count.
+template <int SLOTS, bool PROMOTE>
+__global__ __launch_bounds__(1024) void select_kernel(const SelectParams p) {
+    const int64_t len = p.len, n = p.n, pl = PROMOTE ? 0 : p.pl, pf = PROMOTE ? 0 : p.pf;
     extern __shared__ __align__(16) uint32_t sel_lds[];
     uint32_t *hist = sel_lds, *list = hist + kSelBins, *red = list + kSelList, *key_lds = red + 5 * 16;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const float *srow = scores + (int64_t)blockIdx.x * len;
-    int64_t *orow = out + (int64_t)blockIdx.x * n;
+    const float *srow = (PROMOTE && p.proxy ? p.proxy : p.scores) + (int64_t)blockIdx.x * len;
+    int64_t *orow = PROMOTE ? p.out + 1 : p.out + (int64_t)blockIdx.x * n;
     // len < 2^31: positions in 32 bits
     const uint32_t L = (uint32_t)len, rec = (uint32_t)(len - pl > 0 ? len - pl : 0);
     const uint32_t first = (uint32_t)(pf < len ? pf : len);
@@ -534,8 +547,21 @@ __global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64
     auto to_key = [&](int j, float x) -> uint32_t {
         const uint32_t i = i0 + 64u * (uint32_t)j;
         if (i >= L) return 0xFFFFFFFFu;
+        if (PROMOTE) return ~order_key(x);
         return (i < first || i >= rec) ? kKeyInf : order_key(x);
     };
+    if (PROMOTE && p.proxy) {  // a thread reads back only the scores it writes
+        for (int j = 0; j < nslot; ++j) {
+            const uint32_t i = i0 + 64u * (uint32_t)j;
+            if (i >= L) break;
+            float x = __builtin_fabsf(p.scores[i]);
+            if (p.previous) {
+                const float a = p.decay * p.previous[i], b = p.fresh * x;
+                x = a + b;
+            }
+            p.proxy[i] = x;
+        }
+    }
     uint32_t key_reg[SLOTS > 0 ? (SLOTS < kSelRegSlots ? SLOTS : kSelRegSlots) : 1];
     // f(slot, key) over this wave's slots
     auto each = [&](auto &&f) {
@@ -611,9 +637,30 @@ __global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64
         n_fin += red[32 + w];
         n_inf += red[48 + w];
     }
-    const uint32_t want = (uint32_t)n;
+    uint32_t want = (uint32_t)n;
+    const uint32_t above = PROMOTE ? ~order_key(p.threshold) : 0u;  // keys below it, NaN apart, are above the threshold
+    bool skip_nan = false;
+    if (PROMOTE) {
+        uint32_t c = 0;
+        each([&](int j, uint32_t k) {
+            c += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(k < above && k != 0u));
+        });
+        if (lane == 0) red[64 + wave] = c;
+        __syncthreads();
+        c = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) c += red[64 + w];
+        __syncthreads();  // red is written again below
+        skip_nan = c <= want;  // all of them; else the largest, NaN among them
+        want = min(want, c);
+        if (tid == 0) p.out[0] = (int64_t)want;
+        if (want == 0u) return;
+    }
     uint32_t tau, take_eq;  // the n-th smallest key; how many elements equal to it to take
-    if (want > n_fin) {
+    if (skip_nan) {
+        tau = above;
+        take_eq = 0u;
+    } else if (want > n_fin) {
         tau = want <= n_fin + n_inf ? kKeyInf : 0xFFFFFFFFu;
         take_eq = want - n_fin - (tau == kKeyInf ? 0u : n_inf);
     } else {
@@ -683,8 +730,9 @@ __global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64
     __syncthreads();
     uint32_t lt_run = 0, eq_run = 0;  // of this wave, then before its current slot
     auto is_eq = [&](int j, uint32_t key) { return key == tau && i0 + 64u * (uint32_t)j < L; };
+    auto is_lt = [&](uint32_t key) { return key < tau && !(PROMOTE && skip_nan && key == 0u); };
     each([&](int j, uint32_t key) {
-        lt_run += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(key < tau));
+        lt_run += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(is_lt(key)));
         eq_run += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(is_eq(j, key)));
     });
     if (lane == 0) {
@@ -698,7 +746,7 @@ __global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64
         eq_run += red[16 + w];
     }
     each([&](int j, uint32_t key) {
-        const bool lt = key < tau, eq = is_eq(j, key);
+        const bool lt = is_lt(key), eq = is_eq(j, key);
         const uint64_t ml = __builtin_amdgcn_ballot_w64(lt), me = __builtin_amdgcn_ballot_w64(eq);
         const uint32_t lt_before = lt_run + lanes_below(ml), eq_before = eq_run + lanes_below(me);
         if (lt || (eq && eq_before < take_eq))
@@ -708,16 +756,14 @@ __global__ __launch_bounds__(1024) void select_kernel(const float *scores, int64
     });
 }
 
-hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t n, int64_t pf, int64_t pl,
-                         int64_t *out, hipStream_t s) {
-    if (rows <= 0 || n <= 0) return hipSuccess;
-#define AKV_SEL(slots)                                                                                          \
-    hipLaunchKernelGGL(select_kernel<slots>, dim3((unsigned)rows), dim3(1024), sel_lds_bytes(slots), s, scores, len, \
-                       n, pf, pl, out)
-    if (len <= 2 * 1024) AKV_SEL(2);
-    else if (len <= 8 * 1024) AKV_SEL(8);
-    else if (len <= 32 * 1024) AKV_SEL(32);
-    else if (len <= 64 * 1024) {
+template <bool PROMOTE>
+static hipError_t select_dispatch(const SelectParams &p, int64_t rows, hipStream_t s) {
+#define AKV_SEL(slots) \
+    hipLaunchKernelGGL((select_kernel<slots, PROMOTE>), dim3((unsigned)rows), dim3(1024), sel_lds_bytes(slots), s, p)
+    if (p.len <= 2 * 1024) AKV_SEL(2);
+    else if (p.len <= 8 * 1024) AKV_SEL(8);
+    else if (p.len <= 32 * 1024) AKV_SEL(32);
+    else if (p.len <= 64 * 1024) {
         // raise the dynamic LDS cap above 64 KiB once per device (a bit per device index;
         // host threads that race here both set it, which is harmless)
         static std::atomic<uint64_t> attr_devs{0};
@@ -726,8 +772,8 @@ hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t
         if (e != hipSuccess) return e;
         const uint64_t bit = (dev >= 0 && dev < 64) ? 1ull << dev : 0ull;
         if (!bit || !(attr_devs.load(std::memory_order_acquire) & bit)) {
-            e = hipFuncSetAttribute((const void *)select_kernel<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    sel_lds_bytes(64));
+            e = hipFuncSetAttribute((const void *)select_kernel<64, PROMOTE>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, sel_lds_bytes(64));
             if (e != hipSuccess) return e;
             attr_devs.fetch_or(bit, std::memory_order_release);
         }
@@ -735,6 +781,20 @@ hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t
     } else AKV_SEL(0);
 #undef AKV_SEL
     return hipGetLastError();
+}
+hipError_t select_launch(const float *scores, int64_t rows, int64_t len, int64_t n, int64_t pf, int64_t pl,
+                         int64_t *out, hipStream_t s) {
+    if (rows <= 0 || n <= 0) return hipSuccess;
+    SelectParams p{};
+    p.scores = scores; p.len = len; p.n = n; p.pf = pf; p.pl = pl; p.out = out;
+    return select_dispatch<false>(p, rows, s);
+}
+hipError_t promote_launch(const float *scores, const float *previous, float *proxy, int64_t n, float decay, float fresh,
+                          float threshold, int64_t cap, int64_t *out, hipStream_t s) {
+    SelectParams p{};
+    p.scores = scores; p.len = n; p.n = cap < n ? cap : n; p.out = out;
+    p.previous = previous; p.proxy = proxy; p.decay = decay; p.fresh = fresh; p.threshold = threshold;
+    return select_dispatch<true>(p, 1, s);
 }
 
 hipError_t dequant_launch(const DequantParams &p, hipStream_t s) {

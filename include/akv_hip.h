@@ -340,7 +340,7 @@ int akv_abi_version(void);
 const char *akv_last_error(void);
 /* sizeof of the args structs, for bindings that mirror them (ctypes, cgo):
  * 0 akv_warm_desc, 1 akv_decode_args, 2 akv_quant_args, 3 akv_dequant_args,
- * 4 akv_importance_args, 5 akv_prefill_args; -1 for an unknown id. */
+ * 4 akv_importance_args, 5 akv_prefill_args, 6 akv_rows_job; -1 for an unknown id. */
 int64_t akv_struct_size(int32_t which);
 /* A measurement helper with no counterpart in the reference: reads `bytes` (a multiple of
  * 16, 16-byte aligned) once with 16-byte non-temporal loads, as fast as a read-once kernel
@@ -358,6 +358,49 @@ int akv_stream_read(const void *data, int64_t bytes, uint32_t *sink, void *strea
 int64_t akv_timeline_words(void);
 int akv_timeline_fetch(uint64_t *host, int64_t words);
 int akv_timeline_clear(void *stream);
+
+/* ------------------------------------------------------------- row moves */
+
+/* What a job does with its rows of `row` elements, n of them for each of B x H (batch, head)s:
+ * COPY the `elem`-byte elements as they are; WIDEN src_dt (float16, bfloat16 or float32) to
+ * float32 times `value`; FILL float32 `value`; COUNT start + step * (destination row) as
+ * `elem` = 4 or 8 byte integers.  FILL and COUNT read no source. */
+#define AKV_ROWS_COPY 0
+#define AKV_ROWS_WIDEN 1
+#define AKV_ROWS_FILL 2
+#define AKV_ROWS_COUNT 3
+/* Which rows: SAME row t to row t; KEEP the t-th row not in the call's ascending list to row
+ * t; GATHER row idx[t] to row t; SCATTER row t to row idx[t].  Rows read (SCATTER: written)
+ * outside [0, limit) are skipped. */
+#define AKV_ROWS_SAME 0
+#define AKV_ROWS_KEEP 1
+#define AKV_ROWS_GATHER 2
+#define AKV_ROWS_SCATTER 3
+
+typedef struct akv_rows_job {
+    const void *src;
+    void *dst;
+    int64_t src_b, src_h, src_t; /* byte strides of batch, head and token row */
+    int64_t dst_b, dst_h, dst_t;
+    int64_t n, limit;
+    int64_t start, step;
+    int32_t B, H, row, elem;
+    int32_t kind, map, src_dt;
+    float value;
+} akv_rows_job;
+
+/* Up to 12 jobs in one launch (jobs of one call must not overlap in memory).  idx: int64 list
+ * of n_idx entries on the device (KEEP: ascending and distinct). */
+int akv_rows_move(const akv_rows_job *jobs, int32_t n_jobs, const int64_t *idx, int64_t n_idx, void *stream);
+
+/* The promotion choice over n float32 warm scores: with `proxy` not NULL they are
+ * |scores|, or decay * previous + fresh * |scores| when `previous` is not NULL (one rounding
+ * an operation), and are written to `proxy` (which may be `previous`); else `scores` itself.
+ * out (1 + cap int64): how many were chosen, then their ascending indices: the scores above
+ * `threshold`, or the `cap` largest (NaN largest, equal ones lowest index first) when more
+ * are above it. */
+int akv_promote_select(const float *scores, const float *previous, float *proxy, int64_t n, float decay, float fresh,
+                       float threshold, int64_t cap, int64_t *out, void *stream);
 
 #ifdef __cplusplus
 }
