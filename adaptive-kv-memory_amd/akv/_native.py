@@ -133,6 +133,15 @@ class RowsJob(ctypes.Structure):
     ]
 
 
+class KiviSide(ctypes.Structure):
+    _fields_ = [
+        ("src", _vp), ("src_b", _i64), ("src_h", _i64), ("src_t", _i64),
+        ("codes", _vp), ("scale", _vp), ("zero", _vp), ("scale16", _vp), ("zero16", _vp),
+        ("view", _vp), ("cap", _i64), ("row0", _i64), ("zero_to", _i64), ("view_rows", _i64),
+        ("bits", _i32), ("_pad0", _i32),
+    ]
+
+
 EXPORTS = (
     "akv_abi_version", "akv_last_error", "akv_struct_size",
     "akv_decode_workspace_bytes", "akv_decode_counter_bytes", "akv_decode_attn", "akv_decode_attn_noalloc",
@@ -140,10 +149,10 @@ EXPORTS = (
     "akv_bitpack", "akv_bitunpack", "akv_importance_update",
     "akv_importance_workspace_bytes", "akv_importance_update_ws",
     "akv_prefill_workspace_bytes", "akv_prefill_attn", "akv_select_demote", "akv_stream_read",
-    "akv_rows_move", "akv_promote_select",
+    "akv_rows_move", "akv_promote_select", "akv_kivi_append",
     "akv_timeline_words", "akv_timeline_fetch", "akv_timeline_clear",
 )
-STRUCTS = (WarmDesc, DecodeArgs, QuantArgs, DequantArgs, ImportanceArgs, PrefillArgs, RowsJob)
+STRUCTS = (WarmDesc, DecodeArgs, QuantArgs, DequantArgs, ImportanceArgs, PrefillArgs, RowsJob, KiviSide)
 
 _lib: Optional[ctypes.CDLL] = None
 
@@ -198,6 +207,8 @@ def load() -> ctypes.CDLL:
     lib.akv_rows_move.argtypes = [ctypes.POINTER(RowsJob), _i32, _vp, _i64, _vp]
     lib.akv_promote_select.restype = ctypes.c_int
     lib.akv_promote_select.argtypes = [_vp, _vp, _vp, _i64, ctypes.c_float, ctypes.c_float, ctypes.c_float, _i64, _vp, _vp]
+    lib.akv_kivi_append.restype = ctypes.c_int
+    lib.akv_kivi_append.argtypes = [ctypes.POINTER(KiviSide), _i32, _i32, _i32, _i32, _i64, _i32, _i32, _i32, _vp]
     lib.akv_stream_read.restype = ctypes.c_int
     lib.akv_stream_read.argtypes = [_vp, _i64, _vp, _vp]
     lib.akv_timeline_words.restype = _i64

@@ -5,10 +5,11 @@ full-precision residual window; ``KIVIFusedCache`` (:426-510) is its fused-kerne
 cost profile: each overflow chunk is quantized once, appended, and dequantized once
 into a float16 working copy.  The quantizer (``_quantize_tensor``, :345-370) is fp32
 min / max per (row, group) of the last axis, scale clamped at 1e-10, codes
-rounded half-to-even; here it is one ``akv_quant_pack`` launch (layout
+rounded half-to-even; for KIVICache it is one ``akv_quant_pack`` launch (layout
 ``AKV_QUANT_ARENA`` on fp32 input, which is that arithmetic) and the dequant
 (``_dequantize_tensor``, :372-380: fp32 ``codes * s + z`` cast to fp16) one
-``akv_dequant_unpack`` launch -- both bit-exact with the reference.
+``akv_dequant_unpack`` launch -- both bit-exact with the reference -- and for
+KIVIFusedCache one ``akv_kivi_append`` launch does both for an overflow's keys and values.
 
 Storage: per layer and for K and V, the codes bit-packed (2 / 4 / 8 bits; 4-bit
 high nibble first, 2-bit MSB first) in ``[B * H][capacity][pD * bits / 8]`` and the
@@ -38,6 +39,7 @@ import torch
 
 from . import _native as nat
 from ._legacy import legacy_desc, padded_dim
+from .row_moves import RowMoves, movable
 
 
 @dataclass
@@ -91,14 +93,15 @@ def quantize_rows(x: torch.Tensor, bits: int, group_size: int):
 
 
 def dequantize_rows(codes: torch.Tensor, sc: torch.Tensor, ze: torch.Tensor, bits: int, group_size: int,
-                    D: int, n: Optional[int] = None) -> torch.Tensor:
+                    D: int, n: Optional[int] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """KIVICache._dequantize_tensor (akv/baselines.py:372-380): (R, n, D) float16 of
     fp32 codes * s + z, for contiguous codes (R, S, pD * bits / 8) and fp32 meta
     (R, S, G) of which the first n <= S tokens of each row are read (n = S unless
-    given), in one launch."""
+    given), in one launch; into the first n of the rows of ``out`` (R, >= n, D) if given."""
     R, S = codes.shape[0], codes.shape[1]
     n = S if n is None else n
-    out = torch.empty(R, n, D, dtype=torch.float16, device=codes.device)
+    if out is None:
+        out = torch.empty(R, n, D, dtype=torch.float16, device=codes.device)
     if R * n == 0:
         return out
     keep = []
@@ -111,6 +114,7 @@ def dequantize_rows(codes: torch.Tensor, sc: torch.Tensor, ze: torch.Tensor, bit
     a.out_dtype = nat.DT_F16
     a.warm = desc
     a.k_out = out.data_ptr()
+    a.out_tokens = out.shape[1]
     nat.check(nat.load().akv_dequant_unpack(ctypes.byref(a), nat.stream_of(out)), "KIVI dequantize")
     return out
 
@@ -144,6 +148,27 @@ class _Tier:
             self.sc16 = grow(self.sc16, (R, cap, G), torch.float16)
             self.ze16 = grow(self.ze16, (R, cap, G), torch.float16)
         self.cap = cap
+
+    def reserve(self, n: int) -> int:
+        """Room for n more rows; where the tier grew, the row up to which the caller has to
+        clear those past its own (rows past the tier read as zeros), else 0."""
+        if self.n + n <= self.cap:
+            return 0
+        cap = max(64, self.cap)
+        while cap < self.n + n:
+            cap *= 2
+        mv = RowMoves()
+        for name, width, dtype in (("codes", self.row_bytes, torch.uint8), ("sc", self.G, torch.float32),
+                                   ("ze", self.G, torch.float32), ("sc16", self.G, torch.float16),
+                                   ("ze16", self.G, torch.float16)):
+            if self.keep_f16 or not name.endswith("16"):
+                old, new = getattr(self, name), torch.empty(self.rows, cap, width, dtype=dtype, device=self.device)
+                if old is not None:
+                    mv.copy(new.unsqueeze(0), old.unsqueeze(0), self.n)
+                setattr(self, name, new)
+        mv.run()
+        self.cap = cap
+        return cap
 
     def append(self, codes, sc, ze):
         n = codes.shape[1]
@@ -260,48 +285,98 @@ class KIVICache:
 
 
 class KIVIFusedCache(KIVICache):
-    """akv/baselines.py:426-510: incremental quantization of each overflow chunk and a
-    float16 working copy extended by that chunk's dequant only."""
+    """akv/baselines.py:426-510: incremental quantization of each overflow chunk.  The
+    reference keeps a float16 working copy extended by that chunk's dequant; the same values
+    come from the packed tier here, dequantized straight into each returned view."""
 
     _keep_f16 = True
 
     def __init__(self, config: Optional[KIVIFusedConfig] = None):
         super().__init__(config or KIVIFusedConfig())
-        self._dequant_keys_cache: dict = {}
+        self._dequant_keys_cache: dict = {}    # layer -> the tier its dequantized rows come from
         self._dequant_values_cache: dict = {}
+        self._views: dict = {}  # layer -> (view, rows before the chunk) between an overflow and its view
         self._ws: dict = {}  # per-device decode workspace of fused_attention
 
     def _quantize_overflow(self, layer_idx: int):
-        """akv/baselines.py:455-496."""
+        """akv/baselines.py:455-496.  One launch quantizes, appends and dequantizes the
+        overflow of both tensors and writes its rows of the view that ``_get_full_kv`` then
+        completes; one more cuts the residuals."""
         cfg = self.config
-        res_k, res_v = self._residual_keys[layer_idx], self._residual_values[layer_idx]
-        n_q = res_k.shape[2] - cfg.residual_length
-        tk, tv = res_k[:, :, :n_q], res_v[:, :, :n_q]
-        B, H, _, D = res_k.shape
-        if layer_idx not in self._quant_keys:
-            self._quant_keys[layer_idx] = self._new_tier(tk, cfg.key_bits)
-            self._quant_values[layer_idx] = self._new_tier(tv, cfg.value_bits)
-        kq = quantize_rows(tk, cfg.key_bits, cfg.group_size)
-        vq = quantize_rows(tv, cfg.value_bits, cfg.group_size)
-        self._quant_keys[layer_idx].append(*kq)
-        self._quant_values[layer_idx].append(*vq)
-        nk = dequantize_rows(*kq, cfg.key_bits, cfg.group_size, D).view(B, H, n_q, D)
-        nv = dequantize_rows(*vq, cfg.value_bits, cfg.group_size, D).view(B, H, n_q, D)
-        if layer_idx in self._dequant_keys_cache:
-            self._dequant_keys_cache[layer_idx] = torch.cat([self._dequant_keys_cache[layer_idx], nk], dim=2)
-            self._dequant_values_cache[layer_idx] = torch.cat([self._dequant_values_cache[layer_idx], nv], dim=2)
-        else:
-            self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx] = nk, nv
-        self._residual_keys[layer_idx] = res_k[:, :, n_q:].contiguous()
-        self._residual_values[layer_idx] = res_v[:, :, n_q:].contiguous()
+        res = (self._residual_keys, self._residual_values)
+        for bits, r in ((cfg.key_bits, res[0]), (cfg.value_bits, res[1])):
+            _check_shape(r[layer_idx].shape[3], bits, cfg.group_size)
+        sides, views = [], [None, None]
+        for i, (bits, tiers, served) in enumerate(((cfg.key_bits, self._quant_keys, self._dequant_keys_cache),
+                                                  (cfg.value_bits, self._quant_values, self._dequant_values_cache))):
+            r = res[i][layer_idx]
+            B, H, n_all, D = r.shape
+            n_q = n_all - cfg.residual_length
+            x, left = r[:, :, :n_q], r[:, :, n_q:]
+            n = x.shape[2]
+            if layer_idx not in tiers:
+                tiers[layer_idx] = self._new_tier(x, bits)
+            tier = served[layer_idx] = tiers[layer_idx]
+            grown = tier.reserve(n)
+            if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
+                x = x.float()
+            e = x.element_size()
+            if x.stride(3) != 1 or x.data_ptr() % 16 or any(st * e % 16 for st in x.stride()[:3]):
+                x = nat.dev_contig(x)
+            dt = torch.promote_types(torch.float16, left.dtype)
+            view = None
+            if movable(dt, left) and dt in (torch.float16, torch.float32):
+                view = torch.empty(B, H, tier.n + n + left.shape[2], D, dtype=dt, device=r.device)
+                views[i] = (view, tier.n)
+            sides.append((x, B, H, D, n, dt, nat.KiviSide(
+                x.data_ptr(), x.stride(0) * e, x.stride(1) * e, x.stride(2) * e, tier.codes.data_ptr(),
+                tier.sc.data_ptr(), tier.ze.data_ptr(), tier.sc16.data_ptr(), tier.ze16.data_ptr(),
+                None if view is None else view.data_ptr(), tier.cap, tier.n, grown,
+                0 if view is None else view.shape[2], bits, 0)))
+            tier.n += n
+        groups = [sides] if sides[0][1:6] == sides[1][1:6] and sides[0][0].dtype == sides[1][0].dtype else [sides[:1], sides[1:]]
+        for g in groups:
+            x, B, H, D, n, dt, _ = g[0]
+            arr = (nat.KiviSide * len(g))(*(s[6] for s in g))
+            nat.check(nat.load().akv_kivi_append(
+                arr, len(g), B, H, D, n, nat.dtype_code(x.dtype), cfg.group_size,
+                nat.DT_F16 if dt == torch.float16 else nat.DT_F32, nat.stream_of(x)), "KIVI append")
+        mv = RowMoves()
+        for i in (0, 1):
+            r = res[i][layer_idx]
+            left = r[:, :, r.shape[2] - cfg.residual_length:]
+            if movable(left.dtype, left) and left.stride(3) == 1:
+                new = torch.empty(left.shape, dtype=left.dtype, device=left.device)
+                mv.copy(new, left, left.shape[2])
+                res[i][layer_idx] = new
+            else:
+                res[i][layer_idx] = left.contiguous()
+        mv.run()
+        self._views[layer_idx] = views
 
     def _get_full_kv(self, layer_idx: int):
         """akv/baselines.py:498-510."""
-        rk, rv = self._residual_keys[layer_idx], self._residual_values[layer_idx]
-        if layer_idx in self._dequant_keys_cache:
-            return (torch.cat([self._dequant_keys_cache[layer_idx], rk], dim=2),
-                    torch.cat([self._dequant_values_cache[layer_idx], rv], dim=2))
-        return rk, rv
+        rs = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
+        if layer_idx not in self._dequant_keys_cache:
+            return rs
+        mv, out, views = RowMoves(), [], self._views.pop(layer_idx, [None, None])
+        for i, tier in enumerate((self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx])):
+            n, r = tier.n, rs[i]
+            dt = torch.promote_types(torch.float16, r.dtype)
+            if not movable(dt, r) or r.shape[:2] != (tier.B, tier.H) or r.shape[3] != tier.D:
+                out.append(torch.cat([tier.dequantize(), r], dim=2))
+                continue
+            view, had = views[i] or (torch.empty(tier.B, tier.H, n + r.shape[2], tier.D, dtype=dt, device=r.device), n)
+            if had and dt == torch.float16:  # the rows the overflow launch has not written
+                dequantize_rows(tier.codes, tier.sc, tier.ze, tier.bits, tier.gs, tier.D, n=had,
+                                out=view.view(tier.rows, view.shape[2], tier.D))
+            elif had:
+                old = dequantize_rows(tier.codes, tier.sc, tier.ze, tier.bits, tier.gs, tier.D, n=had)
+                mv.copy(view, old.view(tier.B, tier.H, had, tier.D), had)
+            mv.copy(view, r if r.stride(3) == 1 else r.contiguous(), r.shape[2], at=n)
+            out.append(view)
+        mv.run()
+        return out[0], out[1]
 
     def fused_attention(self, query: torch.Tensor, layer_idx: int, sm_scale: Optional[float] = None) -> torch.Tensor:
         """softmax(q K^T * sm_scale) V over the layer's quantized tier (in place) and its

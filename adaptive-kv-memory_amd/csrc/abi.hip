@@ -8,6 +8,7 @@
 
 #include "akv_common.h"
 #include "decode.h"
+#include "kivi.h"
 #include "prefill.h"
 #include "misc.h"
 #include "quant.h"
@@ -311,6 +312,7 @@ int64_t akv_struct_size(int32_t which) {
         case 4: return (int64_t)sizeof(akv_importance_args);
         case 5: return (int64_t)sizeof(akv_prefill_args);
         case 6: return (int64_t)sizeof(akv_rows_job);
+        case 7: return (int64_t)sizeof(akv_kivi_side);
         default: return -1;
     }
 }
@@ -635,7 +637,9 @@ int akv_dequant_unpack(const akv_dequant_args *a, void *stream) {
     if (a->out_slot && a->out_tokens < 1) return fail(AKV_E_SHAPE, "out_slot needs out_tokens >= 1");
     p.tok_stride = w.token_stride > 0 ? w.token_stride : w.n_warm;
     p.out_slot = a->out_slot;
-    p.out_tokens = a->out_tokens;
+    const bool strided = w.kind == AKV_WARM_LEGACY && a->out_tokens != 0;
+    if (strided && a->out_tokens < w.n_warm) return fail(AKV_E_SHAPE, "out_tokens < n_warm");
+    p.out_tokens = a->out_slot || strided ? a->out_tokens : w.n_warm;
     if (w.kind == AKV_WARM_AFFINE) {
         for (int bits : {w.bits_k, w.bits_v})
             if ((bits < 2 || bits > 4) && bits != 8) return fail(AKV_E_BITS, "Unsupported bits: %d", bits);
@@ -854,6 +858,34 @@ int akv_rows_move(const akv_rows_job *jobs, int32_t n_jobs, const int64_t *idx, 
     }
     hipError_t e = akv::rows_move_launch(jobs, n_jobs, idx, n_idx, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "row move launch");
+    return ok();
+}
+
+int akv_kivi_append(const akv_kivi_side *sides, int32_t n_sides, int32_t B, int32_t H, int32_t D, int64_t n,
+                    int32_t in_dtype, int32_t group_size, int32_t view_dtype, void *stream) {
+    if (!sides || n_sides < 1 || n_sides > 2) return fail(AKV_E_INVALID, "one or two tensors");
+    if (B < 0 || H < 0 || n < 0 || n >= ((int64_t)1 << 31)) return fail(AKV_E_SHAPE, "bad sizes");
+    if ((int64_t)B * H > 65535) return fail(AKV_E_SHAPE, "more than 65535 (batch, head)s");
+    if (D != 64 && D != 128) return fail(AKV_E_UNSUPPORTED, "head_dim 64 or 128");
+    if (group_size != 32 && group_size != 64 && group_size != 128) return fail(AKV_E_UNSUPPORTED, "group_size 32, 64 or 128");
+    if (in_dtype < 0 || in_dtype > 2 || (view_dtype != AKV_DT_F16 && view_dtype != AKV_DT_F32))
+        return fail(AKV_E_DTYPE, "bad dtype");
+    akv::KiviParams p{};
+    p.B = B; p.H = H; p.D = D; p.n = n; p.in_dt = in_dtype; p.group_size = group_size; p.view_dt = view_dtype;
+    for (int i = 0; i < n_sides && n > 0 && B > 0 && H > 0; ++i) {
+        const akv_kivi_side &s = sides[i];
+        if (s.bits != 2 && s.bits != 4 && s.bits != 8) return fail(AKV_E_BITS, "Unsupported bits: %d", s.bits);
+        if (!s.src || !s.codes || !s.scale || !s.zero || !s.scale16 != !s.zero16)
+            return fail(AKV_E_INVALID, "null pointer");
+        if (!aligned16(s.src) || !aligned16(s.codes) || !aligned16(s.view) ||
+            ((s.src_b | s.src_h | s.src_t) & 15))
+            return fail(AKV_E_ALIGN, "rows must be 16-byte aligned");
+        if (s.row0 < 0 || s.row0 + n > s.cap || s.zero_to > s.cap || (s.view && s.row0 + n > s.view_rows))
+            return fail(AKV_E_SHAPE, "rows past a buffer's end");
+        p.side[i] = s;
+    }
+    hipError_t e = akv::kivi_append_launch(p, n_sides, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "KIVI append launch");
     return ok();
 }
 

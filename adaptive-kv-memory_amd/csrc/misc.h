@@ -26,7 +26,7 @@ struct DequantParams {
     const int32_t *blk_of;        // affine: K-meta / outlier block of each token (else t / T)
     int64_t tok_stride;           // token rows per (bh) of codes, V meta, outlier values
     const int64_t *out_slot;      // output token row of each token (else the token's own row)
-    int64_t out_tokens;           // output token rows per (bh) when out_slot is set
+    int64_t out_tokens;           // output token rows per (bh)
 };
 
 struct ImportanceParams {

@@ -21,7 +21,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const DequantParams p) {
     const int64_t bh = task / nch / p.n_warm, t = task / nch % p.n_warm;
     const int64_t row = bh * p.tok_stride + t;  // input row (bh, token)
     const int64_t blk = p.blk_of ? (int64_t)p.blk_of[t] : t / p.T;
-    const int64_t orow = p.out_slot ? bh * p.out_tokens + p.out_slot[t] : bh * p.n_warm + t;
+    const int64_t orow = bh * p.out_tokens + (p.out_slot ? p.out_slot[t] : t);
     for (int which = 0; which < 2; ++which) {
         void *out = which == 0 ? p.k_out : p.v_out;
         if (!out) continue;
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void dequant_chunk_kernel(const DequantParams 
 #pragma unroll
     for (int i = 0; i < kDqTok; ++i) {
         const int64_t t = min(t0 + (int64_t)i * per, p.n_warm - 1), row = bh * p.tok_stride + t;
-        orow[i] = p.out_slot ? bh * p.out_tokens + p.out_slot[t] : bh * p.n_warm + t;
+        orow[i] = bh * p.out_tokens + (p.out_slot ? p.out_slot[t] : t);
         chunk_codes(codes + row * row_bytes, ch8, bits, c[i]);
         if (AFFINE) {
             blk[i] = p.blk_of ? (int64_t)p.blk_of[t] : (int64_t)((uint32_t)t / (uint32_t)p.T);

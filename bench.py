@@ -675,7 +675,7 @@ def bench_kivi(args):
                                   "variant)",
                         "algorithmic_bytes_per_launch": alg, "us_per_launch": round(us_layer, 3)},
            "reference_design_gpu": {"us_per_layer": round(ref_ms * 1e3 / L, 3),
-                                    "what": "float16 working copy + residual concatenated, torch "
+                                    "what": "dequantized rows + residual as one float16 view, torch "
                                             "matmul/softmax/matmul"}}
     add_stream_reference(res["roofline"])
     if not args.no_cpu_baseline:

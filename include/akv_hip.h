@@ -237,7 +237,7 @@ typedef struct akv_dequant_args {
                                       batch element when block_of_token is given */
     const int64_t *out_slot;       /* [Nw] output token row of each warm token: the outputs are then
                                       [B][Hkv][out_tokens][D] and other rows are not written */
-    int64_t out_tokens;
+    int64_t out_tokens;            /* with out_slot, or LEGACY: output token rows per head (LEGACY 0: Nw) */
 } akv_dequant_args;
 
 /* Unpack + dequantize a warm tier to dense values, bit-exact with
@@ -340,7 +340,7 @@ int akv_abi_version(void);
 const char *akv_last_error(void);
 /* sizeof of the args structs, for bindings that mirror them (ctypes, cgo):
  * 0 akv_warm_desc, 1 akv_decode_args, 2 akv_quant_args, 3 akv_dequant_args,
- * 4 akv_importance_args, 5 akv_prefill_args, 6 akv_rows_job; -1 for an unknown id. */
+ * 4 akv_importance_args, 5 akv_prefill_args, 6 akv_rows_job, 7 akv_kivi_side; -1 for an unknown id. */
 int64_t akv_struct_size(int32_t which);
 /* A measurement helper with no counterpart in the reference: reads `bytes` (a multiple of
  * 16, 16-byte aligned) once with 16-byte non-temporal loads, as fast as a read-once kernel
@@ -392,6 +392,26 @@ typedef struct akv_rows_job {
 /* Up to 12 jobs in one launch (jobs of one call must not overlap in memory).  idx: int64 list
  * of n_idx entries on the device (KEEP: ascending and distinct). */
 int akv_rows_move(const akv_rows_job *jobs, int32_t n_jobs, const int64_t *idx, int64_t n_idx, void *stream);
+
+/* One tensor (keys or values) of akv_kivi_append: the tier's rows of (batch, head) r start at
+ * row r * cap, the new tokens' at row0 of it; the view likewise at r * view_rows (NULL: none).  Rows [row0 + n, zero_to) of codes, scales and zeros are cleared. */
+typedef struct akv_kivi_side {
+    const void *src;                 /* [B][H][n][D] with these byte strides, rows on 16 bytes */
+    int64_t src_b, src_h, src_t;
+    void *codes;                     /* packed rows of ceil(D / group_size) * group_size codes */
+    void *scale, *zero;              /* float32, one per group */
+    void *scale16, *zero16;          /* float16 copies, or NULL */
+    void *view;                      /* the dequantized float16 values, in view_dtype */
+    int64_t cap, row0, zero_to, view_rows;
+    int32_t bits, _pad0;             /* 2, 4 or 8 */
+} akv_kivi_side;
+
+/* Quantize n tokens per (batch, head) by groups of a token's channels (KIVICache's
+ * _quantize_tensor, akv/baselines.py:345-380), append them packed to a tier and write their
+ * dequantized values, for one or two tensors of the same shape in one launch.  D 64 or 128,
+ * group_size 32, 64 or 128; view_dtype float16 or float32. */
+int akv_kivi_append(const akv_kivi_side *sides, int32_t n_sides, int32_t B, int32_t H, int32_t D, int64_t n,
+                    int32_t in_dtype, int32_t group_size, int32_t view_dtype, void *stream);
 
 /* The promotion choice over n float32 warm scores: with `proxy` not NULL they are
  * |scores|, or decay * previous + fresh * |scores| when `previous` is not NULL (one rounding
