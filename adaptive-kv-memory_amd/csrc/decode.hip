@@ -908,7 +908,9 @@ __global__ __launch_bounds__(256) void weights_importance_kernel(const DecodePar
 constexpr int kWsQuads = AKV_WS_QUADS;
 // RB: rows per thread and batch of loads, chosen by the host so that one batch covers
 // every row when there are few (the 32k Qwen layer: 96 rows, 3 per thread), else 8.
-template <bool VEC, int RB>
+// Rows of any length: the 16-byte accesses need dword alignment only.
+typedef f4 f4_dword __attribute__((aligned(4)));
+template <int RB>
 __global__ __launch_bounds__(256) void weights_stats_kernel(const DecodeParams p) {
     constexpr int NQ = kWsQuads, TPW = 4 * NQ, NRL = 256 / NQ;  // tokens per workgroup, row lanes
     __shared__ float red[NRL][TPW + 1];
@@ -933,8 +935,8 @@ __global__ __launch_bounds__(256) void weights_stats_kernel(const DecodeParams p
                 M[j] = p.rowstats[2 * r];
                 W[j] = p.rowstats[2 * r + 1];
                 const float *src = p.stash + r * N + n0;
-                if (VEC && n0 + 3 < N) {
-                    x[j] = __builtin_nontemporal_load((const f4 *)src);  // read once
+                if (n0 + 3 < N) {
+                    x[j] = __builtin_nontemporal_load((const f4_dword *)src);  // read once
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -955,8 +957,8 @@ __global__ __launch_bounds__(256) void weights_stats_kernel(const DecodeParams p
             }
             if (p.attn_out) {
                 float *dst = p.stash + r * N + n0;
-                if (VEC && n0 + 3 < N) {
-                    *(f4 *)dst = w;
+                if (n0 + 3 < N) {
+                    *(f4_dword *)dst = w;
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -1183,11 +1185,7 @@ hipError_t decode_launch(const DecodeParams &p, int kb, int vb, int wk, const in
         const dim3 g((unsigned)((nmax + 4 * kWsQuads - 1) / (4 * kWsQuads)));
         constexpr int NRL = 256 / kWsQuads;
         const int64_t per = (rows + NRL - 1) / NRL;  // rows per thread
-#define AKV_WS(RB)                                                                                 \
-    do {                                                                                           \
-        if (p.N % 4 == 0) hipLaunchKernelGGL((weights_stats_kernel<true, RB>), g, dim3(256), 0, s, p); \
-        else hipLaunchKernelGGL((weights_stats_kernel<false, RB>), g, dim3(256), 0, s, p);        \
-    } while (0)
+#define AKV_WS(RB) hipLaunchKernelGGL(weights_stats_kernel<RB>, g, dim3(256), 0, s, p)
         if (per <= 1) AKV_WS(1);
         else if (per <= 2) AKV_WS(2);
         else if (per <= 3) AKV_WS(3);

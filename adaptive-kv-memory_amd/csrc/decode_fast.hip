@@ -212,8 +212,8 @@ __device__ __forceinline__ void issue_hot(u4 r, unsigned char *slot, int lane, i
 }
 
 // Raw logits q.k of 4 consecutive tokens of one row (the weights kernels take them to
-// the log2 domain): one 16-byte store when all 4 are valid and the row offset is
-// 16-byte aligned (vec), else one per token.  The 16-byte stores write through to the
+// the log2 domain): one 16-byte store (at any dword: rows of odd length and segments
+// off 16 bytes too) when all 4 are valid and the rows fit a buffer (vec), else one per token.  The 16-byte stores write through to the
 // device coherence point (cache policy sc1): the stash leaves during the kernel instead
 // of in the end-of-kernel L2 write-back (measured 0.35 us per layer faster at the 32k
 // workload).  Whole warm units take a cheaper path in the loop itself.
@@ -354,17 +354,14 @@ void decode_fast_kernel(const DecodeParams p) {
     const _Float16 hofk = (_Float16)(symk ? p.half_max_k : 0.f), hofv = (_Float16)(symv ? p.half_max_v : 0.f);
     const int64_t warm_base = p.hot_first ? p.n_hot : 0;  // logical position of warm token 0
     const int64_t hot_base = p.hot_first ? 0 : p.n_warm;
-    // the stash rows are N floats apart: 16-byte stores need N and the segment base divisible by 4
     // the stash rows of this (batch, kv-head) as one buffer (byte offsets below 2^31)
     const int64_t sbase = ((int64_t)(b * p.Hq + kvh * p.g) * p.M) * p.N;
     const bool st_buf_ok = (int64_t)p.R * p.N * 4 < ((int64_t)1 << 31);
     const __amdgpu_buffer_rsrc_t srs =
         make_rsrc(p.stash ? p.stash + sbase : p.stash, st_buf_ok ? (uint32_t)(p.R * p.N * 4) : 0u);
-    const bool st_vec_w = st_buf_ok && p.N % 4 == 0 && warm_base % 4 == 0,
-               st_vec_h = st_buf_ok && p.N % 4 == 0 && hot_base % 4 == 0;
     // byte offset of the lane's 4 logits of warm token 0 within those rows (a whole unit's
     // stores add its token offset as the scalar operand)
-    const uint32_t st_w_voff = st_vec_w ? (uint32_t)((strow - sbase + warm_base + 4 * grp) * 4) : 0u;
+    const uint32_t st_w_voff = st_buf_ok ? (uint32_t)((strow - sbase + warm_base + 4 * grp) * 4) : 0u;
 
     // this workgroup's items: warm 32-token units, then hot 16-token tiles (the
     // cheap hot items come last and even out the waves' finishing times)
@@ -387,12 +384,12 @@ void decode_fast_kernel(const DecodeParams p) {
             LEG ? (p.warm_heads == 1 ? 0 : p.warm_heads == p.Hkv ? (int64_t)kvh : bh) * p.w_stride : bh * p.n_warm;
         R.kc = rsrc4((const unsigned char *)p.kc + wrow * L::KR, nwu * L::KR);
         R.vc = rsrc4((const unsigned char *)p.vc + wrow * L::VR, nwu * L::VR);
-        // Per-token meta: with 4 groups a unit's rows are loaded a dword per lane, and every
-        // dword ends on a token; with 1 or 2 groups they come in 16-byte loads, and a load that
-        // crosses the end of the range may be dropped whole by the range check, so the range is
-        // rounded up to 16 bytes (the base is 16-byte aligned, so the last load lies in the
-        // page of its first byte) and the rows past the tier are cleared in LDS before use.
-        const uint32_t mrec = NG == 4 ? nwu * 8u : (nwu * NG * 2 + 15u) & ~15u;
+        // Per-token meta rows: the range check works on dwords, and with 4 or 2 groups every
+        // dword ends on a token.  With 1 group the last token of an odd tier is half a dword, so
+        // the range is rounded up to one (the base is dword-aligned, see
+        // decode_fast_meta_aligned, so it stays in the page of its first byte) and the rows past
+        // the tier are cleared in LDS before use.
+        const uint32_t mrec = (nwu * NG * 2 + 3u) & ~3u;
         if (LEG) {
             R.ks = rsrc4((const _Float16 *)p.ks + wrow * NG, mrec);
             R.kz = rsrc4((const _Float16 *)p.kz + wrow * NG, mrec);
@@ -566,8 +563,8 @@ void decode_fast_kernel(const DecodeParams p) {
 #else
         wait_head();
 #endif
-        if (NG < 4 && id * kUnit + kUnit > nw) {
-            // the tail unit: meta rows past the tier's last token may hold bytes from outside it
+        if (NG == 1 && id * kUnit + kUnit > nw) {
+            // the tail unit: the meta row past the tier's last token may hold bytes from outside it
             const int t = lane & 31;
             if (lane < 32 && t >= nw - id * kUnit) {
 #pragma unroll
@@ -799,7 +796,7 @@ void decode_fast_kernel(const DecodeParams p) {
                 }
             }
             if (p.stash) {
-                if (st_vec_w && tok0 + kUnit <= nw) {  // a whole unit: two 16-byte stores per lane
+                if (st_buf_ok && tok0 + kUnit <= nw) {  // a whole unit: two 16-byte stores per lane
                     if (row_valid) {
 #pragma unroll
                         for (int h = 0; h < 2; ++h)
@@ -811,7 +808,7 @@ void decode_fast_kernel(const DecodeParams p) {
                     for (int h = 0; h < 2; ++h) {
                         const int t0 = tok0 + 16 * h;
                         stash4(p, strow, row_valid, warm_base + t0 + 4 * grp, sc[h], min(4, nw - (t0 + 4 * grp)),
-                               st_vec_w, srs, sbase);
+                               st_buf_ok, srs, sbase);
                     }
                 }
             }
@@ -1004,7 +1001,7 @@ void decode_fast_kernel(const DecodeParams p) {
                 for (int ii = 0; ii < 4; ++ii)
                     if (ii >= nvalid) sh[ii] = -INFINITY;
             }
-            stash4(p, strow, row_valid, hot_base + t0 + 4 * grp, sh, nvalid, st_vec_h, srs, sbase);
+            stash4(p, strow, row_valid, hot_base + t0 + 4 * grp, sh, nvalid, st_buf_ok, srs, sbase);
             hot_p = softmax16(stt, sh, sl2);
         } else {
             // ---- hot V tile: lane = (chunk col, tokens 4 grp .. +3)
@@ -1185,8 +1182,7 @@ bool decode_fast_legacy_shape(int D, int bits, int group_size, int meta_dtype) {
 }
 
 bool decode_fast_meta_aligned(int64_t rows_per_head, int Gv, int64_t heads) {
-    const int ng = kD / Gv;
-    return ng == 4 || heads <= 1 || (rows_per_head * ng * 2) % 16 == 0;
+    return kD / Gv > 1 || heads <= 1 || rows_per_head % 2 == 0;
 }
 
 bool decode_fast_eligible(const DecodeParams &p, int wk) {
