@@ -220,7 +220,7 @@ int check_decode(const akv_decode_args *a) {
 }
 
 struct PrefillPlan {
-    int R, n_row_tiles, nsplit, nchunk, prows;
+    int R, n_row_tiles, nsplit, nchunk;
     int64_t tiles_per_split, part_bytes;
 };
 
@@ -291,9 +291,8 @@ void make_prefill_plan(const akv_prefill_args *a, PrefillPlan *pl) {
     pl->tiles_per_split = (nt + ns - 1) / ns;
     pl->nsplit = (int)((nt + pl->tiles_per_split - 1) / pl->tiles_per_split);
     pl->nchunk = (pl->R + 15) / 16;
-    pl->prows = pl->R < 16 ? pl->R : 16;
-    pl->part_bytes = pl->nsplit > 1
-        ? align256((int64_t)a->B * a->Hkv * pl->nchunk * pl->nsplit * pl->prows * (a->D + 4) * 4) : 0;
+    pl->part_bytes =
+        pl->nsplit > 1 ? align256((int64_t)a->B * a->Hkv * pl->nchunk * pl->nsplit * akv::kPrefillPart * 4) : 0;
 }
 
 }  // namespace
@@ -745,7 +744,7 @@ int akv_prefill_attn(const akv_prefill_args *a, void *stream) {
     p.nsplit = pl.nsplit;
     p.tiles_per_split = pl.tiles_per_split;
     p.part = (float *)a->workspace;
-    p.nchunk = pl.nchunk; p.prows = pl.prows;
+    p.nchunk = pl.nchunk;
     p.kcur = a->k_chunk; p.vcur = a->v_chunk;
     p.n_cur = a->k_chunk ? a->M : 0;
     hipError_t e = akv::prefill_launch(p, (hipStream_t)stream);

@@ -47,7 +47,6 @@ struct DecodeParams {
     float *stash;                 // [B][Hq][M][N] raw logits q.k (or null); x * scale_log2 is the log2 domain
     float *rowstats;              // [B*Hq*M][2] (M, 1 / L): the reciprocal once per row
     _Float16 *out;                // [B][Hq][M][D]
-    int out_bf16;                 // reduce only: write bf16 (chunked prefill with bf16 queries)
     float *attn_out;              // normalised weights (or null)
     float *scores;                // importance EMA (or null)
     int64_t n_scores;

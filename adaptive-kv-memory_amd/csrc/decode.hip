@@ -776,14 +776,8 @@ __device__ __forceinline__ void merge_split_row(const DecodeParams &p, int bhc, 
         const int r = row0 + rr;
         const int h = kvh * p.g + r / p.M, m = r % p.M;
         const int64_t row = (int64_t)(b * p.Hq + h) * p.M + m;
-        if (p.out_bf16) {
-            const u2 ov = {(uint32_t)f32_to_bf16_rne(o[0] / L) | ((uint32_t)f32_to_bf16_rne(o[1] / L) << 16),
-                           (uint32_t)f32_to_bf16_rne(o[2] / L) | ((uint32_t)f32_to_bf16_rne(o[3] / L) << 16)};
-            *(u2 *)(p.out + row * D + 4 * tid) = ov;
-        } else {
-            const h4 ov = {(_Float16)(o[0] / L), (_Float16)(o[1] / L), (_Float16)(o[2] / L), (_Float16)(o[3] / L)};
-            *(h4 *)(p.out + row * D + 4 * tid) = ov;
-        }
+        const h4 ov = {(_Float16)(o[0] / L), (_Float16)(o[1] / L), (_Float16)(o[2] / L), (_Float16)(o[3] / L)};
+        *(h4 *)(p.out + row * D + 4 * tid) = ov;
         if (tid == 0 && p.rowstats) {
             p.rowstats[2 * row] = M;
             p.rowstats[2 * row + 1] = 1.0f / (L * (1.0f / 128.0f));  // 1 / L, the 2^7 probability scale undone
@@ -791,7 +785,7 @@ __device__ __forceinline__ void merge_split_row(const DecodeParams &p, int bhc, 
     }
 }
 
-// Few splits (<= 8, chunked prefill): thread = (row of the chunk, channel quad)
+// Few splits (<= 8): thread = (row of the chunk, channel quad)
 // with all its split loads in flight; 256 / (D/4) rows per workgroup.
 template <int D>
 __global__ __launch_bounds__(256) void reduce_few_kernel(const DecodeParams p) {
@@ -829,14 +823,8 @@ __global__ __launch_bounds__(256) void reduce_few_kernel(const DecodeParams p) {
     const int r = row0 + rr;
     const int h = kvh * p.g + r / p.M, m = r % p.M;
     const int64_t row = (int64_t)(b * p.Hq + h) * p.M + m;
-    if (p.out_bf16) {
-        const u2 ov = {(uint32_t)f32_to_bf16_rne(o[0] / L) | ((uint32_t)f32_to_bf16_rne(o[1] / L) << 16),
-                       (uint32_t)f32_to_bf16_rne(o[2] / L) | ((uint32_t)f32_to_bf16_rne(o[3] / L) << 16)};
-        *(u2 *)(p.out + row * D + 4 * q) = ov;
-    } else {
-        const h4 ov = {(_Float16)(o[0] / L), (_Float16)(o[1] / L), (_Float16)(o[2] / L), (_Float16)(o[3] / L)};
-        *(h4 *)(p.out + row * D + 4 * q) = ov;
-    }
+    const h4 ov = {(_Float16)(o[0] / L), (_Float16)(o[1] / L), (_Float16)(o[2] / L), (_Float16)(o[3] / L)};
+    *(h4 *)(p.out + row * D + 4 * q) = ov;
     if (q == 0 && p.rowstats) {
         p.rowstats[2 * row] = M;
         p.rowstats[2 * row + 1] = 1.0f / (L * (1.0f / 128.0f));  // 1 / L, the 2^7 probability scale undone

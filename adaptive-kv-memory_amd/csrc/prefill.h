@@ -19,15 +19,16 @@ struct PrefillParams {
     int T, Gv, bits_k, bits_v;
     float scale_log2;               // sm_scale * log2(e)
     int n_row_tiles;                // ceil(R / rows per workgroup)
-    int nsplit;                     // token splits (partials merged by decode_reduce_kernel)
+    int nsplit;                     // token splits (partials merged by prefill_merge_kernel)
     int64_t tiles_per_split;        // 32-token tiles per split (hot tiles first, then warm)
-    float *part;                    // partials, decode layout (16-row chunks), when nsplit > 1
-    int nchunk, prows;              // 16-row chunks of R and rows per partial (decode layout)
+    float *part;                    // partials [bh][chunk][split][kPrefillPart] when nsplit > 1
+    int nchunk;                     // 16-row chunks of R
     const void *kcur, *vcur;        // the chunk's own K / V [B][Hkv][M][128] in q's dtype (or null):
     int n_cur;                      // attended causally after the cache; n_cur = M (0 without them)
 };
 
 constexpr int kPrefillRows = 256;   // query rows per workgroup
+constexpr int kPrefillPart = 16 * 128 + 32;  // floats of one split's partial of a 16-row chunk: acc, (max, sum)
 
 // Launch the split kernel and, when nsplit > 1, the merge.
 hipError_t prefill_launch(const PrefillParams &p, hipStream_t s);
