@@ -164,7 +164,9 @@ void prefill_kernel(const PrefillParams p) {
     // Registers of the next tile, one set for every role:
     //   hot K: R[0..3] = 64 B of the token;  hot V: R[i] = 16 B of token i (i < 2);
     //   warm K: R[0] = code bytes, R[1] = s_lo, s_hi, z_lo, z_hi of the prep pair;
-    //   warm V: R[0] = codes of tokens 0, 1 and their scales, R[1][0..1] = their zeros.
+    //   warm V: R[0] = codes of tokens 0, 1 and their scales, R[1][2..3] = their zeros;
+    //   3 bits: the two dwords around a token's codes lie together, R[i][0..1] of token i
+    //   (the registers one load fills: a move would wait for it ahead of the MFMAs).
     u4 hraw[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) hraw[i] = (u4){0u, 0u, 0u, 0u};
@@ -205,17 +207,18 @@ void prefill_kernel(const PrefillParams p) {
                 for (int i = 0; i < 2; ++i) {
                     const uint32_t tk = tok0 + 16 * vh + 4 * grp + 2 * vp + i;
                     if (BV == 3) {
-                        const uint32_t off = tk * VR + 3 * col;
-                        const uint32_t d0 = bld32(rvc, off & ~3u);
-                        const uint32_t d1 = (off & 3u) >= 2u ? bld32(rvc, (off & ~3u) + 4u) : 0u;
-                        hraw[0][i] = __builtin_amdgcn_alignbyte(d1, d0, off & 3u);
+                        // both dwords the 3 bytes may lie in, put together when staged: a use
+                        // here would wait for the loads ahead of the tile's MFMAs
+                        const u2 x = bld64(rvc, (tk * VR + 3 * col) & ~3u);
+                        hraw[i][0] = x[0];
+                        hraw[i][1] = x[1];
                     } else if (BV == 4) {
                         hraw[0][i] = bld32(rvc, tk * VR + 4 * col);
                     } else {
                         hraw[0][i] = bld16(rvc, tk * VR + 2 * col);
                     }
                     hraw[0][2 + i] = bld16(rvs, (tk * NG + gv) * 2u);
-                    hraw[1][i] = bld16(rvz, (tk * NG + gv) * 2u);
+                    hraw[1][2 + i] = bld16(rvz, (tk * NG + gv) * 2u);
                 }
             }
         }
@@ -313,11 +316,17 @@ void prefill_kernel(const PrefillParams p) {
             __builtin_amdgcn_wave_barrier();  // kmeta reads done before the next tile's writes
         } else {
             const h2 vs = as_h2(hraw[0][2] | (hraw[0][3] << 16));
-            const h2 vz = as_h2(hraw[1][0] | (hraw[1][1] << 16));
+            const h2 vz = as_h2(hraw[1][2] | (hraw[1][3] << 16));
             const _Float16 n0 = (_Float16)(-1024.0f);
             const bool vfast = !__builtin_amdgcn_ballot_w64(!finite2(as_u32(vs * (h2){n0, n0})));
             uint32_t win[VSlot<BV>::NW];
-            v_windows<BV>(hraw[0][0], hraw[0][1], win);
+            if constexpr (BV == 3) {  // rows are whole dwords: the byte offset is the chunk's
+                const uint32_t sh = (3u * (uint32_t)col) & 3u;
+                v_windows<BV>(__builtin_amdgcn_alignbyte(hraw[0][1], hraw[0][0], sh),
+                              __builtin_amdgcn_alignbyte(hraw[1][1], hraw[1][0], sh), win);
+            } else {
+                v_windows<BV>(hraw[0][0], hraw[0][1], win);
+            }
             uint32_t vpair[8];
             if (vfast) {
                 h2 vn[v_noffs<BV>()];
