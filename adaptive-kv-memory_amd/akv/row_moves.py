@@ -7,6 +7,7 @@ tensors laid out (B, H, T, C), or (T,), and runs them as one launch on the curre
 from __future__ import annotations
 
 import ctypes
+import struct
 from typing import Optional
 
 import torch
@@ -31,40 +32,50 @@ def movable(out_dtype: torch.dtype, *tensors: torch.Tensor) -> bool:
     return out_dtype in _FLOATS and forward_ad._current_level < 0
 
 
+# the fields of an akv_rows_job, packed in one call (a ctypes structure costs three times that)
+_JOB = struct.Struct("@12q7if")
+assert _JOB.size == ctypes.sizeof(nat.RowsJob)
+
+
 class RowMoves:
     def __init__(self):
         self._jobs = []
         self._hold = []
-
-    @staticmethod
-    def _layout(t: torch.Tensor):
-        e = t.element_size()
-        if t.dim() == 1:
-            return 1, 1, 1, 0, 0, t.stride(0) * e
-        if t.shape[3] > 1 and t.stride(3) != 1:
-            raise ValueError("row moves take rows of consecutive elements")
-        return t.shape[0], t.shape[1], t.shape[3], t.stride(0) * e, t.stride(1) * e, t.stride(2) * e
 
     def copy(self, dst: torch.Tensor, src: torch.Tensor, n: int, rows: int = SAME, at: int = 0, value: float = 1.0):
         """``n`` rows of ``src`` to the rows of ``dst`` from ``at`` on (SCATTER: to the listed
         rows); float32 destinations take 16-bit floats widened, and float32 times ``value``."""
         if n == 0:
             return
-        B, H, C, sb, sh, st = self._layout(src)
-        b, h, c, db, dh, dt = self._layout(dst)
-        if (b, h, c) != (B, H, C):
-            raise ValueError(f"row moves between {tuple(src.shape)} and {tuple(dst.shape)}")
-        token = 0 if src.dim() == 1 else 2
-        rows_in, rows_out = src.shape[token], dst.shape[token]
-        if n > (rows_in if rows != SCATTER else rows_out) or at + (n if rows != SCATTER else 0) > rows_out:
+        ss, ds, st, dt = src.shape, dst.shape, src.stride(), dst.stride()
+        se, de = src.element_size(), dst.element_size()
+        if len(ss) == 1:
+            B = H = C = 1
+            rows_in, rows_out = ss[0], ds[0]
+            sb = sh = db = dh = 0
+            s_row, d_row = st[0] * se, dt[0] * de
+            fits = len(ds) == 1
+        else:
+            B, H, rows_in, C = ss
+            rows_out = ds[2]
+            sb, sh, s_row = st[0] * se, st[1] * se, st[2] * se
+            db, dh, d_row = dt[0] * de, dt[1] * de, dt[2] * de
+            fits = (B, H, C) == (ds[0], ds[1], ds[3]) and (C == 1 or (st[3] == 1 and dt[3] == 1))
+        if not fits:
+            raise ValueError(f"row moves between {tuple(ss)} {st} and {tuple(ds)} {dt}")
+        if rows == SCATTER:
+            past = n > rows_out or n > rows_in
+        else:
+            past = n > rows_in or at + n > rows_out
+        if past:
             raise ValueError("row moves past a tensor's rows")
         widen = src.dtype != dst.dtype or value != 1.0
         if widen and (dst.dtype != torch.float32 or src.dtype not in _FLOATS):
             raise TypeError(f"row moves do not convert {src.dtype} to {dst.dtype}")
         self._hold.append((src, dst))
-        self._jobs.append(nat.RowsJob(
-            src.data_ptr(), dst.data_ptr() + at * dt, sb, sh, st, db, dh, dt, n,
-            rows_out if rows == SCATTER else rows_in, 0, 0, B, H, C, src.element_size(),
+        self._jobs.append(_JOB.pack(
+            src.data_ptr(), dst.data_ptr() + at * d_row, sb, sh, s_row, db, dh, d_row, n,
+            rows_out if rows == SCATTER else rows_in, 0, 0, B, H, C, se,
             _WIDEN if widen else _COPY, rows, nat.dtype_code(src.dtype) if widen else 0, value))
 
     def fill(self, dst: torch.Tensor, n: int, value: float, at: int = 0):
@@ -81,9 +92,10 @@ class RowMoves:
         if dst.dim() != 1 or dst.dtype != dtype or at + n > dst.shape[0]:
             raise ValueError("fill and count take vectors that hold the entries")
         e = dst.element_size()
-        self._hold.append(dst)
-        self._jobs.append(nat.RowsJob(None, dst.data_ptr() + at * e * dst.stride(0), 0, 0, 0, 0, 0, e * dst.stride(0),
-                                      n, n, start, step, 1, 1, 1, e, kind, SAME, 0, value))
+        row = e * dst.stride(0)
+        self._hold.append((dst, dst))
+        self._jobs.append(_JOB.pack(0, dst.data_ptr() + at * row, 0, 0, 0, 0, 0, row, n, n, start, step, 1, 1, 1, e,
+                                    kind, SAME, 0, value))
 
     def run(self, idx: Optional[torch.Tensor] = None, n_idx: int = 0):
         """Launch the collected jobs; ``idx``: the first ``n_idx`` entries of an int64 list."""
@@ -91,9 +103,7 @@ class RowMoves:
             return
         if idx is not None and (idx.dtype != torch.int64 or (n_idx > 1 and idx.stride(-1) != 1) or n_idx > idx.numel()):
             raise ValueError("row moves take an int64 list of consecutive entries")
-        jobs = (nat.RowsJob * len(self._jobs))(*self._jobs)
-        hold = self._hold[0]
-        like = hold if isinstance(hold, torch.Tensor) else hold[1]
+        jobs = (nat.RowsJob * len(self._jobs)).from_buffer_copy(b"".join(self._jobs))
         nat.check(nat.load().akv_rows_move(jobs, len(self._jobs), idx.data_ptr() if n_idx else None, n_idx,
-                                           nat.stream_of(like)), "row moves")
+                                           nat.stream_of(self._hold[0][1])), "row moves")
         self._jobs, self._hold = [], []

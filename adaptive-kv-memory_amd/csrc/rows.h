@@ -12,6 +12,7 @@ constexpr int kRowsMaxJobs = 12;
 struct RowsParams {
     akv_rows_job job[kRowsMaxJobs];
     int unit[kRowsMaxJobs];  // bytes (COPY) or elements of 16 source-side vectors (WIDEN) a thread moves at once
+    int tile[kRowsMaxJobs];  // rows of a workgroup
     const int64_t *idx;
     int64_t n_idx;
 };
