@@ -36,6 +36,7 @@ constexpr int kTileWaves = 4;
 constexpr int kEncTiles = 8;        // tiles per workgroup when a long block's statistics are precomputed
 constexpr int kLongT = 512;         // blocks longer than this may use the workspace
 constexpr int kStatTokens = 512;    // tokens per statistics chunk (at least)
+constexpr int kStatWaves = 16;      // a wave a tile of a chunk: every load of the chunk in flight at once
 constexpr int kMaxChunks = 64;
 
 // K statistics sources of qtile_kernel
@@ -510,10 +511,12 @@ __global__ __launch_bounds__(64 * kTileWaves) void qtile_kernel(const QuantParam
 }
 
 // min / max partials of chunk c of a long block: grid (nblk * nchunk, H, B).  (An outlier
-// channel's partials are not used: the encoder sets its statistics to zero.)
+// channel's partials are not used: the encoder sets its statistics to zero.)  Bound by the
+// latency of the index and row loads, so a wave takes one tile of the chunk, not four in turn:
+// 16,255 tokens x 8 heads (33 MB) 17.7 -> 9.8 us.
 template <int IN, int D>
-__global__ __launch_bounds__(64 * kTileWaves) void kstat_kernel(const QuantParams p) {
-    __shared__ float red[kTileWaves][2][D];
+__global__ __launch_bounds__(64 * kStatWaves) void kstat_kernel(const QuantParams p) {
+    __shared__ float red[kStatWaves][2][D];
     using TL = Tile<D>;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int cg = lane % TL::CG, tg = lane / TL::CG;
@@ -528,7 +531,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void kstat_kernel(const QuantParam
         mn[e] = INFINITY;
         mx[e] = -INFINITY;
     }
-    for (int64_t t = c0 + 32 * wave; t < c1; t += 32 * kTileWaves) {
+    for (int64_t t = c0 + 32 * wave; t < c1; t += 32 * kStatWaves) {
         uint32_t w[TL::TPL][kInWords<IN>];
         load_tile<IN, D>(p, p.k, b, bh, t, (int)min((int64_t)32, c1 - t), cg, tg, w);
         lane_minmax<IN, D>(w, mn, mx);
@@ -542,9 +545,9 @@ __global__ __launch_bounds__(64 * kTileWaves) void kstat_kernel(const QuantParam
         }
     __syncthreads();
     float *part = p.ws + ((bh * p.nblk + blk) * p.nchunk + c) * 2 * D;
-    for (int i = threadIdx.x; i < 2 * D; i += 64 * kTileWaves) {
+    for (int i = threadIdx.x; i < 2 * D; i += 64 * kStatWaves) {
         float v = red[0][i / D][i % D];
-        for (int o = 1; o < kTileWaves; ++o)
+        for (int o = 1; o < kStatWaves; ++o)
             v = i < D ? fminf(v, red[o][i / D][i % D]) : fmaxf(v, red[o][i / D][i % D]);
         part[i] = v;
     }
@@ -812,7 +815,7 @@ static hipError_t launch_tiles(const QuantParams &p, hipStream_t s) {
             ksrc = kKPartials;
             gx = p.nblk * ((tpb + kEncTiles - 1) / kEncTiles);
             hipLaunchKernelGGL((kstat_kernel<IN, D>), dim3((unsigned)(p.nblk * p.nchunk), p.H, p.B),
-                               dim3(64 * kTileWaves), 0, s, p);
+                               dim3(64 * kStatWaves), 0, s, p);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
         } else {
