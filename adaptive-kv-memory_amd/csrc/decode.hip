@@ -905,9 +905,12 @@ __global__ __launch_bounds__(256) void weights_stats_kernel(const DecodeParams p
     const int tid = threadIdx.x, q = tid % NQ, rl = tid / NQ;
     const int64_t rows = (int64_t)p.B * p.Hq * p.M, N = p.N;
     const float sl2 = p.scale_log2;
-    const int64_t n0 = (int64_t)blockIdx.x * TPW + 4 * q;
+    // Workgroups go to the 8 XCDs in turn: each XCD takes a run of neighbouring token tiles, so
+    // that the cache lines two tiles share (rows of odd length) meet in one L2.
+    const int64_t tile = (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    const int64_t n0 = tile * TPW + 4 * q;
     // the old score is loaded with the first batch of logits, not after the reduction
-    const int64_t ns = (int64_t)blockIdx.x * TPW + tid;
+    const int64_t ns = tile * TPW + tid;
     const float sc_old = (p.scores && tid < TPW && ns < p.n_scores) ? p.scores[ns] : 0.f;
     float imp[4] = {0.f, 0.f, 0.f, 0.f};
     for (int64_t r0 = rl; r0 < rows; r0 += NRL * RB) {
@@ -1170,7 +1173,8 @@ hipError_t decode_launch(const DecodeParams &p, int kb, int vb, int wk, const in
     if (p.stash && p.split_ctr) {
         // the split kernel merged its splits and wrote the row statistics
         const int64_t nmax = p.N > p.n_scores ? p.N : p.n_scores;
-        const dim3 g((unsigned)((nmax + 4 * kWsQuads - 1) / (4 * kWsQuads)));
+        // a multiple of 8 workgroups, so that they divide over the XCDs
+        const dim3 g((unsigned)(((nmax + 4 * kWsQuads - 1) / (4 * kWsQuads) + 7) / 8 * 8));
         constexpr int NRL = 256 / kWsQuads;
         const int64_t per = (rows + NRL - 1) / NRL;  // rows per thread
 #define AKV_WS(RB) hipLaunchKernelGGL(weights_stats_kernel<RB>, g, dim3(256), 0, s, p)
