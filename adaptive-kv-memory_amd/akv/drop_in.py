@@ -134,14 +134,14 @@ class _EventTier:
     its event and ``pos`` to its chronological position.  Capacities double as
     tokens arrive."""
 
-    def __init__(self, B, H, D, bits_k, bits_v, n_out, dev):
+    def __init__(self, B, H, D, bits_k, bits_v, n_out, dev, rows: int = 0):
+        """``rows``: the first event's tokens, for which the first capacity makes room."""
         self.B, self.H, self.D, self.bits_k, self.bits_v, self.n_out = B, H, D, bits_k, bits_v, n_out
         self.dev = dev
         self.n = 0
         self.n_events = 0
-        self.cap = self.ecap = 0
-        self.t = {}
-        self._grow(256, 16)
+        self.cap, self.ecap = 256 if rows <= 256 else 2 * rows, 16
+        self.t = self._alloc(self.cap, self.ecap)
 
     def _alloc(self, cap, ecap):
         B, H, D, n_out, dev = self.B, self.H, self.D, self.n_out, self.dev
@@ -179,14 +179,13 @@ class _EventTier:
         mv.run()
         self.t, self.cap, self.ecap = t, cap, ecap
 
-    def append(self, w: WarmTier, positions: torch.Tensor, idx: torch.Tensor):
+    def append(self, w: WarmTier, positions: torch.Tensor, mv: RowMoves):
         """One demotion event: ``w`` holds its n tokens as a single K block; their positions
-        are ``positions[idx]``."""
+        are those of ``positions`` at the list ``mv`` is run with."""
         n = w.n_warm
         if self.n + n > self.cap or self.n_events + 1 > self.ecap:
             self._grow(max(self.cap, 2 * (self.n + n)), max(self.ecap, 2 * (self.n_events + 1)))
         t, a, e = self.t, self.n, self.n_events
-        mv = RowMoves()
         for name, x in (("kc", w.k_codes), ("vc", w.v_codes), ("vs", w.v_scale), ("vz", w.v_zero)):
             mv.copy(t[name], x, n, at=a)
         mv.copy(t["ks"], w.k_scale, 1, at=e)
@@ -198,7 +197,6 @@ class _EventTier:
             mv.copy(t["voi"].unsqueeze(1), w.v_oidx.unsqueeze(1), 1, at=e)
         mv.count(t["blk"], n, e, 0, at=a)
         mv.copy(t["pos"], positions, n, GATHER, at=a)
-        mv.run(idx, n)
         self.n += n
         self.n_events += 1
 
@@ -250,8 +248,9 @@ class _EventTier:
         a.out_tokens = out_k.shape[2]
         nat.check(nat.load().akv_dequant_unpack(ctypes.byref(a), nat.stream_of(out_k)), "AKVLayer warm view")
 
-    def take(self, idx: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-        """The float16 values of warm tokens ``idx`` (warm-tier order), (B, H, n, D)."""
+    def pull(self, idx: torch.Tensor, vector: Optional[torch.Tensor] = None):
+        """The float16 K, V (B, H, n, D) of the warm tokens of the ascending list ``idx``, which
+        leave the tier, and ``vector`` as ``remove`` gives it."""
         n = idx.numel()
         sub = _EventTier.__new__(_EventTier)
         sub.__dict__.update({k: v for k, v in self.__dict__.items() if k != "t"})
@@ -265,19 +264,21 @@ class _EventTier:
                 mv.copy(sub.t[name], x, n, GATHER)
             else:
                 sub.t[name] = x
-        mv.run(idx, n)
+        kept = self.remove(idx, n, vector, mv)
         sub.n, sub.cap = n, n
         k = torch.empty(self.B, self.H, n, self.D, dtype=torch.float16, device=self.dev)
         v = torch.empty_like(k)
         sub.dequantize_into(k, v, slots=False)
-        return k, v
+        return k, v, kept
 
-    def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None,
+               mv: Optional[RowMoves] = None) -> Optional[torch.Tensor]:
         """Drop the ``n`` warm tokens of the ascending list ``idx`` (their events' K meta rows
         stay); ``vector`` (one float32 per warm token) is returned without theirs.  The kept
-        rows go to fresh tensors: rows shift by up to n, so a move in place would race."""
+        rows go to fresh tensors: rows shift by up to n, so a move in place would race.  ``mv``:
+        jobs on the same list that go with the launch."""
         kept = self.n - n
-        mv = RowMoves()
+        mv = mv or RowMoves()
         for name in self._TOKEN_AXIS:
             if name in self.t:
                 x = self.t[name]
@@ -327,8 +328,10 @@ class _HeadBitsTier:
             v = hv.index_select(1, heads).index_select(2, idx).reshape(B * hs, 1, n, D)
             w = quantize_kv(k, v, bits, bits, block_t=max(n, 1), group_v=D, outlier_fraction=outlier_fraction)
             if tier is None:
-                g[2] = tier = _EventTier(B * hs, 1, D, bits, bits, w.n_out, self.dev)
-            tier.append(w, positions, idx)
+                g[2] = tier = _EventTier(B * hs, 1, D, bits, bits, w.n_out, self.dev, n)
+            mv = RowMoves()
+            tier.append(w, positions, mv)
+            mv.run(idx, n)
             packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
                        + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
         self.n += n
@@ -348,15 +351,18 @@ class _HeadBitsTier:
             if out_v is not None:
                 out_v.index_copy_(1, heads, tv.view(self.B, hs, rows, self.D))
 
-    def take(self, idx: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+    def pull(self, idx: torch.Tensor, vector: Optional[torch.Tensor] = None):
         n = idx.numel()
         k = torch.empty(self.B, self.H, n, self.D, dtype=torch.float16, device=self.dev)
         v = torch.empty_like(k)
-        for bits, heads, tier in self.groups:
-            tk, tv = tier.take(idx)
+        kept = None
+        for i, (bits, heads, tier) in enumerate(self.groups):
+            tk, tv, out = tier.pull(idx, vector if i == 0 else None)
+            kept = out if i == 0 else kept
             k.index_copy_(1, heads, tk.view(self.B, heads.numel(), n, self.D))
             v.index_copy_(1, heads, tv.view(self.B, heads.numel(), n, self.D))
-        return k, v
+        self.n -= n
+        return k, v, kept
 
     def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
         out = None
@@ -551,8 +557,7 @@ class AKVLayer:
         idx = chosen[1:1 + n]
         warm_len = self._warm.n
         positions = self._warm.positions()
-        pk, pv = self._warm.take(idx)
-        kept = self._warm.remove(idx, n, self._proxy_score if use_proxy else None)
+        pk, pv, kept = self._warm.pull(idx, self._proxy_score if use_proxy else None)
         if use_proxy:
             self._proxy_score = kept
         self._warm_bytes_packed = int(self._warm_bytes_packed * (max(0, warm_len - n) / warm_len))
@@ -564,6 +569,7 @@ class AKVLayer:
         dev = hk.device
         B, H, _, D = hk.shape
         idx = select_demote_indices(self._importance, n_demote, hot_len, self.hot_budget, device=dev)
+        mv = RowMoves()  # the event's rows into the packed tier, the kept ones of the hot tier
         if self.per_head_bits and len(self.per_head_bits) == H:
             if self._warm is None:
                 self._warm = _HeadBitsTier(B, H, D, self.per_head_bits, dev)
@@ -572,13 +578,12 @@ class AKVLayer:
             w = quantize_kv(hk, hv, self.warm_key_bits, self.warm_value_bits, block_t=max(n_demote, 1), group_v=D,
                             outlier_fraction=self.outlier_fraction, sel=idx.unsqueeze(0).expand(B, n_demote))
             if self._warm is None:
-                self._warm = _EventTier(B, H, D, self.warm_key_bits, self.warm_value_bits, w.n_out, dev)
-            self._warm.append(w, self._hot_positions, idx)
+                self._warm = _EventTier(B, H, D, self.warm_key_bits, self.warm_value_bits, w.n_out, dev, n_demote)
+            self._warm.append(w, self._hot_positions, mv)
             # measure_packed_bytes per batch element: packed codes + fp16 scale and zero, K and V
             self._warm_bytes_packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
                                         + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
         self._warm_len += n_demote
-        mv = RowMoves()
         if self._proxy_score is not None:  # new warm tokens start with no evidence
             old = self._proxy_score
             self._proxy_score = torch.empty(old.shape[0] + n_demote, dtype=torch.float32, device=dev)

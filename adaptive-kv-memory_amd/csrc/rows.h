@@ -8,7 +8,7 @@
 
 namespace akv {
 
-constexpr int kRowsMaxJobs = 12;
+constexpr int kRowsMaxJobs = 20;
 struct RowsParams {
     akv_rows_job job[kRowsMaxJobs];
     int unit[kRowsMaxJobs];  // bytes (COPY) or elements of 16 source-side vectors (WIDEN) a thread moves at once

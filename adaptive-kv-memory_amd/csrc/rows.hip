@@ -7,11 +7,12 @@
 // -- about kRowsUnits units of up to 16 bytes, four a thread -- and resolves the source or
 // destination rows of a list once before its threads move them: for KEEP a search of the
 // ascending list, first among 1024 samples of it in LDS, so that a list of that size costs one
-// trip to memory and a prompt's 16 thousand five instead of fourteen.  Rows that follow each other on both sides (codes and meta appended to
-// a tier) are one range, cut into units whatever the row's length: 2-byte scale rows would
-// otherwise go 2 bytes a thread.  The four launches of a 16k prompt: 33 -> 26 us.
-// Cache updates, one tensor at a time -> this: a 16k prompt of 8 heads 517 -> 146 us; a 2 x
-// 2-head bfloat16 layer's prompt and 12 tokens with promotions 13.3 -> 4.6 ms.
+// trip to memory and a prompt's 16 thousand five instead of fourteen.  Rows that follow each
+// other on both sides (codes and meta appended to a tier) are one range, cut into units
+// whatever the row's length: 2-byte scale rows would otherwise go 2 bytes a thread.
+// Cache updates, one tensor at a time -> this: a 16k prompt of 8 heads 517 -> 119 us (its
+// launches here 33 us before tiles by units and the sampled search, 26 after); a 2 x 2-head
+// bfloat16 layer's prompt and 12 tokens with promotions 13.3 -> 4.4 ms.
 #include "rows.h"
 
 #include <algorithm>

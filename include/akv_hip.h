@@ -389,7 +389,7 @@ typedef struct akv_rows_job {
     float value;
 } akv_rows_job;
 
-/* Up to 12 jobs in one launch (jobs of one call must not overlap in memory).  idx: int64 list
+/* Up to 20 jobs in one launch (jobs of one call must not overlap in memory).  idx: int64 list
  * of n_idx entries on the device (KEEP: ascending and distinct). */
 int akv_rows_move(const akv_rows_job *jobs, int32_t n_jobs, const int64_t *idx, int64_t n_idx, void *stream);
 
