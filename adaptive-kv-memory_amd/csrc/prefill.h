@@ -28,7 +28,7 @@ struct PrefillParams {
 };
 
 constexpr int kPrefillRows = 256;   // query rows per workgroup
-constexpr int kPrefillPart = 16 * 128 + 32;  // floats of one split's partial of a 16-row chunk: acc, (max, sum)
+constexpr int kPrefillPart = 16 * (128 + 4);  // floats of one split's partial of a 16-row chunk: acc, (max, sum), unused
 
 // Launch the split kernel and, when nsplit > 1, the merge.
 hipError_t prefill_launch(const PrefillParams &p, hipStream_t s);
