@@ -295,13 +295,14 @@ class KIVIFusedCache(KIVICache):
         super().__init__(config or KIVIFusedConfig())
         self._dequant_keys_cache: dict = {}    # layer -> the tier its dequantized rows come from
         self._dequant_values_cache: dict = {}
-        self._views: dict = {}  # layer -> (view, rows before the chunk) between an overflow and its view
+        self._views: dict = {}  # layer -> between an overflow and its view: (view, rows before the chunk) of
+                                # K and V, the residual tokens, the moves still to run
         self._ws: dict = {}  # per-device decode workspace of fused_attention
 
     def _quantize_overflow(self, layer_idx: int):
         """akv/baselines.py:455-496.  One launch quantizes, appends and dequantizes the
-        overflow of both tensors and writes its rows of the view that ``_get_full_kv`` then
-        completes; one more cuts the residuals."""
+        overflow of both tensors and writes its rows of the view; ``_get_full_kv`` runs the
+        one that cuts the residuals and completes the view."""
         cfg = self.config
         res = (self._residual_keys, self._residual_values)
         for bits, r in ((cfg.key_bits, res[0]), (cfg.value_bits, res[1])):
@@ -341,7 +342,7 @@ class KIVIFusedCache(KIVICache):
             nat.check(nat.load().akv_kivi_append(
                 arr, len(g), B, H, D, n, nat.dtype_code(x.dtype), cfg.group_size,
                 nat.DT_F16 if dt == torch.float16 else nat.DT_F32, nat.stream_of(x)), "KIVI append")
-        mv = RowMoves()
+        mv, lefts = RowMoves(), []
         for i in (0, 1):
             r = res[i][layer_idx]
             left = r[:, :, r.shape[2] - cfg.residual_length:]
@@ -350,16 +351,18 @@ class KIVIFusedCache(KIVICache):
                 mv.copy(new, left, left.shape[2])
                 res[i][layer_idx] = new
             else:
-                res[i][layer_idx] = left.contiguous()
-        mv.run()
-        self._views[layer_idx] = views
+                res[i][layer_idx] = left = left.contiguous()
+            lefts.append(left)
+        self._views[layer_idx] = views, lefts, mv
 
     def _get_full_kv(self, layer_idx: int):
         """akv/baselines.py:498-510."""
         rs = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
         if layer_idx not in self._dequant_keys_cache:
             return rs
-        mv, out, views = RowMoves(), [], self._views.pop(layer_idx, [None, None])
+        # an overflow's residual moves go with the view's; the view reads the tokens they read
+        views, rs, mv = self._views.pop(layer_idx, ([None, None], rs, RowMoves()))
+        out = []
         for i, tier in enumerate((self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx])):
             n, r = tier.n, rs[i]
             dt = torch.promote_types(torch.float16, r.dtype)
