@@ -164,9 +164,11 @@ void prefill_kernel(const PrefillParams p) {
     // Registers of the next tile, one set for every role:
     //   hot K: R[0..3] = 64 B of the token;  hot V: R[i] = 16 B of token i (i < 2);
     //   warm K: R[0] = code bytes, R[1] = s_lo, s_hi, z_lo, z_hi of the prep pair;
-    //   warm V: R[0] = codes of tokens 0, 1 and their scales, R[1][2..3] = their zeros;
+    //   warm V: R[0] = codes of tokens 0, 1 and their scales, R[1][0..1] = their zeros;
     //   3 bits: the two dwords around a token's codes lie together, R[i][0..1] of token i
-    //   (the registers one load fills: a move would wait for it ahead of the MFMAs).
+    //   (the registers one load fills: a move would wait for it ahead of the MFMAs), the zeros
+    //   in R[1][2..3].
+    constexpr int kVz = BV == 3 ? 2 : 0;
     u4 hraw[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) hraw[i] = (u4){0u, 0u, 0u, 0u};
@@ -218,7 +220,7 @@ void prefill_kernel(const PrefillParams p) {
                         hraw[0][i] = bld16(rvc, tk * VR + 2 * col);
                     }
                     hraw[0][2 + i] = bld16(rvs, (tk * NG + gv) * 2u);
-                    hraw[1][2 + i] = bld16(rvz, (tk * NG + gv) * 2u);
+                    hraw[1][kVz + i] = bld16(rvz, (tk * NG + gv) * 2u);
                 }
             }
         }
@@ -316,7 +318,7 @@ void prefill_kernel(const PrefillParams p) {
             __builtin_amdgcn_wave_barrier();  // kmeta reads done before the next tile's writes
         } else {
             const h2 vs = as_h2(hraw[0][2] | (hraw[0][3] << 16));
-            const h2 vz = as_h2(hraw[1][2] | (hraw[1][3] << 16));
+            const h2 vz = as_h2(hraw[1][kVz] | (hraw[1][kVz + 1] << 16));
             const _Float16 n0 = (_Float16)(-1024.0f);
             const bool vfast = !__builtin_amdgcn_ballot_w64(!finite2(as_u32(vs * (h2){n0, n0})));
             uint32_t win[VSlot<BV>::NW];
@@ -575,13 +577,21 @@ void prefill_kernel(const PrefillParams p) {
     }
 }
 
-// Merge of the token splits, one workgroup per chunk of 16 rows.  HBM / L2-bound: a split's
+// o / L in the query dtype, 4 channels
+__device__ __forceinline__ u2 out_quad(f4 o, float L, int bf16) {
+    return bf16 ? (u2){(uint32_t)f32_to_bf16_rne(o[0] / L) | ((uint32_t)f32_to_bf16_rne(o[1] / L) << 16),
+                       (uint32_t)f32_to_bf16_rne(o[2] / L) | ((uint32_t)f32_to_bf16_rne(o[3] / L) << 16)}
+                : (u2){as_u32((h2){(_Float16)(o[0] / L), (_Float16)(o[1] / L)}),
+                       as_u32((h2){(_Float16)(o[2] / L), (_Float16)(o[3] / L)})};
+}
+
+// Merge of up to 8 token splits, one workgroup per chunk of 16 rows.  HBM / L2-bound: a split's
 // partial of a chunk is 8 blocks of 64 lanes x 16 bytes in the order the attention waves hold
 // them (block 2 i + half, lane (row col, channel quarter grp): channels 8 (4 grp + i) + 4 half
 // ..+3), then the rows' (max, sum).  So every store of the attention kernel and every load here
 // is 1 KiB of consecutive addresses; stored row by row, each store instruction touched 64
 // cache lines: 2 x 12 x 333 positions over 11,007 tokens (8 splits, 34 MB) 91.8 -> 85.4 us.
-// All loads of 8 splits are in flight at once; the output tile turns through LDS into rows.
+// All splits' loads are in flight at once; the output tile turns through LDS into rows.
 __global__ __launch_bounds__(512) void prefill_merge_kernel(const PrefillParams p) {
     constexpr int KS = 8;
     __shared__ __align__(16) uint16_t tile[16][kPD + 8];
@@ -592,19 +602,59 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(const PrefillParams 
     const float *part = p.part + (bh * p.nchunk + chunk) * p.nsplit * (int64_t)kPrefillPart;
     float M = -INFINITY, L = 0.f;
     f4 o = {0.f, 0.f, 0.f, 0.f};
-    for (int s0 = 0; s0 < p.nsplit; s0 += KS) {
+    f2 ml[KS];
+    f4 x[KS];
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const float *src = part + min(k, p.nsplit - 1) * (int64_t)kPrefillPart;
+        ml[k] = *(const f2 *)(src + 16 * kPD + 2 * col);
+        x[k] = ((const f4 *)src)[blk * 64 + lane];
+        if (k < p.nsplit) M = fmaxf(M, ml[k][0]);
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        if (k >= p.nsplit || ml[k][0] == -INFINITY) continue;
+        const float f = __builtin_amdgcn_exp2f(ml[k][0] - M);
+        o += f * x[k];
+        L += f * ml[k][1];
+    }
+    *(u2 *)&tile[col][8 * (4 * grp + blk / 2) + 4 * (blk & 1)] = out_quad(o, L, p.q_bf16);
+    __syncthreads();
+    const int r = 16 * chunk + (int)threadIdx.x / 16, c = threadIdx.x % 16;
+    if (threadIdx.x >= 256 || r >= p.R) return;
+    const int b = (int)(bh / p.Hkv), hq = (int)(bh % p.Hkv) * p.g + r / p.M;
+    const int64_t orow = ((int64_t)(b * p.Hq + hq) * p.M + r % p.M) * kPD;
+    *(u4 *)((uint16_t *)p.out + orow + 8 * c) = *(const u4 *)&tile[threadIdx.x / 16][8 * c];
+}
+
+// More than 8 splits (short chunks): the same with a workgroup per block of a chunk and its 8
+// waves over the splits, 8 loads of a wave in flight, merged in LDS -- there are few chunks
+// then, and one workgroup walking their splits 8 at a time is a chain of trips to memory
+// (16 heads x 75 positions over 21,194 tokens: 45.7 us a call with a workgroup per row, 42.0 so).
+__global__ __launch_bounds__(512) void prefill_merge_many_kernel(const PrefillParams p) {
+    constexpr int KS = 8, NW = 8;
+    __shared__ f2 mls[NW][16];
+    __shared__ f4 os[NW][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, blk = blockIdx.y;
+    const int col = lane & 15, grp = lane >> 4;
+    const int chunk = blockIdx.x % p.nchunk;
+    const int64_t bh = blockIdx.x / p.nchunk;
+    const float *part = p.part + (bh * p.nchunk + chunk) * p.nsplit * (int64_t)kPrefillPart;
+    float M = -INFINITY, L = 0.f;
+    f4 o = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = wave; s0 < p.nsplit; s0 += NW * KS) {
         f2 ml[KS];
         f4 x[KS];
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            const float *src = part + min(s0 + k, p.nsplit - 1) * (int64_t)kPrefillPart;
+            const float *src = part + min(s0 + NW * k, p.nsplit - 1) * (int64_t)kPrefillPart;
             ml[k] = *(const f2 *)(src + 16 * kPD + 2 * col);
             x[k] = ((const f4 *)src)[blk * 64 + lane];
-            if (s0 + k >= p.nsplit) ml[k][0] = -INFINITY;
         }
         float nm = M;
 #pragma unroll
-        for (int k = 0; k < KS; ++k) nm = fmaxf(nm, ml[k][0]);
+        for (int k = 0; k < KS; ++k)
+            if (s0 + NW * k < p.nsplit) nm = fmaxf(nm, ml[k][0]);
         if (M > -INFINITY) {  // a further batch of splits
             const float f = __builtin_amdgcn_exp2f(M - nm);
             o *= f;
@@ -613,23 +663,31 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(const PrefillParams 
         M = nm;
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            const float f = ml[k][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[k][0] - M);
-            if (s0 + k >= p.nsplit) continue;
+            if (s0 + NW * k >= p.nsplit || ml[k][0] == -INFINITY) continue;
+            const float f = __builtin_amdgcn_exp2f(ml[k][0] - M);
             o += f * x[k];
             L += f * ml[k][1];
         }
     }
-    const u2 w = p.q_bf16 ? (u2){(uint32_t)f32_to_bf16_rne(o[0] / L) | ((uint32_t)f32_to_bf16_rne(o[1] / L) << 16),
-                                 (uint32_t)f32_to_bf16_rne(o[2] / L) | ((uint32_t)f32_to_bf16_rne(o[3] / L) << 16)}
-                          : (u2){as_u32((h2){(_Float16)(o[0] / L), (_Float16)(o[1] / L)}),
-                                 as_u32((h2){(_Float16)(o[2] / L), (_Float16)(o[3] / L)})};
-    *(u2 *)&tile[col][8 * (4 * grp + blk / 2) + 4 * (blk & 1)] = w;
+    os[wave][lane] = o;
+    if (grp == 0) mls[wave][col] = (f2){M, L};
     __syncthreads();
-    const int r = 16 * chunk + (int)threadIdx.x / 16, c = threadIdx.x % 16;
-    if (threadIdx.x >= 256 || r >= p.R) return;
+    const int r = 16 * chunk + col;
+    if (wave != 0 || r >= p.R) return;
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, mls[w][col][0]);
+    o = (f4){0.f, 0.f, 0.f, 0.f};
+    L = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        const f2 ml = mls[w][col];
+        const float f = ml[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[0] - M);
+        o += f * os[w][lane];
+        L += f * ml[1];
+    }
     const int b = (int)(bh / p.Hkv), hq = (int)(bh % p.Hkv) * p.g + r / p.M;
     const int64_t orow = ((int64_t)(b * p.Hq + hq) * p.M + r % p.M) * kPD;
-    *(u4 *)((uint16_t *)p.out + orow + 8 * c) = *(const u4 *)&tile[threadIdx.x / 16][8 * c];
+    *(u2 *)((uint16_t *)p.out + orow + 8 * (4 * grp + blk / 2) + 4 * (blk & 1)) = out_quad(o, L, p.q_bf16);
 }
 
 int prefill_lds_bytes() { return kPLds; }
@@ -660,7 +718,9 @@ hipError_t prefill_launch(const PrefillParams &p, hipStream_t s) {
     AKV_PKV(4, 4)
 #undef AKV_PKV
     if (e != hipSuccess || p.nsplit == 1) return e;
-    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)(p.B * p.Hkv * p.nchunk)), dim3(512), 0, s, p);
+    const unsigned chunks = (unsigned)(p.B * p.Hkv * p.nchunk);
+    if (p.nsplit <= 8) hipLaunchKernelGGL(prefill_merge_kernel, dim3(chunks), dim3(512), 0, s, p);
+    else hipLaunchKernelGGL(prefill_merge_many_kernel, dim3(chunks, 8), dim3(512), 0, s, p);
     return hipGetLastError();
 }
 
