@@ -302,13 +302,17 @@ def quant_pack(a: QuantArgs, like: torch.Tensor, what: str) -> None:
 
 
 def importance_update(a: ImportanceArgs, like: torch.Tensor, what: str) -> None:
-    """``akv_importance_update_ws`` on the current stream of ``like``'s device, with scratch for
-    the calls that ask for some (many query rows)."""
+    """The importance update on the current stream of ``like``'s device, with scratch for the
+    calls that ask for some (many query rows; a few unpooled ones never do, and a decode
+    step's call is not held up by asking)."""
     lib = load()
     ref = ctypes.byref(a)
-    nbytes = max(0, lib.akv_importance_workspace_bytes(ref))  # < 0: the call itself reports it
-    ws = workspace(nbytes, like.device) if nbytes > 0 else None
-    check(lib.akv_importance_update_ws(ref, ptr(ws), nbytes, stream_of(like)), what)
+    nbytes = lib.akv_importance_workspace_bytes(ref) if a.M >= 16 or a.pool_kernel > 1 else 0
+    if nbytes > 0:
+        ws = workspace(nbytes, like.device)
+        check(lib.akv_importance_update_ws(ref, ptr(ws), nbytes, stream_of(like)), what)
+    else:
+        check(lib.akv_importance_update(ref, stream_of(like)), what)
 
 
 class DecodeWorkspace:

@@ -381,7 +381,7 @@ struct ImpVec {
         }
     }
 };
-constexpr int kImpWaves = 4, kImpMinQueries = 8;
+constexpr int kImpWaves = 4, kImpMinQueries = 20, kImpMinPooledRows = 40;
 template <int DT>
 __global__ __launch_bounds__(64 * kImpWaves) void importance_part_kernel(const ImportanceParams p, float *part,
                                                                          int64_t q_per) {
@@ -859,13 +859,14 @@ hipError_t stream_read_launch(const void *p, int64_t bytes, uint32_t *sink, hipS
     return hipGetLastError();
 }
 // Query blocks of importance_part_kernel (0: the one-launch kernels); about four workgroups
-// per compute unit, each wave at least one query.  The second launch has to pay: without
-// pooling one launch takes 4.1-5.6 us at 4 query rows and 6.5-8.7 us at 8 (700 to 8,191 keys,
-// 8 to 32 heads) against 5.8-7.1 us split at any count up to 16; with pooling 4.1-10.8 us at
-// one row and 6.3-20.7 us at two against 5.8-6.9 us.
+// per compute unit, each wave at least one query.  On the device the split (5.8-7.1 us at any
+// count up to 16) passes the one launch at 8 query rows without pooling (6.5-8.7 us; 11-15 at
+// 16, ~0.55 a row) and at ~12 (batch, head, query) rows with it (~0.3 us a row: 10.8 us at 32,
+// 20.5 at 64); but an eager call with a workspace and a second launch costs 12.2 us of host time
+// against 10.6, so the lines lie where the one launch takes longer than that.
 static int64_t importance_q_blocks(const ImportanceParams &p, int64_t *q_per) {
     const int64_t q = p.M - p.m0, kv = p.attn_dt == AKV_DT_F32 ? 4 : 8;
-    if (q < (p.pool > 1 ? 2 : kImpMinQueries) || p.N < kv || p.n_scores == 0) return 0;
+    if ((p.pool > 1 ? p.B * p.H * q < kImpMinPooledRows : q < kImpMinQueries) || p.N < kv || p.n_scores == 0) return 0;
     const int64_t tiles = (p.N + 64 * kv - 1) / (64 * kv);
     const int64_t want = max((int64_t)1, min((q + kImpWaves - 1) / kImpWaves, 1024 / tiles));
     *q_per = ((q + want - 1) / want + kImpWaves - 1) / kImpWaves * kImpWaves;

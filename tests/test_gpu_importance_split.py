@@ -1,4 +1,5 @@
-"""The importance update with its query sum split over workgroups (8 query rows and more):
+"""The importance update with its query sum split over workgroups (20 query rows and more, or
+40 (batch, head, query) rows with pooling):
 every dtype, row lengths at and around the 16-byte chunk and the 64-lane tile, partial query
 blocks, head counts off 8, pooling and windows, scores shorter and longer than the rows."""
 import numpy as np
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dt", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("B,H,M,N,W,ks,ns", [
-    (1, 1, 8, 8, 0, 1, 8), (1, 3, 9, 9, 0, 1, 9), (2, 4, 8, 255, 0, 1, 255), (1, 8, 17, 511, 0, 1, 511),
+    (1, 1, 20, 8, 0, 1, 8), (1, 3, 21, 9, 0, 1, 9), (2, 4, 24, 255, 0, 1, 255), (1, 8, 29, 511, 0, 1, 511),
+    (1, 8, 5, 300, 0, 7, 300), (2, 12, 2, 700, 0, 7, 700),
     (1, 9, 33, 513, 0, 1, 600), (2, 6, 40, 1000, 32, 7, 1000), (1, 16, 64, 1025, 9, 64, 1025), (1, 2, 300, 77, 0, 5, 40),
     (2, 1, 257, 2047, 0, 1, 2047),
 ])
