@@ -495,7 +495,7 @@ class AKVLayer:
         if front:
             mv.copy(pos, promoted[2], front, GATHER)
         if old:
-            mv.copy(pos, self._hot_positions, old, at=front)
+            mv.copy(pos, self._hot_positions.to(dev), old, at=front)
         mv.count(pos, new, self._total_len, at=front + old)
         imp = None
         if not self.protect:

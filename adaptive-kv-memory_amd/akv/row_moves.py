@@ -47,6 +47,8 @@ class RowMoves:
         rows); float32 destinations take 16-bit floats widened, and float32 times ``value``."""
         if n == 0:
             return
+        if not (src.is_cuda and dst.is_cuda):
+            nat.require_device(src, dst)
         ss, ds, st, dt = src.shape, dst.shape, src.stride(), dst.stride()
         se, de = src.element_size(), dst.element_size()
         if len(ss) == 1:
@@ -101,8 +103,8 @@ class RowMoves:
         """Launch the collected jobs; ``idx``: the first ``n_idx`` entries of an int64 list."""
         if not self._jobs:
             return
-        if idx is not None and (idx.dtype != torch.int64 or (n_idx > 1 and idx.stride(-1) != 1) or n_idx > idx.numel()):
-            raise ValueError("row moves take an int64 list of consecutive entries")
+        if idx is not None and (not idx.is_cuda or idx.dtype != torch.int64 or (n_idx > 1 and idx.stride(-1) != 1) or n_idx > idx.numel()):
+            raise ValueError("row moves take an int64 list of consecutive entries on the device")
         jobs = (nat.RowsJob * len(self._jobs)).from_buffer_copy(b"".join(self._jobs))
         nat.check(nat.load().akv_rows_move(jobs, len(self._jobs), idx.data_ptr() if n_idx else None, n_idx,
                                            nat.stream_of(self._hold[0][1])), "row moves")
