@@ -384,12 +384,12 @@ void decode_fast_kernel(const DecodeParams p) {
             LEG ? (p.warm_heads == 1 ? 0 : p.warm_heads == p.Hkv ? (int64_t)kvh : bh) * p.w_stride : bh * p.n_warm;
         R.kc = rsrc4((const unsigned char *)p.kc + wrow * L::KR, nwu * L::KR);
         R.vc = rsrc4((const unsigned char *)p.vc + wrow * L::VR, nwu * L::VR);
-        // Per-token meta rows: the range check works on dwords, and with 4 or 2 groups every
-        // dword ends on a token.  With 1 group the last token of an odd tier is half a dword, so
-        // the range is rounded up to one (the base is dword-aligned, see
-        // decode_fast_meta_aligned, so it stays in the page of its first byte) and the rows past
-        // the tier are cleared in LDS before use.
-        const uint32_t mrec = (nwu * NG * 2 + 3u) & ~3u;
+        // Per-token meta: with 4 groups a unit's rows are loaded a dword per lane, and every
+        // dword ends on a token; with 1 or 2 groups they come in 16-byte loads, and a load that
+        // crosses the end of the range may be dropped whole by the range check, so the range is
+        // rounded up to 16 bytes (the base is 16-byte aligned, so the last load lies in the
+        // page of its first byte) and the rows past the tier are cleared in LDS before use.
+        const uint32_t mrec = NG == 4 ? nwu * 8u : (nwu * NG * 2 + 15u) & ~15u;
         if (LEG) {
             R.ks = rsrc4((const _Float16 *)p.ks + wrow * NG, mrec);
             R.kz = rsrc4((const _Float16 *)p.kz + wrow * NG, mrec);
@@ -563,8 +563,8 @@ void decode_fast_kernel(const DecodeParams p) {
 #else
         wait_head();
 #endif
-        if (NG == 1 && id * kUnit + kUnit > nw) {
-            // the tail unit: the meta row past the tier's last token may hold bytes from outside it
+        if (NG < 4 && id * kUnit + kUnit > nw) {
+            // the tail unit: meta rows past the tier's last token may hold bytes from outside it
             const int t = lane & 31;
             if (lane < 32 && t >= nw - id * kUnit) {
 #pragma unroll
@@ -1181,8 +1181,14 @@ bool decode_fast_legacy_shape(int D, int bits, int group_size, int meta_dtype) {
            meta_dtype == AKV_DT_F16;
 }
 
+// With 1 or 2 groups the meta rows of every head start on 16 bytes.  The others stay on
+// decode_split_kernel, whose results repeat bit for bit and round V as the reference does: 3 x 28
+// heads x 3 positions over 9,334 tokens with weights and importance (2 groups, 9,001 warm tokens)
+// take 82 us there against 28 here, but here the waves draw their units from a counter, and the
+// output differed by 3e-4 of its norm from run to run.
 bool decode_fast_meta_aligned(int64_t rows_per_head, int Gv, int64_t heads) {
-    return kD / Gv > 1 || heads <= 1 || rows_per_head % 2 == 0;
+    const int ng = kD / Gv;
+    return ng == 4 || heads <= 1 || (rows_per_head * ng * 2) % 16 == 0;
 }
 
 bool decode_fast_eligible(const DecodeParams &p, int wk) {
