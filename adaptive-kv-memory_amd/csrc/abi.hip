@@ -71,7 +71,8 @@ bool fast_path(const akv_decode_args *a) {
           akv::decode_fast_meta_aligned(w.n_warm, w.group_v, (int64_t)a->B * a->Hkv)))
         return false;
     // outlier channels: up to 4 per block with 32-channel V groups; the ring must fit the LDS
-    if (w.n_out != 0 && !(w.n_out <= 4 && w.group_v == 32 && w.k_odata && w.v_odata && w.k_oidx && w.v_oidx))
+    if (w.n_out != 0 && !(w.n_out <= 4 && w.group_v == 32 && w.k_odata && w.v_odata && w.k_oidx && w.v_oidx &&
+                          akv::decode_fast_outliers_aligned(w.k_odata, w.v_odata)))
         return false;
     return akv::decode_fast_lds_bytes(akv::decode_fast_slot_bytes(w.bits_k, w.bits_v, w.group_v, w.n_out, false),
                                       w.n_out) <= 160 * 1024;

@@ -77,6 +77,8 @@ bool decode_fast_legacy_shape(int D, int bits, int group_size, int meta_dtype);
 // The fast kernel loads per-token meta rows of 1 or 2 groups in 16-byte pieces: with `heads`
 // tiers of `rows_per_head` token rows each, every tier's meta must start on 16 bytes.
 bool decode_fast_meta_aligned(int64_t rows_per_head, int Gv, int64_t heads);
+// The fast kernel loads the outlier values by dwords from the tensors' start on.
+bool decode_fast_outliers_aligned(const void *k_odata, const void *v_odata);
 int64_t decode_fast_lds_bytes(int64_t slot_bytes, int n_out);
 int decode_fast_waves(int n_out);
 hipError_t decode_fast_split_launch(const DecodeParams &p, int kb, int vb, int wk, hipStream_t s);

@@ -110,9 +110,10 @@ constexpr int kWaves = AKV_FAST_WAVES;  // waves per workgroup (one workgroup pe
 constexpr int kUnit = 32;               // warm tokens per ring slot
 constexpr int kNS = AKV_FAST_NS;        // ring slots per wave (deeper rings only lengthen the tail)
 // OUT selects the outlier-channel variant: 0 none; 1 exactly one channel per
-// block (the one-channel paths only: 147-156 VGPRs, so 12 waves with 2 slots
+// block (the one-channel paths only: 163-168 VGPRs, so 12 waves with 2 slots
 // like OUT = 0); kMaxOut up to 4 channels, whose general corrections hold more
 // state per lane: 8 waves (2 per SIMD, twice the registers each) with 3 slots.
+// ODD: a head has an odd number of outlier values (odd length and count).
 #ifndef AKV_FAST_WAVES_OUT
 #define AKV_FAST_WAVES_OUT 8
 #endif
@@ -157,7 +158,7 @@ struct WarmRes {
     u4 ko, vo, ki, vi;  // outlier values and indices
 };
 
-template <int BK, int BV, int NG, int OUT, bool LEG>
+template <int BK, int BV, int NG, int OUT, bool ODD, bool LEG>
 __device__ __forceinline__ void issue_warm(const WarmRes &R, unsigned char *slot, int lane, int u, int T, int tshift,
                                            int n_out) {
     using L = WarmLayout<BK, BV, NG, OUT, LEG>;
@@ -199,8 +200,10 @@ __device__ __forceinline__ void issue_warm(const WarmRes &R, unsigned char *slot
     if (OUT) {
         const uint32_t ob = (uint32_t)(kUnit * n_out * 2);  // 64 n_out bytes of values per unit
         const uint64_t im = lane_mask((n_out * 8 + 15) & ~15);
-        dma16(R.ko, base + L::KO, v16, (uint32_t)u * ob, lane_mask((int)ob));
-        dma16(R.vo, base + L::VO, v16, (uint32_t)u * ob, lane_mask((int)ob));
+        // ODD: a piece more, as the values may start half a dword in (n_out 1 or 3: it fits)
+        const uint64_t om = lane_mask((int)ob + (ODD ? 16 : 0));
+        dma16(R.ko, base + L::KO, v16, (uint32_t)u * ob, om);
+        dma16(R.vo, base + L::VO, v16, (uint32_t)u * ob, om);
         dma16(R.ki, base + L::KI, v16, blk * (uint32_t)(n_out * 8), im);
         dma16(R.vi, base + L::VI, v16, blk * (uint32_t)(n_out * 8), im);
     }
@@ -285,7 +288,7 @@ __device__ __forceinline__ void wait_younger(int nw, int nh) {
     else wait_vm<0>();
 }
 
-template <int BK, int BV, int NG, int NS, int OUT, bool LEG>
+template <int BK, int BV, int NG, int NS, int OUT, bool ODD, bool LEG>
 __global__ __launch_bounds__(64 * FastCfg<OUT>::NW)
 __attribute__((amdgpu_waves_per_eu(FastCfg<OUT>::NW / 4, FastCfg<OUT>::NW / 4)))
 void decode_fast_kernel(const DecodeParams p) {
@@ -375,6 +378,7 @@ void decode_fast_kernel(const DecodeParams p) {
     if (threadIdx.x == 0) *work = (unsigned)NW;
 
     WarmRes R;
+    int ofix = 0;  // ODD: the first unit whose outlier values are put right; -1: all, by half a dword
     {
         const uint32_t nwu = (uint32_t)p.n_warm;
         // first token row of this (batch, kv-head)'s warm tier: dense per (batch, kv-head) for the
@@ -400,9 +404,17 @@ void decode_fast_kernel(const DecodeParams p) {
         R.vs = rsrc4((const _Float16 *)p.vs + wrow * NG, mrec);
         R.vz = rsrc4((const _Float16 *)p.vz + wrow * NG, mrec);
         if (OUT) {
-            const int no = OUT == 1 ? 1 : p.n_out;
-            R.ko = rsrc4(p.k_odata + bh * p.n_warm * no, nwu * (uint32_t)no * 2);
-            R.vo = rsrc4(p.v_odata + bh * p.n_warm * no, nwu * (uint32_t)no * 2);
+            // ODD: with an odd number of values per head every second head's start half a dword
+            // in.  LDS loads and the range check work on dwords: those ranges start at the dword,
+            // and a range that ends in half a dword is rounded up to it.
+            const int no = OUT == 1 ? 1 : p.n_out, oshift = ODD ? (int)(bh & 1) : 0;
+            uint32_t orec = nwu * (uint32_t)no * 2u;
+            if (ODD) {
+                ofix = oshift ? -1 : (int)(p.n_warm / kUnit);
+                orec = (orec + 2u * (uint32_t)oshift + 3u) & ~3u;
+            }
+            R.ko = rsrc4(p.k_odata + bh * p.n_warm * no - oshift, orec);
+            R.vo = rsrc4(p.v_odata + bh * p.n_warm * no - oshift, orec);
             R.ki = rsrc4(p.k_oidx + (int64_t)b * p.nblk * no, (uint32_t)(p.nblk * no * 8));
             R.vi = rsrc4(p.v_oidx + (int64_t)b * p.nblk * no, (uint32_t)(p.nblk * no * 8));
         }
@@ -440,7 +452,7 @@ void decode_fast_kernel(const DecodeParams p) {
         }
     };
     auto issue = [&](int k, int id, unsigned char *slot) {
-        if (k == kWarm) issue_warm<BK, BV, NG, OUT, LEG>(R, slot, lane, id, p.T, p.tshift, OUT == 1 ? 1 : p.n_out);
+        if (k == kWarm) issue_warm<BK, BV, NG, OUT, ODD, LEG>(R, slot, lane, id, p.T, p.tshift, OUT == 1 ? 1 : p.n_out);
         else if (k == kHotK) issue_hot(rkh, slot, lane, id);
         else if (k == kHotV) issue_hot(rvh, slot, lane, id);
     };
@@ -578,6 +590,25 @@ void decode_fast_kernel(const DecodeParams p) {
                 }
             }
             __builtin_amdgcn_wave_barrier();
+        }
+        if constexpr (ODD) {
+            if (id >= ofix) {
+                // outlier values half a dword in: move them down to where the even heads' lie; and
+                // in the tail unit clear what the range's last dword holds past the tier
+                const int no = OUT == 1 ? 1 : p.n_out, left = (nw - id * kUnit) * no - 2 * lane;
+                if (lane < kUnit / 2 * no) {
+                    uint32_t *kd = (uint32_t *)(slot + L::KO) + lane, *vd = (uint32_t *)(slot + L::VO) + lane;
+                    uint32_t a = kd[0], c = vd[0];
+                    if (ofix < 0) {
+                        a = __builtin_amdgcn_alignbyte(kd[1], a, 2);
+                        c = __builtin_amdgcn_alignbyte(vd[1], c, 2);
+                    }
+                    const uint32_t m = left >= 2 ? ~0u : left == 1 ? 0xFFFFu : 0u;
+                    *kd = a & m;
+                    *vd = c & m;
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
         }
         {
             // ---- LDS reads at the top of the unit, issued together (the empty asm with a memory
@@ -1191,6 +1222,10 @@ bool decode_fast_meta_aligned(int64_t rows_per_head, int Gv, int64_t heads) {
     return ng == 4 || heads <= 1 || (rows_per_head * ng * 2) % 16 == 0;
 }
 
+bool decode_fast_outliers_aligned(const void *k_odata, const void *v_odata) {
+    return (((uintptr_t)k_odata | (uintptr_t)v_odata) & 3u) == 0;
+}
+
 bool decode_fast_eligible(const DecodeParams &p, int wk) {
     if (wk == AKV_WARM_LEGACY) {
         if (!(decode_fast_legacy_shape(p.D, p.kc_row * 8 / kD, p.gs, p.meta_dt) && p.kc_row == p.vc_row &&
@@ -1202,12 +1237,13 @@ bool decode_fast_eligible(const DecodeParams &p, int wk) {
           decode_fast_meta_aligned(p.n_warm, p.Gv, (int64_t)p.B * p.Hkv)))
         return false;
     // outlier channels: up to kMaxOut per block, V groups of 32 channels; the ring must fit the LDS
-    if (p.n_out != 0 && !(p.n_out <= kMaxOut && p.Gv == 32 && p.k_odata && p.v_odata && p.k_oidx && p.v_oidx))
+    if (p.n_out != 0 && !(p.n_out <= kMaxOut && p.Gv == 32 && p.k_odata && p.v_odata && p.k_oidx && p.v_oidx &&
+                          decode_fast_outliers_aligned(p.k_odata, p.v_odata)))
         return false;
     return p.slot_bytes > 0 && decode_fast_lds_bytes(p.slot_bytes, p.n_out) <= kLdsCap;
 }
 
-template <int BK, int BV, int NG, int NS, int OUT, bool LEG>
+template <int BK, int BV, int NG, int NS, int OUT, bool ODD, bool LEG>
 static hipError_t launch_fast_ns(const DecodeParams &p, hipStream_t s) {
     const dim3 grid((unsigned)(p.nsplit * p.Hkv * p.B * p.nchunk));  // decoded in the kernel
     const size_t lds = (size_t)decode_fast_lds_bytes(p.slot_bytes, OUT ? p.n_out : 0);
@@ -1219,26 +1255,34 @@ static hipError_t launch_fast_ns(const DecodeParams &p, hipStream_t s) {
     if (e != hipSuccess) return e;
     const uint64_t bit = (dev >= 0 && dev < 64) ? 1ull << dev : 0ull;
     if (!bit || !(attr_devs.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)decode_fast_kernel<BK, BV, NG, NS, OUT, LEG>,
+        e = hipFuncSetAttribute((const void *)decode_fast_kernel<BK, BV, NG, NS, OUT, ODD, LEG>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLdsCap);
         if (e != hipSuccess) return e;
         attr_devs.fetch_or(bit, std::memory_order_release);
     }
-    hipLaunchKernelGGL((decode_fast_kernel<BK, BV, NG, NS, OUT, LEG>), grid, dim3(64 * FastCfg<OUT>::NW), lds, s, p);
+    hipLaunchKernelGGL((decode_fast_kernel<BK, BV, NG, NS, OUT, ODD, LEG>), grid, dim3(64 * FastCfg<OUT>::NW), lds, s,
+                       p);
     return hipGetLastError();
 }
 
 template <int BK, int BV, int NG, bool LEG>
 static hipError_t launch_fast(const DecodeParams &p, hipStream_t s) {
-    return launch_fast_ns<BK, BV, NG, kNS, 0, LEG>(p, s);
+    return launch_fast_ns<BK, BV, NG, kNS, 0, false, LEG>(p, s);
 }
 
 template <int BK, int BV, bool LEG>
 static hipError_t launch_fast_ng(const DecodeParams &p, hipStream_t s) {
-    if (!LEG && p.n_out > 0)
-        return p.Gv != 32 ? hipErrorInvalidValue
-               : p.n_out == 1 ? launch_fast_ns<BK, BV, 4, kNS, 1, false>(p, s)
-                              : launch_fast_ns<BK, BV, 4, kNSOut, kMaxOut, false>(p, s);
+    if (!LEG && p.n_out > 0) {
+        // an odd number of outlier values per head has its own instantiations: straightening them
+        // in these cost the even ones 2% (8 sequences x 31,744 tokens, one channel: 26.6 -> 27.1 us)
+        const bool odd = p.n_warm & p.n_out & 1;
+        if (p.Gv != 32) return hipErrorInvalidValue;
+        if (p.n_out == 1)
+            return odd ? launch_fast_ns<BK, BV, 4, kNS, 1, true, false>(p, s)
+                       : launch_fast_ns<BK, BV, 4, kNS, 1, false, false>(p, s);
+        return odd ? launch_fast_ns<BK, BV, 4, kNSOut, kMaxOut, true, false>(p, s)
+                   : launch_fast_ns<BK, BV, 4, kNSOut, kMaxOut, false, false>(p, s);
+    }
     if (p.Gv == 32) return launch_fast<BK, BV, 4, LEG>(p, s);
     if (p.Gv == 64) return launch_fast<BK, BV, 2, LEG>(p, s);
     if (p.Gv == 128) return launch_fast<BK, BV, 1, LEG>(p, s);

@@ -6,7 +6,7 @@ import ctypes
 import pytest
 
 
-def _workspace(kind="affine", B=3, Hq=28, Hkv=4, M=3, n_warm=9001, group=64, n_out=0, stride=0):
+def _workspace(kind="affine", B=3, Hq=28, Hkv=4, M=3, n_warm=9001, group=64, n_out=0, stride=0, odata=0x30000):
     from akv import _native as nat
     lib = nat.load()
     a = nat.DecodeArgs()
@@ -22,7 +22,8 @@ def _workspace(kind="affine", B=3, Hq=28, Hkv=4, M=3, n_warm=9001, group=64, n_o
     if kind == "affine":
         w.kind, w.bits_k, w.bits_v, w.block_t, w.group_v, w.n_out = nat.WARM_AFFINE, 2, 2, 32, group, n_out
         if n_out:
-            w.k_oidx = w.v_oidx = w.k_odata = w.v_odata = 0x30000
+            w.k_oidx = w.v_oidx = 0x30000
+            w.k_odata = w.v_odata = odata
     else:
         w.kind, w.bits_k, w.bits_v, w.group_size = nat.WARM_LEGACY, 4, 4, group
         w.meta_dtype, w.legacy_sym, w.warm_heads = nat.DT_F16, 0, B * Hkv
@@ -44,3 +45,13 @@ def test_meta_rows_off_16_bytes_leave_the_fast_kernel(kind, group, n, fast):
     assert _fast(kind=kind, group=group, n_warm=n) == fast
     if kind == "legacy":  # a tier's rows are `stride` apart whatever its length
         assert _fast(kind=kind, group=group, n_warm=9001, stride=n + 8) == fast
+
+
+@pytest.mark.parametrize("n_out", [1, 2, 3, 4])
+@pytest.mark.parametrize("n", [9000, 9001])
+def test_outlier_values_off_a_dword_leave_the_fast_kernel(n_out, n):
+    """Odd lengths and counts stay (every second head's values start half a dword in, which the
+    kernel straightens); tensors that start half a dword in do not."""
+    kw = dict(B=3, Hq=4, Hkv=4, M=1, n_warm=n, group=32, n_out=n_out)
+    assert _fast(**kw)
+    assert not _fast(**kw, odata=0x30002)

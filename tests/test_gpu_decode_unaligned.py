@@ -110,3 +110,33 @@ def test_odd_two_group_tiers_repeat(B, Hkv, Hq, M, bits, Nw, Nh):
         runs.append((*akv.decode_attention(q, kh, vh, warm, scores=s, decay=0.9, return_weights=True), s))
     for run in runs[1:]:
         assert all(torch.equal(a, b) for a, b in zip(run, runs[0]))
+
+
+@pytest.mark.parametrize("B,Hkv,Hq,M,frac", [(1, 1, 4, 1, 0.01), (2, 3, 6, 2, 0.01), (2, 2, 2, 1, 0.024)])
+@pytest.mark.parametrize("Nw", [31, 777, 4001])
+@pytest.mark.parametrize("weights", [False, True])
+def test_odd_outlier_counts(B, Hkv, Hq, M, frac, Nw, weights):
+    """One and three protected channels over tiers of odd length: a head's outlier values are an odd
+    number of 16-bit values, so every second head's start at half a dword."""
+    import akv
+    announce(f"decode odd outliers B{B} Hkv{Hkv} M{M} frac{frac} Nw={Nw} weights={weights}")
+    g = torch.Generator(device="cuda").manual_seed(Nw + B)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda").half()  # noqa: E731
+    Nh = 37
+    kw, vw, kh, vh, q = r(B, Hkv, Nw, 128), r(B, Hkv, Nw, 128), r(B, Hkv, Nh, 128), r(B, Hkv, Nh, 128), r(B, Hq, M, 128)
+    kw[..., 5] *= 8  # the channel that is protected carries most of a logit
+    vw[..., 77] *= 8
+    warm = akv.quantize_kv(kw, vw, 4, 2, 32, 32, outlier_fraction=frac)
+    assert warm.n_out % 2 == 1
+    kd, vd = akv.dequantize(warm)
+    exp, p = _reference(q, torch.cat([kd, kh], dim=2), torch.cat([vd, vh], dim=2))
+    s0 = torch.rand(Nw + Nh, generator=g, device="cuda")
+    s = s0.clone()
+    out = akv.decode_attention(q, kh, vh, warm, scores=s, decay=0.9, return_weights=weights)
+    if weights:
+        out, w = out
+        # fp32 logits of |s| < 128 and exp2: 128 * 2^-23 relative, a few times over
+        torch.testing.assert_close(w.double(), p, rtol=1e-4, atol=1e-9)
+    # 16-bit probabilities and output: 2^-11 of values up to 40 in the protected channel, averaged
+    assert float((out.double() - exp).norm() / exp.norm()) <= 1e-3
+    torch.testing.assert_close(s.double(), s0.double() * 0.9 + p.sum((0, 1, 2)) / (B * Hq), rtol=1e-4, atol=1e-8)
