@@ -578,14 +578,15 @@ __global__ __launch_bounds__(256) AKV_SPLIT_ATTR void decode_split_kernel(const 
 
                 const h4 pop = softmax_tile(stt, s, sl2);
                 // ---- V dequant (4 tokens x 8 channels of chunk col) + PV per channel slot
-                int vo_dj[2] = {-1, -1};  // outlier channels of this block in this lane's chunk (first two)
+                // outlier channels of this block in this lane's chunk: byte c is 1 + the outlier
+                // whose channel is 8 col + c (0: none; n_out <= D, so it fits)
+                uint64_t vo_of = 0;
                 if (OUTL) {
                     const int64_t blk = t0 / p.T;
-                    int cnt = 0;
 #pragma unroll 1
-                    for (int j = 0; j < p.n_out && cnt < 2; ++j) {
+                    for (int j = 0; j < p.n_out; ++j) {
                         const int dj = min(max((int)p.v_oidx[((int64_t)b * p.nblk + blk) * p.n_out + j], 0), D - 1);
-                        if (dj / 8 == col) vo_dj[cnt++] = j;
+                        if (dj / 8 == col) vo_of |= (uint64_t)(j + 1) << (8 * (dj % 8));
                     }
                 }
 #pragma unroll
@@ -634,13 +635,9 @@ __global__ __launch_bounds__(256) AKV_SPLIT_ATTR void decode_split_kernel(const 
                         a23 = (h2){(_Float16)d[2], (_Float16)d[3]};
                     }
                     h4 vop = {a01[0], a01[1], a23[0], a23[1]};
-                    if (OUTL && vo_dj[0] >= 0) {  // rare: outlier channels replace values
-#pragma unroll
-                        for (int q = 0; q < 2; ++q) {
-                            const int jo = vo_dj[q];
-                            if (jo < 0) continue;
-                            const int dj = (int)p.v_oidx[((int64_t)b * p.nblk + t0 / p.T) * p.n_out + jo];
-                            if (vpair_chan<VB>(j) != dj % 8) continue;
+                    if (OUTL && vo_of) {  // rare: outlier channels replace values
+                        const int jo = (int)(vo_of >> (8 * vpair_chan<VB>(j)) & 0xFFu) - 1;
+                        if (jo >= 0) {
 #pragma unroll
                             for (int i = 0; i < 4; ++i) {
                                 const int64_t tv = min(t0 + 4 * grp + i, nwarm - 1);
