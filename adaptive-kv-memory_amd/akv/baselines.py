@@ -127,7 +127,7 @@ class _Tier:
         self.B, self.H, self.rows, self.D, self.bits, self.gs = B, H, B * H, D, bits, gs
         pD = padded_dim(D, gs)
         self.row_bytes, self.G = pD * bits // 8, pD // gs
-        self.n, self.cap, self.keep_f16 = 0, 0, keep_f16
+        self.n, self.cap, self.dirty, self.keep_f16 = 0, 0, 0, keep_f16
         self.device = device
         self.codes = self.sc = self.ze = self.sc16 = self.ze16 = None
 
@@ -149,15 +149,15 @@ class _Tier:
             self.ze16 = grow(self.ze16, (R, cap, G), torch.float16)
         self.cap = cap
 
-    def reserve(self, n: int) -> int:
-        """Room for n more rows; where the tier grew, the row up to which the caller has to
-        clear those past its own (rows past the tier read as zeros), else 0."""
+    def reserve(self, n: int):
+        """Room for n more rows.  Rows past the tier read as zeros: those of a grown tier, up to row
+        ``dirty``, have to be cleared by the launch that appends."""
         if self.n + n <= self.cap:
-            return 0
+            return
         cap = max(64, self.cap)
         while cap < self.n + n:
             cap *= 2
-        mv = RowMoves()
+        mv, grown = RowMoves(), {}
         for name, width, dtype in (("codes", self.row_bytes, torch.uint8), ("sc", self.G, torch.float32),
                                    ("ze", self.G, torch.float32), ("sc16", self.G, torch.float16),
                                    ("ze16", self.G, torch.float16)):
@@ -165,10 +165,9 @@ class _Tier:
                 old, new = getattr(self, name), torch.empty(self.rows, cap, width, dtype=dtype, device=self.device)
                 if old is not None:
                     mv.copy(new.unsqueeze(0), old.unsqueeze(0), self.n)
-                setattr(self, name, new)
+                grown[name] = new
         mv.run()
-        self.cap = cap
-        return cap
+        self.__dict__.update(grown, cap=cap, dirty=cap)
 
     def append(self, codes, sc, ze):
         n = codes.shape[1]
@@ -223,16 +222,15 @@ class KIVICache:
         cfg = self.config
         nat.require_device(key_states, value_states)
         if layer_idx not in self._residual_keys:
-            self._residual_keys[layer_idx] = key_states
-            self._residual_values[layer_idx] = value_states
+            rk, rv = key_states, value_states
             self._seq_lens[layer_idx] = key_states.shape[2]
         else:
-            self._residual_keys[layer_idx] = torch.cat([self._residual_keys[layer_idx], key_states], dim=2)
-            self._residual_values[layer_idx] = torch.cat([self._residual_values[layer_idx], value_states], dim=2)
+            rk = torch.cat([self._residual_keys[layer_idx], key_states], dim=2)
+            rv = torch.cat([self._residual_values[layer_idx], value_states], dim=2)
             self._seq_lens[layer_idx] += key_states.shape[2]
-        if self._residual_keys[layer_idx].shape[2] > cfg.residual_length:
-            self._quantize_overflow(layer_idx)
-        return self._get_full_kv(layer_idx)
+        self._residual_keys[layer_idx], self._residual_values[layer_idx] = rk, rv
+        views = self._quantize_overflow(layer_idx) if rk.shape[2] > cfg.residual_length else None
+        return self._get_full_kv(layer_idx) if views is None else views
 
     def _new_tier(self, x: torch.Tensor, bits: int) -> "_Tier":
         B, H, _, D = x.shape
@@ -295,88 +293,97 @@ class KIVIFusedCache(KIVICache):
         super().__init__(config or KIVIFusedConfig())
         self._dequant_keys_cache: dict = {}    # layer -> the tier its dequantized rows come from
         self._dequant_values_cache: dict = {}
-        self._views: dict = {}  # layer -> between an overflow and its view: (view, rows before the chunk) of
-                                # K and V, the residual tokens, the moves still to run
         self._ws: dict = {}  # per-device decode workspace of fused_attention
 
     def _quantize_overflow(self, layer_idx: int):
-        """akv/baselines.py:455-496.  One launch quantizes, appends and dequantizes the
-        overflow of both tensors and writes its rows of the view; ``_get_full_kv`` runs the
-        one that cuts the residuals and completes the view."""
+        """akv/baselines.py:455-496; returns the layer's full K / V.  One launch quantizes,
+        appends and dequantizes the overflow of both tensors and writes its rows of the view, one
+        cuts the residuals and completes the view.  Everything is allocated before the first
+        launch, and tiers and residuals change after the last: a call that fails before leaves
+        the tokens in the residual window."""
         cfg = self.config
-        res = (self._residual_keys, self._residual_values)
+        res = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
         for bits, r in ((cfg.key_bits, res[0]), (cfg.value_bits, res[1])):
-            _check_shape(r[layer_idx].shape[3], bits, cfg.group_size)
-        sides, views = [], [None, None]
-        for i, (bits, tiers, served) in enumerate(((cfg.key_bits, self._quant_keys, self._dequant_keys_cache),
-                                                  (cfg.value_bits, self._quant_values, self._dequant_values_cache))):
-            r = res[i][layer_idx]
+            _check_shape(r.shape[3], bits, cfg.group_size)
+        sides, args, mv = [], [], RowMoves()
+        for bits, tiers, r in ((cfg.key_bits, self._quant_keys, res[0]), (cfg.value_bits, self._quant_values, res[1])):
             B, H, n_all, D = r.shape
-            n_q = n_all - cfg.residual_length
-            x, left = r[:, :, :n_q], r[:, :, n_q:]
-            n = x.shape[2]
-            if layer_idx not in tiers:
-                tiers[layer_idx] = self._new_tier(x, bits)
-            tier = served[layer_idx] = tiers[layer_idx]
-            grown = tier.reserve(n)
+            n = n_all - cfg.residual_length
+            x, left = r[:, :, :n], r[:, :, n:]
+            tier = tiers[layer_idx] if layer_idx in tiers else self._new_tier(x, bits)
+            tier.reserve(n)
             if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
                 x = x.float()
             e = x.element_size()
             if x.stride(3) != 1 or x.data_ptr() % 16 or any(st * e % 16 for st in x.stride()[:3]):
                 x = nat.dev_contig(x)
             dt = torch.promote_types(torch.float16, left.dtype)
-            view = None
+            view = old = None
             if movable(dt, left) and dt in (torch.float16, torch.float32):
-                view = torch.empty(B, H, tier.n + n + left.shape[2], D, dtype=dt, device=r.device)
-                views[i] = (view, tier.n)
-            sides.append((x, B, H, D, n, dt, nat.KiviSide(
+                view, old = self._new_view(tier, tier.n, n, left, dt, mv)
+            if movable(left.dtype, left) and left.stride(3) == 1:
+                kept = torch.empty(left.shape, dtype=left.dtype, device=left.device)
+                mv.copy(kept, left, left.shape[2])
+            else:
+                kept = left.contiguous()
+            sides.append((tier, n, view, old, kept))
+            args.append((x, B, H, D, n, dt, nat.KiviSide(
                 x.data_ptr(), x.stride(0) * e, x.stride(1) * e, x.stride(2) * e, tier.codes.data_ptr(),
                 tier.sc.data_ptr(), tier.ze.data_ptr(), tier.sc16.data_ptr(), tier.ze16.data_ptr(),
-                None if view is None else view.data_ptr(), tier.cap, tier.n, grown,
+                None if view is None else view.data_ptr(), tier.cap, tier.n, tier.dirty,
                 0 if view is None else view.shape[2], bits, 0)))
-            tier.n += n
-        groups = [sides] if sides[0][1:6] == sides[1][1:6] and sides[0][0].dtype == sides[1][0].dtype else [sides[:1], sides[1:]]
+        groups = [args] if args[0][1:6] == args[1][1:6] and args[0][0].dtype == args[1][0].dtype else [args[:1], args[1:]]
         for g in groups:
             x, B, H, D, n, dt, _ = g[0]
             arr = (nat.KiviSide * len(g))(*(s[6] for s in g))
             nat.check(nat.load().akv_kivi_append(
                 arr, len(g), B, H, D, n, nat.dtype_code(x.dtype), cfg.group_size,
                 nat.DT_F16 if dt == torch.float16 else nat.DT_F32, nat.stream_of(x)), "KIVI append")
-        mv, lefts = RowMoves(), []
-        for i in (0, 1):
-            r = res[i][layer_idx]
-            left = r[:, :, r.shape[2] - cfg.residual_length:]
-            if movable(left.dtype, left) and left.stride(3) == 1:
-                new = torch.empty(left.shape, dtype=left.dtype, device=left.device)
-                mv.copy(new, left, left.shape[2])
-                res[i][layer_idx] = new
-            else:
-                res[i][layer_idx] = left = left.contiguous()
-            lefts.append(left)
-        self._views[layer_idx] = views, lefts, mv
+        for tier, _, view, old, _ in sides:
+            if view is not None:
+                self._fill_view(tier, view, old, tier.n)
+        mv.run()
+        (kt, nk, _, _, rk), (vt, nv, _, _, rv) = sides
+        kt.n, vt.n, kt.dirty, vt.dirty = kt.n + nk, vt.n + nv, 0, 0
+        self._quant_keys[layer_idx], self._quant_values[layer_idx] = kt, vt
+        self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx] = kt, vt
+        self._residual_keys[layer_idx], self._residual_values[layer_idx] = rk, rv
+        return tuple(torch.cat([tier.dequantize(), kept], dim=2) if view is None else view
+                     for tier, _, view, _, kept in sides)
+
+    @staticmethod
+    def _new_view(tier: _Tier, had: int, n: int, left: torch.Tensor, dt: torch.dtype, mv: RowMoves):
+        """The view over ``had`` rows of the tier, n more that the caller writes and the residual
+        ``left``, whose move is queued: (view, and for a float32 view the float16 buffer of those
+        ``had`` rows, whose move is queued too)."""
+        view = torch.empty(tier.B, tier.H, had + n + left.shape[2], tier.D, dtype=dt, device=left.device)
+        old = None
+        if had and dt != torch.float16:
+            old = torch.empty(tier.rows, had, tier.D, dtype=torch.float16, device=left.device)
+            mv.copy(view, old.view(tier.B, tier.H, had, tier.D), had)
+        mv.copy(view, left if left.stride(3) == 1 else left.contiguous(), left.shape[2], at=had + n)
+        return view, old
+
+    @staticmethod
+    def _fill_view(tier: _Tier, view: torch.Tensor, old: Optional[torch.Tensor], had: int):
+        """Dequantize the first ``had`` rows of the tier into ``view`` (float32: into ``old``)."""
+        if had:
+            dequantize_rows(tier.codes, tier.sc, tier.ze, tier.bits, tier.gs, tier.D, n=had,
+                            out=view.view(tier.rows, view.shape[2], tier.D) if old is None else old)
 
     def _get_full_kv(self, layer_idx: int):
         """akv/baselines.py:498-510."""
         rs = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
         if layer_idx not in self._dequant_keys_cache:
             return rs
-        # an overflow's residual moves go with the view's; the view reads the tokens they read
-        views, rs, mv = self._views.pop(layer_idx, ([None, None], rs, RowMoves()))
-        out = []
-        for i, tier in enumerate((self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx])):
-            n, r = tier.n, rs[i]
+        mv, out = RowMoves(), []
+        for tier, r in zip((self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx]), rs):
             dt = torch.promote_types(torch.float16, r.dtype)
             if not movable(dt, r) or r.shape[:2] != (tier.B, tier.H) or r.shape[3] != tier.D:
                 out.append(torch.cat([tier.dequantize(), r], dim=2))
                 continue
-            view, had = views[i] or (torch.empty(tier.B, tier.H, n + r.shape[2], tier.D, dtype=dt, device=r.device), n)
-            if had and dt == torch.float16:  # the rows the overflow launch has not written
-                dequantize_rows(tier.codes, tier.sc, tier.ze, tier.bits, tier.gs, tier.D, n=had,
-                                out=view.view(tier.rows, view.shape[2], tier.D))
-            elif had:
-                old = dequantize_rows(tier.codes, tier.sc, tier.ze, tier.bits, tier.gs, tier.D, n=had)
-                mv.copy(view, old.view(tier.B, tier.H, had, tier.D), had)
-            mv.copy(view, r if r.stride(3) == 1 else r.contiguous(), r.shape[2], at=n)
+            view, old = self._new_view(tier, tier.n, 0, r, dt, mv)
+            self._fill_view(tier, view, old, tier.n)
             out.append(view)
         mv.run()
         return out[0], out[1]
