@@ -181,7 +181,8 @@ class _EventTier:
 
     def append(self, w: WarmTier, positions: torch.Tensor, mv: RowMoves):
         """One demotion event: ``w`` holds its n tokens as a single K block; their positions
-        are those of ``positions`` at the list ``mv`` is run with."""
+        are those of ``positions`` at the list ``mv`` is run with.  Returns what takes the event
+        into the tier, to be called once ``mv`` has run."""
         n = w.n_warm
         if self.n + n > self.cap or self.n_events + 1 > self.ecap:
             self._grow(max(self.cap, 2 * (self.n + n)), max(self.ecap, 2 * (self.n_events + 1)))
@@ -197,8 +198,10 @@ class _EventTier:
             mv.copy(t["voi"].unsqueeze(1), w.v_oidx.unsqueeze(1), 1, at=e)
         mv.count(t["blk"], n, e, 0, at=a)
         mv.copy(t["pos"], positions, n, GATHER, at=a)
-        self.n += n
-        self.n_events += 1
+
+        def commit():
+            self.n, self.n_events = a + n, e + 1
+        return commit
 
     def positions(self) -> torch.Tensor:
         return self.t["pos"][: self.n]
@@ -249,8 +252,8 @@ class _EventTier:
         nat.check(nat.load().akv_dequant_unpack(ctypes.byref(a), nat.stream_of(out_k)), "AKVLayer warm view")
 
     def pull(self, idx: torch.Tensor, vector: Optional[torch.Tensor] = None):
-        """The float16 K, V (B, H, n, D) of the warm tokens of the ascending list ``idx``, which
-        leave the tier, and ``vector`` as ``remove`` gives it."""
+        """The float16 K, V (B, H, n, D) of the warm tokens of the ascending list ``idx``, then
+        ``vector`` without them and what takes them out of the tier, as ``remove`` gives both."""
         n = idx.numel()
         sub = _EventTier.__new__(_EventTier)
         sub.__dict__.update({k: v for k, v in self.__dict__.items() if k != "t"})
@@ -264,33 +267,34 @@ class _EventTier:
                 mv.copy(sub.t[name], x, n, GATHER)
             else:
                 sub.t[name] = x
-        kept = self.remove(idx, n, vector, mv)
-        sub.n, sub.cap = n, n
         k = torch.empty(self.B, self.H, n, self.D, dtype=torch.float16, device=self.dev)
         v = torch.empty_like(k)
+        kept, commit = self.remove(idx, n, vector, mv)
+        sub.n, sub.cap = n, n
         sub.dequantize_into(k, v, slots=False)
-        return k, v, kept
+        return k, v, kept, commit
 
     def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None,
-               mv: Optional[RowMoves] = None) -> Optional[torch.Tensor]:
-        """Drop the ``n`` warm tokens of the ascending list ``idx`` (their events' K meta rows
-        stay); ``vector`` (one float32 per warm token) is returned without theirs.  The kept
-        rows go to fresh tensors: rows shift by up to n, so a move in place would race.  ``mv``:
-        jobs on the same list that go with the launch."""
+               mv: Optional[RowMoves] = None):
+        """The tier without the ``n`` warm tokens of the ascending list ``idx`` (their events' K
+        meta rows stay): ``vector`` (one float32 per warm token) without theirs, and what takes
+        them out of the tier.  The kept rows go to fresh tensors: rows shift by up to n, so a
+        move in place would race.  ``mv``: jobs on the same list that go with the launch."""
         kept = self.n - n
         mv = mv or RowMoves()
-        for name in self._TOKEN_AXIS:
-            if name in self.t:
-                x = self.t[name]
-                self.t[name] = torch.empty_like(x)
-                mv.copy(self.t[name], x, kept, KEEP)
+        fresh = {name: torch.empty_like(self.t[name]) for name in self._TOKEN_AXIS if name in self.t}
+        for name, x in fresh.items():
+            mv.copy(x, self.t[name], kept, KEEP)
         out = None
         if vector is not None:
             out = torch.empty(kept, dtype=vector.dtype, device=vector.device)
             mv.copy(out, vector, kept, KEEP)
         mv.run(idx, n)
-        self.n = kept
-        return out
+
+        def commit():
+            self.t.update(fresh)
+            self.n = kept
+        return out, commit
 
     def index_batch(self, beam_idx: torch.Tensor):
         for name in list(self.t):
@@ -315,27 +319,32 @@ class _HeadBitsTier:
             heads = [h for h, b in enumerate(per_head_bits) if b == bits]
             self.groups.append([bits, torch.tensor(heads, dtype=torch.long, device=dev), None])
 
-    def demote(self, hk, hv, idx, outlier_fraction, positions) -> int:
+    def demote(self, hk, hv, idx, outlier_fraction, positions):
         """Quantize hot tokens ``idx`` (at ``positions[idx]``) of every head with its width as one event; returns
-        the measured packed bytes (codes + scale + zero of K and V, per head)."""
+        the measured packed bytes (codes + scale + zero of K and V, per head) and what takes the event
+        into the tier."""
         B, _, _, D = hk.shape
         n = idx.numel()
-        packed = 0
-        for g in self.groups:
-            bits, heads, tier = g
+        packed, staged = 0, []
+        for bits, heads, tier in self.groups:
             hs = heads.numel()
             k = hk.index_select(1, heads).index_select(2, idx).reshape(B * hs, 1, n, D)
             v = hv.index_select(1, heads).index_select(2, idx).reshape(B * hs, 1, n, D)
             w = quantize_kv(k, v, bits, bits, block_t=max(n, 1), group_v=D, outlier_fraction=outlier_fraction)
             if tier is None:
-                g[2] = tier = _EventTier(B * hs, 1, D, bits, bits, w.n_out, self.dev, n)
+                tier = _EventTier(B * hs, 1, D, bits, bits, w.n_out, self.dev, n)
             mv = RowMoves()
-            tier.append(w, positions, mv)
+            staged.append((tier, tier.append(w, positions, mv)))
             mv.run(idx, n)
             packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
                        + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
-        self.n += n
-        return packed
+
+        def commit():
+            for g, (tier, take) in zip(self.groups, staged):
+                g[2] = tier
+                take()
+            self.n += n
+        return packed, commit
 
     def resident_bytes(self) -> int:
         return sum(g[2].resident_bytes() for g in self.groups if g[2] is not None)
@@ -351,26 +360,33 @@ class _HeadBitsTier:
             if out_v is not None:
                 out_v.index_copy_(1, heads, tv.view(self.B, hs, rows, self.D))
 
+    def _taken(self, n: int, commits: list):
+        def commit():
+            for take in commits:
+                take()
+            self.n -= n
+        return commit
+
     def pull(self, idx: torch.Tensor, vector: Optional[torch.Tensor] = None):
         n = idx.numel()
         k = torch.empty(self.B, self.H, n, self.D, dtype=torch.float16, device=self.dev)
         v = torch.empty_like(k)
-        kept = None
+        kept, commits = None, []
         for i, (bits, heads, tier) in enumerate(self.groups):
-            tk, tv, out = tier.pull(idx, vector if i == 0 else None)
+            tk, tv, out, commit = tier.pull(idx, vector if i == 0 else None)
             kept = out if i == 0 else kept
+            commits.append(commit)
             k.index_copy_(1, heads, tk.view(self.B, heads.numel(), n, self.D))
             v.index_copy_(1, heads, tv.view(self.B, heads.numel(), n, self.D))
-        self.n -= n
-        return k, v, kept
+        return k, v, kept, self._taken(n, commits)
 
-    def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
-        out = None
+    def remove(self, idx: torch.Tensor, n: int, vector: Optional[torch.Tensor] = None):
+        out, commits = None, []
         for i, g in enumerate(self.groups):
-            kept = g[2].remove(idx, n, vector if i == 0 else None)
+            kept, commit = g[2].remove(idx, n, vector if i == 0 else None)
             out = kept if i == 0 else out
-        self.n -= n
-        return out
+            commits.append(commit)
+        return out, self._taken(n, commits)
 
     def positions(self) -> torch.Tensor:
         return self.groups[0][2].positions()
@@ -482,7 +498,8 @@ class AKVLayer:
         """The hot tier with the promoted tokens in front and the new ones (k, v) behind, their
         positions, and the importance: 2 for the promoted, decayed for the old, 1 for the new
         (akv/drop_in.py:375-389, :433-484); one launch.  ``promoted``: (K, V, the warm tier's
-        positions, their indices among them)."""
+        positions, their indices among them, what takes them out of the warm tier).  The tiers
+        change after the launch: a call that fails before leaves them as they were."""
         dev = k.device
         old = 0 if self._hot_keys is None else self._hot_keys.shape[2]
         new = k.shape[2]
@@ -507,6 +524,8 @@ class AKVLayer:
                 mv.fill(imp, old, 1.0, at=front)
             mv.fill(imp, new, 1.0, at=front + old)
         mv.run(None if promoted is None else promoted[3], front)
+        if promoted is not None:
+            promoted[4]()
         self._hot_keys, self._hot_values, self._hot_positions, self._importance = keys, values, pos, imp
         self._total_len += new
 
@@ -548,65 +567,75 @@ class AKVLayer:
         return out
 
     def _take_promoted(self, chosen: torch.Tensor, use_proxy: bool):
-        """akv/drop_in.py:433-484 / :543-589: the chosen warm tokens leave the packed tier;
-        returns what ``_append_hot`` puts in front of the hot tier, or None.  The count is the
-        one value an update waits for: the shapes that follow depend on it."""
+        """akv/drop_in.py:433-484 / :543-589: what ``_append_hot`` puts in front of the hot tier, or
+        None; its last entry takes the chosen warm tokens out of the packed tier.  The count is
+        the one value an update waits for: the shapes that follow depend on it."""
         n = int(chosen[0])
         if n == 0:
             return None
         idx = chosen[1:1 + n]
         warm_len = self._warm.n
         positions = self._warm.positions()
-        pk, pv, kept = self._warm.pull(idx, self._proxy_score if use_proxy else None)
-        if use_proxy:
-            self._proxy_score = kept
-        self._warm_bytes_packed = int(self._warm_bytes_packed * (max(0, warm_len - n) / warm_len))
-        self._warm_len -= n
-        return pk, pv, positions, idx
+        pk, pv, kept, take = self._warm.pull(idx, self._proxy_score if use_proxy else None)
+
+        def commit():
+            take()
+            if use_proxy:
+                self._proxy_score = kept
+            self._warm_bytes_packed = int(self._warm_bytes_packed * (max(0, warm_len - n) / warm_len))
+            self._warm_len -= n
+        return pk, pv, positions, idx, commit
 
     def _demote(self, n_demote: int, hot_len: int):
+        """The tiers change once everything is allocated and launched: a call that fails before
+        leaves the tokens in the hot tier, over its budget until the next one."""
         hk, hv = self._hot_keys, self._hot_values
         dev = hk.device
         B, H, _, D = hk.shape
         idx = select_demote_indices(self._importance, n_demote, hot_len, self.hot_budget, device=dev)
         mv = RowMoves()  # the event's rows into the packed tier, the kept ones of the hot tier
+        warm = self._warm
         if self.per_head_bits and len(self.per_head_bits) == H:
-            if self._warm is None:
-                self._warm = _HeadBitsTier(B, H, D, self.per_head_bits, dev)
-            self._warm_bytes_packed += self._warm.demote(hk, hv, idx, self.outlier_fraction, self._hot_positions)
+            if warm is None:
+                warm = _HeadBitsTier(B, H, D, self.per_head_bits, dev)
+            packed, take = warm.demote(hk, hv, idx, self.outlier_fraction, self._hot_positions)
         else:
             w = quantize_kv(hk, hv, self.warm_key_bits, self.warm_value_bits, block_t=max(n_demote, 1), group_v=D,
                             outlier_fraction=self.outlier_fraction, sel=idx.unsqueeze(0).expand(B, n_demote))
-            if self._warm is None:
-                self._warm = _EventTier(B, H, D, self.warm_key_bits, self.warm_value_bits, w.n_out, dev, n_demote)
-            self._warm.append(w, self._hot_positions, mv)
+            if warm is None:
+                warm = _EventTier(B, H, D, self.warm_key_bits, self.warm_value_bits, w.n_out, dev, n_demote)
+            take = warm.append(w, self._hot_positions, mv)
             # measure_packed_bytes per batch element: packed codes + fp16 scale and zero, K and V
-            self._warm_bytes_packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
-                                        + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
-        self._warm_len += n_demote
-        if self._proxy_score is not None:  # new warm tokens start with no evidence
-            old = self._proxy_score
-            self._proxy_score = torch.empty(old.shape[0] + n_demote, dtype=torch.float32, device=dev)
-            mv.copy(self._proxy_score, old, old.shape[0])
-            mv.fill(self._proxy_score, n_demote, 0.0, at=old.shape[0])
+            packed = (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
+                      + w.v_codes.nbytes + w.v_scale.nbytes + w.v_zero.nbytes)
+        proxy = self._proxy_score
+        if proxy is not None:  # new warm tokens start with no evidence
+            old = proxy.shape[0]
+            proxy = torch.empty(old + n_demote, dtype=torch.float32, device=dev)
+            mv.copy(proxy, self._proxy_score, old)
+            mv.fill(proxy, n_demote, 0.0, at=old)
         kept = hot_len - n_demote
-        pos, imp = self._hot_positions, self._importance
-        self._hot_positions = torch.empty(kept, dtype=torch.int64, device=dev)
-        self._importance = torch.empty(kept, dtype=torch.float32, device=dev)
-        mv.copy(self._hot_positions, pos, kept, KEEP)
-        mv.copy(self._importance, imp, kept, KEEP)
+        pos = torch.empty(kept, dtype=torch.int64, device=dev)
+        imp = torch.empty(kept, dtype=torch.float32, device=dev)
+        mv.copy(pos, self._hot_positions, kept, KEEP)
+        mv.copy(imp, self._importance, kept, KEEP)
         if movable(hk.dtype, hk) and movable(hv.dtype, hv):
             tiers = []
             for x in (hk, hv):
                 x = x if x.stride(3) == 1 or D <= 1 else x.contiguous()
                 tiers.append(torch.empty(B, H, kept, D, dtype=x.dtype, device=dev))
                 mv.copy(tiers[-1], x, kept, KEEP)
-            self._hot_keys, self._hot_values = tiers
         else:
             keep = torch.ones(hot_len, dtype=torch.bool, device=dev)
             keep[idx] = False
-            self._hot_keys, self._hot_values = hk[:, :, keep], hv[:, :, keep]
+            tiers = [hk[:, :, keep], hv[:, :, keep]]
         mv.run(idx, n_demote)
+        take()
+        self._warm, self._proxy_score = warm, proxy
+        self._warm_len += n_demote
+        self._warm_bytes_packed += packed
+        self._hot_keys, self._hot_values = tiers
+        self._hot_positions, self._importance = pos, imp
 
     def update(self, key_states: torch.Tensor, value_states: torch.Tensor,
                cache_kwargs: Optional[dict] = None) -> tuple[torch.Tensor, torch.Tensor]:
@@ -668,14 +697,7 @@ class AKVLayer:
         their proxy scores, and the length becomes max_length."""
         if self._total_len <= max_length:
             return
-        if self._hot_keys is not None:
-            keep = self._hot_positions < max_length
-            if not bool(keep.all()):
-                self._hot_keys = self._hot_keys[:, :, keep]
-                self._hot_values = self._hot_values[:, :, keep]
-                self._hot_positions = self._hot_positions[keep]
-                if self._importance is not None and self._importance.shape[0] == keep.shape[0]:
-                    self._importance = self._importance[keep]
+        take = hot = None
         if self._warm is not None and self._warm.n:
             warm_len = self._warm.n
             drop = (self._warm.positions() >= max_length).nonzero().flatten()
@@ -683,11 +705,22 @@ class AKVLayer:
             if n_drop:
                 proxy = self._proxy_score
                 fits = proxy is not None and proxy.shape[0] == warm_len
-                kept = self._warm.remove(drop, n_drop, proxy if fits else None)
-                if fits:
-                    self._proxy_score = kept
-                self._warm_bytes_packed = int(self._warm_bytes_packed * ((warm_len - n_drop) / warm_len))
-                self._warm_len -= n_drop
+                kept, take = self._warm.remove(drop, n_drop, proxy if fits else None)
+        if self._hot_keys is not None:
+            keep = self._hot_positions < max_length
+            if not bool(keep.all()):
+                imp = self._importance
+                if imp is not None and imp.shape[0] == keep.shape[0]:
+                    imp = imp[keep]
+                hot = self._hot_keys[:, :, keep], self._hot_values[:, :, keep], self._hot_positions[keep], imp
+        if take is not None:
+            take()
+            if fits:
+                self._proxy_score = kept
+            self._warm_bytes_packed = int(self._warm_bytes_packed * ((warm_len - n_drop) / warm_len))
+            self._warm_len -= n_drop
+        if hot is not None:
+            self._hot_keys, self._hot_values, self._hot_positions, self._importance = hot
         self._total_len = max_length
 
     def warm_view(self) -> tuple[Optional[torch.Tensor], Optional[torch.Tensor]]:

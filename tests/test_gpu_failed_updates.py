@@ -98,3 +98,77 @@ def test_kivi_refused_launch(monkeypatch):
     assert caches[1]._quant_keys[0].n == 74 and caches[1]._residual_keys[0].shape[2] == 21
     for a, b in zip(caches[0].update(*chunks[2], 0), caches[1].update(*chunks[2], 0)):
         assert torch.equal(a, b)
+
+
+def _whole(layer, seen, k):
+    """Every token is in one tier once, at its position, and the views hold the tokens."""
+    total = layer.get_seq_length()
+    pos = [layer._hot_positions] + ([layer._warm_positions] if layer._warm is not None else [])
+    pos = torch.cat(pos).sort().values
+    assert torch.equal(pos, torch.arange(total, device="cuda")), k
+    n_warm = total - layer._hot_keys.shape[2]
+    assert layer._warm_len == n_warm and layer._importance.shape[0] == layer._hot_keys.shape[2], k
+    assert bool(torch.isfinite(layer._importance).all()), k
+    if layer._proxy_score is not None:
+        assert layer._proxy_score.shape[0] <= n_warm and bool(torch.isfinite(layer._proxy_score).all()), k
+    for view, x in zip((layer.keys, layer.values), seen):
+        # 4 bits over a range of ~9, twice where a token was promoted and demoted again
+        assert float((view - x).abs().max()) < 1.0, k
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(outlier_fraction=0.03), dict(per_head_bits=[4, 3, 4])])
+@pytest.mark.parametrize("lens,at", [((70, 9), 0), ((40, 50, 1), 1), ((120, 30, 1, 1), 2), ((90, 200, 1), 1)])
+def test_layer_update(kw, lens, at):
+    from akv.drop_in import AKVLayer
+    announce(f"failed layer update {kw} {lens} at {at}")
+    chunks = _chunks(lens, 2, 3, 64, torch.float16, 8)
+    k = 0
+    while True:
+        k += 1
+        layer = AKVLayer(warm_bits=4, hot_budget=64, promotion_threshold=0.02, **kw)
+        for c in chunks[:at]:
+            layer.update(*c)
+        taken = layer.get_seq_length()
+        with pytest.MonkeyPatch.context() as mp:
+            fail = _Failing(mp, k)
+            try:
+                layer.update(*chunks[at])
+            except torch.OutOfMemoryError:
+                pass
+        if not fail.hit:
+            break
+        if layer.get_seq_length() == taken:
+            layer.update(*chunks[at])
+        seen = [torch.cat([c[i] for c in chunks[:at + 1]], dim=2) for i in range(2)]
+        for c in chunks[at + 1:]:
+            seen = [torch.cat([s, x], dim=2) for s, x in zip(seen, c)]
+            layer.update(*c)
+        if len(chunks) > at + 1 or layer.keys.shape[2] == seen[0].shape[2]:
+            _whole(layer, seen, k)
+    assert k > 8
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(per_head_bits=[4, 3, 4])])
+def test_layer_crop(kw):
+    from akv.drop_in import AKVLayer
+    announce(f"failed crop {kw}")
+    chunks = _chunks((150, 1, 3), 1, 3, 64, torch.float16, 9)
+    k = 0
+    while True:
+        k += 1
+        layer = AKVLayer(warm_bits=4, hot_budget=64, **kw)
+        for c in chunks[:2]:
+            layer.update(*c)
+        with pytest.MonkeyPatch.context() as mp:
+            fail = _Failing(mp, k)
+            try:
+                layer.crop(60)
+            except torch.OutOfMemoryError:
+                assert layer.get_seq_length() == 151
+                assert layer._hot_keys.shape[2] + layer._warm_len == 151
+        layer.crop(60)
+        layer.update(*chunks[2])
+        _whole(layer, [torch.cat([chunks[0][i][:, :, :60], chunks[2][i]], dim=2) for i in range(2)], k)
+        if not fail.hit:
+            break
+    assert k > 4  # the packed tier loses tokens too
