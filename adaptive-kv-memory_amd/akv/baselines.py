@@ -39,7 +39,7 @@ import torch
 
 from . import _native as nat
 from ._legacy import legacy_desc, padded_dim
-from .row_moves import RowMoves, movable
+from .row_moves import RowMoves, row_moves
 
 
 @dataclass
@@ -157,7 +157,7 @@ class _Tier:
         cap = max(64, self.cap)
         while cap < self.n + n:
             cap *= 2
-        mv, grown = RowMoves(), {}
+        mv, grown = row_moves(), {}
         for name, width, dtype in (("codes", self.row_bytes, torch.uint8), ("sc", self.G, torch.float32),
                                    ("ze", self.G, torch.float32), ("sc16", self.G, torch.float16),
                                    ("ze16", self.G, torch.float16)):
@@ -305,7 +305,7 @@ class KIVIFusedCache(KIVICache):
         res = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
         for bits, r in ((cfg.key_bits, res[0]), (cfg.value_bits, res[1])):
             _check_shape(r.shape[3], bits, cfg.group_size)
-        sides, args, mv = [], [], RowMoves()
+        sides, args, mv = [], [], row_moves()
         for bits, tiers, r in ((cfg.key_bits, self._quant_keys, res[0]), (cfg.value_bits, self._quant_values, res[1])):
             B, H, n_all, D = r.shape
             n = n_all - cfg.residual_length
@@ -319,9 +319,9 @@ class KIVIFusedCache(KIVICache):
                 x = nat.dev_contig(x)
             dt = torch.promote_types(torch.float16, left.dtype)
             view = old = None
-            if movable(dt, left) and dt in (torch.float16, torch.float32):
+            if mv.takes(dt, left) and dt in (torch.float16, torch.float32):
                 view, old = self._new_view(tier, tier.n, n, left, dt, mv)
-            if movable(left.dtype, left) and left.stride(3) == 1:
+            if mv.takes(left.dtype, left) and left.stride(3) == 1:
                 kept = torch.empty(left.shape, dtype=left.dtype, device=left.device)
                 mv.copy(kept, left, left.shape[2])
             else:
@@ -376,10 +376,10 @@ class KIVIFusedCache(KIVICache):
         rs = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
         if layer_idx not in self._dequant_keys_cache:
             return rs
-        mv, out = RowMoves(), []
+        mv, out = row_moves(), []
         for tier, r in zip((self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx]), rs):
             dt = torch.promote_types(torch.float16, r.dtype)
-            if not movable(dt, r) or r.shape[:2] != (tier.B, tier.H) or r.shape[3] != tier.D:
+            if not mv.takes(dt, r) or r.shape[:2] != (tier.B, tier.H) or r.shape[3] != tier.D:
                 out.append(torch.cat([tier.dequantize(), r], dim=2))
                 continue
             view, old = self._new_view(tier, tier.n, 0, r, dt, mv)

@@ -20,7 +20,7 @@ from typing import Optional
 import torch
 
 from . import _native as nat
-from .row_moves import GATHER, KEEP, SCATTER, RowMoves, movable
+from .row_moves import GATHER, KEEP, SCATTER, RowMoves, row_moves
 from .warm_tier import WarmTier, packed_row_bytes, quantize_kv
 
 _PRESETS = {
@@ -172,7 +172,7 @@ class _EventTier:
 
     def _grow(self, cap, ecap):
         t = self._alloc(cap, ecap)
-        mv = RowMoves()
+        mv = row_moves()
         for name, old in self.t.items():
             mv.copy(self._rows4(name, t[name]), self._rows4(name, old),
                     self.n if name in self._TOKEN_AXIS else self.n_events)
@@ -258,7 +258,7 @@ class _EventTier:
         sub = _EventTier.__new__(_EventTier)
         sub.__dict__.update({k: v for k, v in self.__dict__.items() if k != "t"})
         sub.t = {}
-        mv = RowMoves()
+        mv = row_moves()
         for name, x in self.t.items():
             if name in self._TOKEN_AXIS:
                 shape = list(x.shape)
@@ -281,7 +281,7 @@ class _EventTier:
         them out of the tier.  The kept rows go to fresh tensors: rows shift by up to n, so a
         move in place would race.  ``mv``: jobs on the same list that go with the launch."""
         kept = self.n - n
-        mv = mv or RowMoves()
+        mv = mv or row_moves()
         fresh = {name: torch.empty_like(self.t[name]) for name in self._TOKEN_AXIS if name in self.t}
         for name, x in fresh.items():
             mv.copy(x, self.t[name], kept, KEEP)
@@ -333,7 +333,7 @@ class _HeadBitsTier:
             w = quantize_kv(k, v, bits, bits, block_t=max(n, 1), group_v=D, outlier_fraction=outlier_fraction)
             if tier is None:
                 tier = _EventTier(B * hs, 1, D, bits, bits, w.n_out, self.dev, n)
-            mv = RowMoves()
+            mv = row_moves()
             staged.append((tier, tier.append(w, positions, mv)))
             mv.run(idx, n)
             packed += (w.k_codes.nbytes + w.k_scale.nbytes + w.k_zero.nbytes
@@ -482,7 +482,7 @@ class AKVLayer:
         first, dt = parts[0], parts[0].dtype
         for x in parts[1:]:
             dt = torch.promote_types(dt, x.dtype)
-        if not movable(dt, *parts) or any(x.dim() != 4 or x.device != first.device or x.shape[:2] != first.shape[:2]
+        if not mv.takes(dt, *parts) or any(x.dim() != 4 or x.device != first.device or x.shape[:2] != first.shape[:2]
                                           or x.shape[3] != first.shape[3] for x in parts):
             return torch.cat(parts, dim=2)
         out = torch.empty(first.shape[0], first.shape[1], sum(x.shape[2] for x in parts), first.shape[3], dtype=dt,
@@ -504,7 +504,7 @@ class AKVLayer:
         old = 0 if self._hot_keys is None else self._hot_keys.shape[2]
         new = k.shape[2]
         front = 0 if promoted is None else promoted[0].shape[2]
-        mv = RowMoves()
+        mv = row_moves()
         parts_k = ([] if promoted is None else [promoted[0]]) + ([] if self._hot_keys is None else [self._hot_keys]) + [k]
         parts_v = ([] if promoted is None else [promoted[1]]) + ([] if self._hot_keys is None else [self._hot_values]) + [v]
         keys, values = self._join(mv, parts_k), self._join(mv, parts_v)
@@ -593,7 +593,7 @@ class AKVLayer:
         dev = hk.device
         B, H, _, D = hk.shape
         idx = select_demote_indices(self._importance, n_demote, hot_len, self.hot_budget, device=dev)
-        mv = RowMoves()  # the event's rows into the packed tier, the kept ones of the hot tier
+        mv = row_moves()  # the event's rows into the packed tier, the kept ones of the hot tier
         warm = self._warm
         if self.per_head_bits and len(self.per_head_bits) == H:
             if warm is None:
@@ -619,7 +619,7 @@ class AKVLayer:
         imp = torch.empty(kept, dtype=torch.float32, device=dev)
         mv.copy(pos, self._hot_positions, kept, KEEP)
         mv.copy(imp, self._importance, kept, KEEP)
-        if movable(hk.dtype, hk) and movable(hv.dtype, hv):
+        if mv.takes(hk.dtype, hk) and mv.takes(hv.dtype, hv):
             tiers = []
             for x in (hk, hv):
                 x = x if x.stride(3) == 1 or D <= 1 else x.contiguous()
@@ -680,8 +680,8 @@ class AKVLayer:
         fv = torch.empty_like(fk)
         self._warm.dequantize_into(fk, fv)
         hp = self._hot_positions
-        if movable(out_dt, hk) and movable(out_dt, hv):
-            mv = RowMoves()
+        mv = row_moves()
+        if mv.takes(out_dt, hk, hv):
             mv.copy(fk, hk, hk.shape[2], SCATTER)
             mv.copy(fv, hv, hv.shape[2], SCATTER)
             mv.run(hp, hp.shape[0])

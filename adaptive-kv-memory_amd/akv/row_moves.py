@@ -12,12 +12,27 @@ from typing import Optional
 
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 from . import _native as nat
 
 SAME, KEEP, GATHER, SCATTER = range(4)
 _COPY, _WIDEN, _FILL, _COUNT = range(4)
 _FLOATS = (torch.float16, torch.bfloat16, torch.float32)
+
+
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_jit_tracing, _function_mode, _compiling = torch._C._is_tracing, torch._C._get_function_stack_at, torch.compiler.is_compiling
+
+
+def observed() -> bool:
+    """Whether something has to see the operations themselves: a dispatch or function mode (a
+    trace, fake tensors, a logger; torch's default-device context is none of these), torch.jit
+    tracing or compilation."""
+    if _compiling() or _dispatch_modes() or _jit_tracing():
+        return True
+    n = _function_modes()
+    return n != 0 and any(type(_function_mode(i)) is not DeviceContext for i in range(n))
 
 
 def movable(out_dtype: torch.dtype, *tensors: torch.Tensor) -> bool:
@@ -38,6 +53,8 @@ assert _JOB.size == ctypes.sizeof(nat.RowsJob)
 
 
 class RowMoves:
+    takes = staticmethod(movable)
+
     def __init__(self):
         self._jobs = []
         self._hold = []
@@ -109,3 +126,52 @@ class RowMoves:
         nat.check(nat.load().akv_rows_move(jobs, len(self._jobs), idx.data_ptr() if n_idx else None, n_idx,
                                            nat.stream_of(self._hold[0][1])), "row moves")
         self._jobs, self._hold = [], []
+
+
+class _TorchMoves:
+    """The same jobs as torch's own operations, one after another."""
+
+    def __init__(self):
+        self._jobs = []
+
+    def takes(self, out_dtype: torch.dtype, *tensors: torch.Tensor) -> bool:
+        return False
+
+    def copy(self, dst, src, n, rows=SAME, at=0, value=1.0):
+        self._jobs.append((self._copy, dst, src, n, rows, at, value))
+
+    def fill(self, dst, n, value, at=0):
+        self._jobs.append((lambda idx, part: part.fill_(value), dst.narrow(0, at, n)))
+
+    def count(self, dst, n, start, step=1, at=0):
+        self._jobs.append((lambda idx, part: part.copy_(
+            torch.arange(n, dtype=part.dtype, device=part.device) * step + start), dst.narrow(0, at, n)))
+
+    def run(self, idx=None, n_idx=0):
+        for job, *args in self._jobs:
+            job(None if idx is None else idx[:n_idx], *args)
+        self._jobs = []
+
+    @staticmethod
+    def _copy(idx, dst, src, n, rows, at, value):
+        ax = 0 if src.dim() == 1 else 2
+        if rows == KEEP:
+            mask = torch.ones(src.shape[ax], dtype=torch.bool, device=src.device)
+            if idx is not None:
+                mask[idx] = False
+            src = src.index_select(ax, mask.nonzero().flatten()[:n])
+        elif rows == GATHER:
+            src = src.index_select(ax, idx[:n])
+        else:
+            src = src.narrow(ax, 0, n)
+        if value != 1.0:
+            src = src.float() * value
+        if rows == SCATTER:
+            dst.index_copy_(ax, idx[:n], src.to(dst.dtype))
+        else:
+            dst.narrow(ax, at, n).copy_(src)
+
+
+def row_moves():
+    """A collector of row moves, by torch's own operations where somebody looks on."""
+    return _TorchMoves() if observed() else RowMoves()
