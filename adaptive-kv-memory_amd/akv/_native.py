@@ -146,6 +146,7 @@ EXPORTS = (
     "akv_abi_version", "akv_last_error", "akv_struct_size",
     "akv_decode_workspace_bytes", "akv_decode_counter_bytes", "akv_decode_attn", "akv_decode_attn_noalloc",
     "akv_quant_pack", "akv_quant_workspace_bytes", "akv_quant_pack_ws", "akv_dequant_unpack",
+    "akv_dequant_unpack_rows",
     "akv_bitpack", "akv_bitunpack", "akv_importance_update",
     "akv_importance_workspace_bytes", "akv_importance_update_ws",
     "akv_prefill_workspace_bytes", "akv_prefill_attn", "akv_select_demote", "akv_stream_read",
@@ -187,6 +188,8 @@ def load() -> ctypes.CDLL:
     lib.akv_quant_pack_ws.argtypes = [ctypes.POINTER(QuantArgs), _vp, _i64, _vp]
     lib.akv_dequant_unpack.restype = ctypes.c_int
     lib.akv_dequant_unpack.argtypes = [ctypes.POINTER(DequantArgs), _vp]
+    lib.akv_dequant_unpack_rows.restype = ctypes.c_int
+    lib.akv_dequant_unpack_rows.argtypes = [ctypes.POINTER(DequantArgs), _i64, _vp]
     lib.akv_bitpack.restype = ctypes.c_int
     lib.akv_bitpack.argtypes = [_vp, _vp, _i64, _i32, _i32, _vp]
     lib.akv_bitunpack.restype = ctypes.c_int

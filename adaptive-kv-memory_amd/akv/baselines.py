@@ -114,8 +114,7 @@ def dequantize_rows(codes: torch.Tensor, sc: torch.Tensor, ze: torch.Tensor, bit
     a.out_dtype = nat.DT_F16
     a.warm = desc
     a.k_out = out.data_ptr()
-    a.out_tokens = out.shape[1]
-    nat.check(nat.load().akv_dequant_unpack(ctypes.byref(a), nat.stream_of(out)), "KIVI dequantize")
+    nat.check(nat.load().akv_dequant_unpack_rows(ctypes.byref(a), out.shape[1], nat.stream_of(out)), "KIVI dequantize")
     return out
 
 

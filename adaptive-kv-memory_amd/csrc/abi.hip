@@ -617,7 +617,12 @@ int akv_quant_pack_ws(const akv_quant_args *a, void *workspace, int64_t workspac
 
 int akv_quant_pack(const akv_quant_args *a, void *stream) { return akv_quant_pack_ws(a, nullptr, 0, stream); }
 
-int akv_dequant_unpack(const akv_dequant_args *a, void *stream) {
+}  // extern "C"
+
+namespace {
+
+// out_rows: output token rows per head, or 0: as many as tokens (or, with slots, out_tokens)
+int dequant_run(const akv_dequant_args *a, int64_t out_rows, void *stream) {
     if (!a) return fail(AKV_E_INVALID, "args is NULL");
     if (a->abi_version != AKV_ABI_VERSION) return fail(AKV_E_ABI, "ABI mismatch");
     const akv_warm_desc &w = a->warm;
@@ -637,9 +642,7 @@ int akv_dequant_unpack(const akv_dequant_args *a, void *stream) {
     if (a->out_slot && a->out_tokens < 1) return fail(AKV_E_SHAPE, "out_slot needs out_tokens >= 1");
     p.tok_stride = w.token_stride > 0 ? w.token_stride : w.n_warm;
     p.out_slot = a->out_slot;
-    const bool strided = w.kind == AKV_WARM_LEGACY && a->out_tokens != 0;
-    if (strided && a->out_tokens < w.n_warm) return fail(AKV_E_SHAPE, "out_tokens < n_warm");
-    p.out_tokens = a->out_slot || strided ? a->out_tokens : w.n_warm;
+    p.out_tokens = a->out_slot ? a->out_tokens : out_rows > 0 ? out_rows : w.n_warm;
     if (w.kind == AKV_WARM_AFFINE) {
         for (int bits : {w.bits_k, w.bits_v})
             if ((bits < 2 || bits > 4) && bits != 8) return fail(AKV_E_BITS, "Unsupported bits: %d", bits);
@@ -682,6 +685,19 @@ int akv_dequant_unpack(const akv_dequant_args *a, void *stream) {
     hipError_t e = akv::dequant_launch(p, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "dequant launch");
     return ok();
+}
+
+}  // namespace
+
+extern "C" {
+
+int akv_dequant_unpack(const akv_dequant_args *a, void *stream) { return dequant_run(a, 0, stream); }
+
+int akv_dequant_unpack_rows(const akv_dequant_args *a, int64_t out_rows, void *stream) {
+    if (!a) return fail(AKV_E_INVALID, "args is NULL");
+    if (a->out_slot) return fail(AKV_E_INVALID, "output slots say their rows in out_tokens");
+    if (out_rows < 1 || out_rows < a->warm.n_warm) return fail(AKV_E_SHAPE, "out_rows < n_warm");
+    return dequant_run(a, out_rows, stream);
 }
 
 int akv_bitpack(const void *codes, void *packed, int64_t rows, int32_t dim, int32_t bits, void *stream) {

@@ -237,7 +237,7 @@ typedef struct akv_dequant_args {
                                       batch element when block_of_token is given */
     const int64_t *out_slot;       /* [Nw] output token row of each warm token: the outputs are then
                                       [B][Hkv][out_tokens][D] and other rows are not written */
-    int64_t out_tokens;            /* with out_slot, or LEGACY: output token rows per head (LEGACY 0: Nw) */
+    int64_t out_tokens;            /* with out_slot only */
 } akv_dequant_args;
 
 /* Unpack + dequantize a warm tier to dense values, bit-exact with
@@ -250,6 +250,9 @@ typedef struct akv_dequant_args {
  * (akv/drop_in.py:762-787).  AFFINE outputs are float16, or float32 holding the
  * float16 values (the reference's cat with float32 / bfloat16 hot tokens). */
 int akv_dequant_unpack(const akv_dequant_args *args, void *stream);
+/* The same into outputs of out_rows >= n_warm token rows per head, of which the first n_warm are
+ * written (no out_slot). */
+int akv_dequant_unpack_rows(const akv_dequant_args *args, int64_t out_rows, void *stream);
 
 /* -------------------------------------------------------------- bitpack */
 
