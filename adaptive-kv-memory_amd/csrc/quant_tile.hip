@@ -745,7 +745,12 @@ __global__ __launch_bounds__(128) void outlier_rank_kernel(const QuantParams p) 
 
 // ------------------------------------------------------------- host side
 
+// The tensors of the batch elements are the grid's last dimension: past its limit the call stays
+// with quant_kernel, whose last dimension is the batch alone.
+constexpr int64_t kGridYZ = 65535;
+
 bool quant_tile_eligible(const QuantParams &p) {
+    if ((int64_t)p.B * ((p.k != nullptr) + (p.v != nullptr)) > kGridYZ) return false;
     const uintptr_t al = (uintptr_t)p.k | (uintptr_t)p.v | (uintptr_t)p.k_codes | (uintptr_t)p.v_codes;
     const uintptr_t meta = p.k_mode == 0 ? (uintptr_t)p.k_scale | (uintptr_t)p.k_zero : 0;
     return ((al | meta) & 15u) == 0 && p.ar_dt == p.in_dt && !p.symmetric;
@@ -763,10 +768,9 @@ int quant_stat_chunks(const QuantParams &p, int *tokens) {
     return (int)((T + ct - 1) / ct);
 }
 
-
-// Outlier norms go through the workspace for blocks longer than kLongT.
+// Outlier norms go through the workspace for blocks longer than kLongT (a grid row each).
 bool quant_norms_in_ws(const QuantParams &p) {
-    return p.n_out > 0 && p.T > kLongT && p.n_sel > kLongT && (p.k || p.v);
+    return p.n_out > 0 && p.T > kLongT && p.n_sel > kLongT && p.nblk <= kGridYZ && (p.k || p.v);
 }
 
 template <int IN, int D>
