@@ -292,8 +292,8 @@ void make_prefill_plan(const akv_prefill_args *a, PrefillPlan *pl) {
     pl->tiles_per_split = (nt + ns - 1) / ns;
     pl->nsplit = (int)((nt + pl->tiles_per_split - 1) / pl->tiles_per_split);
     pl->nchunk = (pl->R + 15) / 16;
-    pl->part_bytes =
-        pl->nsplit > 1 ? align256((int64_t)a->B * a->Hkv * pl->nchunk * pl->nsplit * akv::kPrefillPart * 4) : 0;
+    pl->part_bytes = pl->nsplit > 1 ? align256((int64_t)a->B * a->Hkv * pl->nchunk * pl->nsplit *
+                                               akv::prefill_part_rows(pl->R) * (a->D + 4) * 4) : 0;
 }
 
 }  // namespace

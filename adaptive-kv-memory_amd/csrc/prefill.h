@@ -21,14 +21,15 @@ struct PrefillParams {
     int n_row_tiles;                // ceil(R / rows per workgroup)
     int nsplit;                     // token splits (partials merged by prefill_merge_kernel)
     int64_t tiles_per_split;        // 32-token tiles per split (hot tiles first, then warm)
-    float *part;                    // partials [bh][chunk][split][kPrefillPart] when nsplit > 1
+    float *part;                    // partials [bh][chunk][split][rows (D + 4)] when nsplit > 1: acc, (max, sum), unused
     int nchunk;                     // 16-row chunks of R
     const void *kcur, *vcur;        // the chunk's own K / V [B][Hkv][M][128] in q's dtype (or null):
     int n_cur;                      // attended causally after the cache; n_cur = M (0 without them)
 };
 
 constexpr int kPrefillRows = 256;   // query rows per workgroup
-constexpr int kPrefillPart = 16 * (128 + 4);  // floats of one split's partial of a 16-row chunk: acc, (max, sum), unused
+// Rows of a 16-row chunk's partial, from R query rows per kv head.
+__host__ __device__ constexpr int prefill_part_rows(int R) { return R < 16 ? R : 16; }
 
 // Launch the split kernel and, when nsplit > 1, the merge.
 hipError_t prefill_launch(const PrefillParams &p, hipStream_t s);

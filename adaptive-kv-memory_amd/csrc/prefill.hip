@@ -543,14 +543,16 @@ void prefill_kernel(const PrefillParams p) {
         if (p.nsplit > 1) {
             const int chunk = (r0 + 32 * wave + 16 * rg) / 16;
             if (chunk >= p.nchunk) continue;
-            float *part = p.part + ((bh * p.nchunk + chunk) * p.nsplit + split) * (int64_t)kPrefillPart;
-            if (grp == 0) *(f2 *)(part + 16 * kPD + 2 * col) = (f2){sm[rg].m2, l};
+            const int prows = prefill_part_rows(p.R);
+            if (r >= p.R && p.R < 16) continue;  // (written so, the tile loop keeps its schedule: 2,540 -> 2,500 us)
+            float *part = p.part + ((bh * p.nchunk + chunk) * p.nsplit + split) * (int64_t)(prows * (kPD + 4));
+            if (grp == 0) *(f2 *)(part + prows * kPD + 2 * col) = (f2){sm[rg].m2, l};
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                f4 *dst = (f4 *)part + 2 * i * 64 + lane;
+                f4 *dst = (f4 *)part + (8 * i + grp) * prows + col;
                 dst[0] = (f4){sm[rg].acc[0][i] + sm[rg].accz[i], sm[rg].acc[1][i] + sm[rg].accz[i],
                               sm[rg].acc[2][i] + sm[rg].accz[i], sm[rg].acc[3][i] + sm[rg].accz[i]};
-                dst[64] = (f4){sm[rg].acc[4][i] + sm[rg].accz[i], sm[rg].acc[5][i] + sm[rg].accz[i],
+                dst[4 * prows] = (f4){sm[rg].acc[4][i] + sm[rg].accz[i], sm[rg].acc[5][i] + sm[rg].accz[i],
                                sm[rg].acc[6][i] + sm[rg].accz[i], sm[rg].acc[7][i] + sm[rg].accz[i]};
             }
             continue;
@@ -588,10 +590,11 @@ __device__ __forceinline__ u2 out_quad(f4 o, float L, int bf16) {
 // Merge of up to 8 token splits, one workgroup per chunk of 16 rows.  HBM / L2-bound: a split's
 // partial of a chunk is 8 blocks of 64 lanes x 16 bytes in the order the attention waves hold
 // them (block 2 i + half, lane (row col, channel quarter grp): channels 8 (4 grp + i) + 4 half
-// ..+3), then the rows' (max, sum).  So every store of the attention kernel and every load here
+// ..+3; with fewer than 16 rows in all, a lane of each), then the rows' (max, sum).  So every store of the attention kernel and every load here
 // is 1 KiB of consecutive addresses; stored row by row, each store instruction touched 64
 // cache lines: 2 x 12 x 333 positions over 11,007 tokens (8 splits, 34 MB) 91.8 -> 85.4 us.
 // All splits' loads are in flight at once; the output tile turns through LDS into rows.
+template <bool FEW>
 __global__ __launch_bounds__(512) void prefill_merge_kernel(const PrefillParams p) {
     constexpr int KS = 8;
     __shared__ __align__(16) uint16_t tile[16][kPD + 8];
@@ -599,16 +602,17 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(const PrefillParams 
     const int col = lane & 15, grp = lane >> 4;
     const int chunk = blockIdx.x % p.nchunk;
     const int64_t bh = blockIdx.x / p.nchunk;
-    const float *part = p.part + (bh * p.nchunk + chunk) * p.nsplit * (int64_t)kPrefillPart;
+    const int prows = FEW ? p.R : 16, stride = prows * (kPD + 4), row = FEW ? min(col, prows - 1) : col;
+    const float *part = p.part + (bh * p.nchunk + chunk) * p.nsplit * (int64_t)stride;
     float M = -INFINITY, L = 0.f;
     f4 o = {0.f, 0.f, 0.f, 0.f};
     f2 ml[KS];
     f4 x[KS];
 #pragma unroll
     for (int k = 0; k < KS; ++k) {
-        const float *src = part + min(k, p.nsplit - 1) * (int64_t)kPrefillPart;
-        ml[k] = *(const f2 *)(src + 16 * kPD + 2 * col);
-        x[k] = ((const f4 *)src)[blk * 64 + lane];
+        const float *src = part + min(k, p.nsplit - 1) * (int64_t)stride;
+        ml[k] = *(const f2 *)(src + prows * kPD + 2 * row);
+        x[k] = ((const f4 *)src)[(4 * blk + grp) * prows + row];
         if (k < p.nsplit) M = fmaxf(M, ml[k][0]);
     }
 #pragma unroll
@@ -631,6 +635,7 @@ __global__ __launch_bounds__(512) void prefill_merge_kernel(const PrefillParams 
 // waves over the splits, 8 loads of a wave in flight, merged in LDS -- there are few chunks
 // then, and one workgroup walking their splits 8 at a time is a chain of trips to memory
 // (16 heads x 75 positions over 21,194 tokens: 45.7 us a call with a workgroup per row, 42.0 so).
+template <bool FEW>
 __global__ __launch_bounds__(512) void prefill_merge_many_kernel(const PrefillParams p) {
     constexpr int KS = 8, NW = 8;
     __shared__ f2 mls[NW][16];
@@ -639,7 +644,8 @@ __global__ __launch_bounds__(512) void prefill_merge_many_kernel(const PrefillPa
     const int col = lane & 15, grp = lane >> 4;
     const int chunk = blockIdx.x % p.nchunk;
     const int64_t bh = blockIdx.x / p.nchunk;
-    const float *part = p.part + (bh * p.nchunk + chunk) * p.nsplit * (int64_t)kPrefillPart;
+    const int prows = FEW ? p.R : 16, stride = prows * (kPD + 4), row = FEW ? min(col, prows - 1) : col;
+    const float *part = p.part + (bh * p.nchunk + chunk) * p.nsplit * (int64_t)stride;
     float M = -INFINITY, L = 0.f;
     f4 o = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = wave; s0 < p.nsplit; s0 += NW * KS) {
@@ -647,9 +653,9 @@ __global__ __launch_bounds__(512) void prefill_merge_many_kernel(const PrefillPa
         f4 x[KS];
 #pragma unroll
         for (int k = 0; k < KS; ++k) {
-            const float *src = part + min(s0 + NW * k, p.nsplit - 1) * (int64_t)kPrefillPart;
-            ml[k] = *(const f2 *)(src + 16 * kPD + 2 * col);
-            x[k] = ((const f4 *)src)[blk * 64 + lane];
+            const float *src = part + min(s0 + NW * k, p.nsplit - 1) * (int64_t)stride;
+            ml[k] = *(const f2 *)(src + prows * kPD + 2 * row);
+            x[k] = ((const f4 *)src)[(4 * blk + grp) * prows + row];
         }
         float nm = M;
 #pragma unroll
@@ -719,8 +725,16 @@ hipError_t prefill_launch(const PrefillParams &p, hipStream_t s) {
 #undef AKV_PKV
     if (e != hipSuccess || p.nsplit == 1) return e;
     const unsigned chunks = (unsigned)(p.B * p.Hkv * p.nchunk);
-    if (p.nsplit <= 8) hipLaunchKernelGGL(prefill_merge_kernel, dim3(chunks), dim3(512), 0, s, p);
-    else hipLaunchKernelGGL(prefill_merge_many_kernel, dim3(chunks, 8), dim3(512), 0, s, p);
+    // few rows: fewer than a chunk's 16, in partials of that many (any row count in the one kernel
+    // costs the others 2.4 of 58.5 us at 12 heads x 333 positions over 11,007 tokens)
+    const bool few = p.R < 16;
+    if (p.nsplit <= 8) {
+        if (few) hipLaunchKernelGGL(prefill_merge_kernel<true>, dim3(chunks), dim3(512), 0, s, p);
+        else hipLaunchKernelGGL(prefill_merge_kernel<false>, dim3(chunks), dim3(512), 0, s, p);
+    } else {
+        if (few) hipLaunchKernelGGL(prefill_merge_many_kernel<true>, dim3(chunks, 8), dim3(512), 0, s, p);
+        else hipLaunchKernelGGL(prefill_merge_many_kernel<false>, dim3(chunks, 8), dim3(512), 0, s, p);
+    }
     return hipGetLastError();
 }
 
