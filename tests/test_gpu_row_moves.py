@@ -103,3 +103,33 @@ def test_update_keeps_autograd_and_refuses_other_shapes():
     with pytest.raises(RuntimeError):
         layer.update(*(_x((1, 3, 1, 64), torch.float16, i) for i in range(2)))
     assert n == (layer._warm.n, layer._hot_keys.shape[2], layer.get_seq_length())
+
+
+@pytest.mark.parametrize("T,n", [(3100, 1025), (3100, 2047), (3100, 2049), (20011, 1024), (20011, 4097), (20011, 15000), (20011, 20010)])
+@pytest.mark.parametrize("kind", ["random", "run", "ends", "every"])
+def test_keep_against_long_lists(T, n, kind):
+    """Lists past the 1024 samples of the kernel's first search: the second search sees 2 to 20
+    entries between two samples, in lists without any structure and with all of it."""
+    from akv.row_moves import KEEP, RowMoves
+    announce(f"row moves KEEP T={T} n={n} {kind}")
+    g = torch.Generator(device="cuda").manual_seed(T + n)
+    if kind == "random":
+        drop = torch.randperm(T, generator=g, device="cuda")[:n]
+    elif kind == "run":  # a prompt's oldest tokens
+        drop = torch.arange(n, device="cuda") + min(4, T - n)
+    elif kind == "ends":  # rows 0 and T - 1 among them
+        drop = torch.cat([torch.arange(n // 2, device="cuda"), torch.arange(T - (n - n // 2), T, device="cuda")])
+    else:
+        drop = torch.linspace(0, T - 1, n, device="cuda", dtype=torch.float64).round().long().unique()
+    drop = drop.sort().values
+    left = torch.ones(T, dtype=torch.bool, device="cuda")
+    left[drop] = False
+    nk = T - drop.numel()
+    x, pos = _x((2, 3, T, 24), torch.float16, n), torch.arange(T, device="cuda") * 7
+    a, b = torch.zeros(2, 3, nk + 1, 24, dtype=torch.float16, device="cuda"), torch.zeros(nk + 1, dtype=torch.int64, device="cuda")
+    mv = RowMoves()
+    mv.copy(a, x, nk, KEEP)
+    mv.copy(b, pos, nk, KEEP)
+    mv.run(drop, drop.numel())
+    assert torch.equal(a[:, :, :nk], x[:, :, left]) and not bool(a[:, :, nk].any())
+    assert torch.equal(b[:nk], pos[left]) and int(b[nk]) == 0
