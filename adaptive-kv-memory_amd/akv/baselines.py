@@ -119,34 +119,16 @@ def dequantize_rows(codes: torch.Tensor, sc: torch.Tensor, ze: torch.Tensor, bit
 
 
 class _Tier:
-    """One layer's quantized K or V: packed codes and fp32 (and, for the fused
+    """One layer's quantized K or V: packed codes and fp32 (and, for KIVIFusedCache's
     attention, fp16) scales / zeros per (batch * head, token), tokens in order."""
 
-    def __init__(self, B: int, H: int, D: int, bits: int, gs: int, device, keep_f16: bool):
+    def __init__(self, B: int, H: int, D: int, bits: int, gs: int, device):
         self.B, self.H, self.rows, self.D, self.bits, self.gs = B, H, B * H, D, bits, gs
         pD = padded_dim(D, gs)
         self.row_bytes, self.G = pD * bits // 8, pD // gs
-        self.n, self.cap, self.dirty, self.keep_f16 = 0, 0, 0, keep_f16
+        self.n, self.cap, self.dirty = 0, 0, 0
         self.device = device
         self.codes = self.sc = self.ze = self.sc16 = self.ze16 = None
-
-    def _grow(self, need: int):
-        cap = max(64, self.cap)
-        while cap < need:
-            cap *= 2
-        def grow(t, shape, dtype):
-            new = torch.zeros(shape, dtype=dtype, device=self.device)
-            if t is not None and self.n:
-                new[:, : self.n] = t[:, : self.n]
-            return new
-        R, G = self.rows, self.G
-        self.codes = grow(self.codes, (R, cap, self.row_bytes), torch.uint8)
-        self.sc = grow(self.sc, (R, cap, G), torch.float32)
-        self.ze = grow(self.ze, (R, cap, G), torch.float32)
-        if self.keep_f16:
-            self.sc16 = grow(self.sc16, (R, cap, G), torch.float16)
-            self.ze16 = grow(self.ze16, (R, cap, G), torch.float16)
-        self.cap = cap
 
     def reserve(self, n: int):
         """Room for n more rows.  Rows past the tier read as zeros: those of a grown tier, up to row
@@ -160,26 +142,18 @@ class _Tier:
         for name, width, dtype in (("codes", self.row_bytes, torch.uint8), ("sc", self.G, torch.float32),
                                    ("ze", self.G, torch.float32), ("sc16", self.G, torch.float16),
                                    ("ze16", self.G, torch.float16)):
-            if self.keep_f16 or not name.endswith("16"):
-                old, new = getattr(self, name), torch.empty(self.rows, cap, width, dtype=dtype, device=self.device)
-                if old is not None:
-                    mv.copy(new.unsqueeze(0), old.unsqueeze(0), self.n)
-                grown[name] = new
+            old, new = getattr(self, name), torch.empty(self.rows, cap, width, dtype=dtype, device=self.device)
+            if old is not None:
+                mv.copy(new.unsqueeze(0), old.unsqueeze(0), self.n)
+            grown[name] = new
         mv.run()
         self.__dict__.update(grown, cap=cap, dirty=cap)
 
-    def append(self, codes, sc, ze):
-        n = codes.shape[1]
-        if self.n + n > self.cap:
-            self._grow(self.n + n)
-        s = slice(self.n, self.n + n)
-        self.codes[:, s] = codes
-        self.sc[:, s] = sc
-        self.ze[:, s] = ze
-        if self.keep_f16:
-            self.sc16[:, s] = sc
-            self.ze16[:, s] = ze
-        self.n += n
+    def fill(self, codes, sc, ze):
+        """A tier that holds these tokens and no float16 meta (KIVICache makes one per overflow)."""
+        self.codes, self.sc, self.ze = codes, sc, ze
+        self.n = self.cap = codes.shape[1]
+        return self
 
     def __getitem__(self, key: str):
         """The reference's quant dict entries over the tier ('data', 'scales', 'zeros':
@@ -204,8 +178,6 @@ class _Tier:
 class KIVICache:
     """akv/baselines.py:249-403: every overflow re-quantizes the merged history and
     every update dequantizes the whole quantized tier."""
-
-    _keep_f16 = False
 
     def __init__(self, config: Optional[KIVIConfig] = None):
         self.config = config or KIVIConfig()
@@ -233,7 +205,7 @@ class KIVICache:
 
     def _new_tier(self, x: torch.Tensor, bits: int) -> "_Tier":
         B, H, _, D = x.shape
-        return _Tier(B, H, D, bits, self.config.group_size, x.device, self._keep_f16)
+        return _Tier(B, H, D, bits, self.config.group_size, x.device)
 
     def _quantize_overflow(self, layer_idx: int):
         """akv/baselines.py:291-322: quantize the overflow; merge by dequantizing the
@@ -245,9 +217,8 @@ class KIVICache:
         if layer_idx in self._quant_keys:
             tk = torch.cat([self._quant_keys[layer_idx].dequantize(), tk], dim=2)
             tv = torch.cat([self._quant_values[layer_idx].dequantize(), tv], dim=2)
-        kt, vt = self._new_tier(tk, cfg.key_bits), self._new_tier(tv, cfg.value_bits)
-        kt.append(*quantize_rows(tk, cfg.key_bits, cfg.group_size))
-        vt.append(*quantize_rows(tv, cfg.value_bits, cfg.group_size))
+        kt = self._new_tier(tk, cfg.key_bits).fill(*quantize_rows(tk, cfg.key_bits, cfg.group_size))
+        vt = self._new_tier(tv, cfg.value_bits).fill(*quantize_rows(tv, cfg.value_bits, cfg.group_size))
         self._quant_keys[layer_idx], self._quant_values[layer_idx] = kt, vt
         self._residual_keys[layer_idx] = res_k[:, :, n_q:].contiguous()
         self._residual_values[layer_idx] = res_v[:, :, n_q:].contiguous()
@@ -285,8 +256,6 @@ class KIVIFusedCache(KIVICache):
     """akv/baselines.py:426-510: incremental quantization of each overflow chunk.  The
     reference keeps a float16 working copy extended by that chunk's dequant; the same values
     come from the packed tier here, dequantized straight into each returned view."""
-
-    _keep_f16 = True
 
     def __init__(self, config: Optional[KIVIFusedConfig] = None):
         super().__init__(config or KIVIFusedConfig())
