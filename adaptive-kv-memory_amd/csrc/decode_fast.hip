@@ -113,7 +113,8 @@ constexpr int kNS = AKV_FAST_NS;        // ring slots per wave (deeper rings onl
 // block (the one-channel paths only: 163-168 VGPRs, so 12 waves with 2 slots
 // like OUT = 0); kMaxOut up to 4 channels, whose general corrections hold more
 // state per lane: 8 waves (2 per SIMD, twice the registers each) with 3 slots.
-// ODD: a head has an odd number of outlier values (odd length and count).
+// A negative OUT (-1, -kMaxOut) is the same for heads with an odd number of outlier values (odd
+// length and count).
 #ifndef AKV_FAST_WAVES_OUT
 #define AKV_FAST_WAVES_OUT 8
 #endif
@@ -121,7 +122,9 @@ constexpr int kNS = AKV_FAST_NS;        // ring slots per wave (deeper rings onl
 #define AKV_FAST_NS_OUT 3
 #endif
 constexpr int kWavesOut = AKV_FAST_WAVES_OUT, kNSOut = AKV_FAST_NS_OUT;
-template <int OUT> struct FastCfg {
+template <int OV> struct FastCfg {
+    static constexpr int OUT = OV < 0 ? -OV : OV;
+    static constexpr bool ODD = OV < 0;
     static constexpr int NW = OUT > 1 ? kWavesOut : kWaves, NS = OUT > 1 ? kNSOut : kNS;
 };
 constexpr int kLdsCap = 160 * 1024;  // LDS of one CU
@@ -288,11 +291,12 @@ __device__ __forceinline__ void wait_younger(int nw, int nh) {
     else wait_vm<0>();
 }
 
-template <int BK, int BV, int NG, int NS, int OUT, bool ODD, bool LEG>
-__global__ __launch_bounds__(64 * FastCfg<OUT>::NW)
-__attribute__((amdgpu_waves_per_eu(FastCfg<OUT>::NW / 4, FastCfg<OUT>::NW / 4)))
+template <int BK, int BV, int NG, int NS, int OV, bool LEG>
+__global__ __launch_bounds__(64 * FastCfg<OV>::NW)
+__attribute__((amdgpu_waves_per_eu(FastCfg<OV>::NW / 4, FastCfg<OV>::NW / 4)))
 void decode_fast_kernel(const DecodeParams p) {
-    constexpr int NW = FastCfg<OUT>::NW;  // waves of the workgroup
+    constexpr int OUT = FastCfg<OV>::OUT, NW = FastCfg<OV>::NW;  // waves of the workgroup
+    constexpr bool ODD = FastCfg<OV>::ODD;
     static_assert(NS >= 2 && NS <= 4, "ring depth");
     static_assert(!(LEG && OUT), "the legacy layout has no outlier channels");
     using L = WarmLayout<BK, BV, NG, OUT, LEG>;
@@ -1243,10 +1247,10 @@ bool decode_fast_eligible(const DecodeParams &p, int wk) {
     return p.slot_bytes > 0 && decode_fast_lds_bytes(p.slot_bytes, p.n_out) <= kLdsCap;
 }
 
-template <int BK, int BV, int NG, int NS, int OUT, bool ODD, bool LEG>
+template <int BK, int BV, int NG, int NS, int OV, bool LEG>
 static hipError_t launch_fast_ns(const DecodeParams &p, hipStream_t s) {
     const dim3 grid((unsigned)(p.nsplit * p.Hkv * p.B * p.nchunk));  // decoded in the kernel
-    const size_t lds = (size_t)decode_fast_lds_bytes(p.slot_bytes, OUT ? p.n_out : 0);
+    const size_t lds = (size_t)decode_fast_lds_bytes(p.slot_bytes, OV ? p.n_out : 0);
     // raise the dynamic LDS cap above 64 KiB once per device (a bit per device index;
     // host threads that race here both set it, which is harmless)
     static std::atomic<uint64_t> attr_devs{0};
@@ -1255,19 +1259,18 @@ static hipError_t launch_fast_ns(const DecodeParams &p, hipStream_t s) {
     if (e != hipSuccess) return e;
     const uint64_t bit = (dev >= 0 && dev < 64) ? 1ull << dev : 0ull;
     if (!bit || !(attr_devs.load(std::memory_order_acquire) & bit)) {
-        e = hipFuncSetAttribute((const void *)decode_fast_kernel<BK, BV, NG, NS, OUT, ODD, LEG>,
+        e = hipFuncSetAttribute((const void *)decode_fast_kernel<BK, BV, NG, NS, OV, LEG>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kLdsCap);
         if (e != hipSuccess) return e;
         attr_devs.fetch_or(bit, std::memory_order_release);
     }
-    hipLaunchKernelGGL((decode_fast_kernel<BK, BV, NG, NS, OUT, ODD, LEG>), grid, dim3(64 * FastCfg<OUT>::NW), lds, s,
-                       p);
+    hipLaunchKernelGGL((decode_fast_kernel<BK, BV, NG, NS, OV, LEG>), grid, dim3(64 * FastCfg<OV>::NW), lds, s, p);
     return hipGetLastError();
 }
 
 template <int BK, int BV, int NG, bool LEG>
 static hipError_t launch_fast(const DecodeParams &p, hipStream_t s) {
-    return launch_fast_ns<BK, BV, NG, kNS, 0, false, LEG>(p, s);
+    return launch_fast_ns<BK, BV, NG, kNS, 0, LEG>(p, s);
 }
 
 template <int BK, int BV, bool LEG>
@@ -1278,10 +1281,9 @@ static hipError_t launch_fast_ng(const DecodeParams &p, hipStream_t s) {
         const bool odd = p.n_warm & p.n_out & 1;
         if (p.Gv != 32) return hipErrorInvalidValue;
         if (p.n_out == 1)
-            return odd ? launch_fast_ns<BK, BV, 4, kNS, 1, true, false>(p, s)
-                       : launch_fast_ns<BK, BV, 4, kNS, 1, false, false>(p, s);
-        return odd ? launch_fast_ns<BK, BV, 4, kNSOut, kMaxOut, true, false>(p, s)
-                   : launch_fast_ns<BK, BV, 4, kNSOut, kMaxOut, false, false>(p, s);
+            return odd ? launch_fast_ns<BK, BV, 4, kNS, -1, false>(p, s) : launch_fast_ns<BK, BV, 4, kNS, 1, false>(p, s);
+        return odd ? launch_fast_ns<BK, BV, 4, kNSOut, -kMaxOut, false>(p, s)
+                   : launch_fast_ns<BK, BV, 4, kNSOut, kMaxOut, false>(p, s);
     }
     if (p.Gv == 32) return launch_fast<BK, BV, 4, LEG>(p, s);
     if (p.Gv == 64) return launch_fast<BK, BV, 2, LEG>(p, s);
