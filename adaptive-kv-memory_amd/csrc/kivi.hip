@@ -8,7 +8,7 @@
 // max by shuffles, and every thread dequantizes the codes it has just made from registers.
 // Before, each tensor went through a float32 copy, a quantize, five slice copies into the
 // zero-filled tier, a dequantize and a concatenation: 4,097 tokens x 32 heads of 128, K and V
-// at 2 bits, 226 -> 82 us an update (this launch 45 us, 3.3 TB/s; the divisions, one an
+// at 2 bits, 226 -> 61-67 us an update (this launch 43-46 us, 3.3 TB/s; the divisions, one an
 // element in the reference's arithmetic, cost about as much as the stores).
 #include "kivi.h"
 

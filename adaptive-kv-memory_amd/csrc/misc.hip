@@ -83,7 +83,7 @@ __global__ __launch_bounds__(256) void dequant_kernel(const DequantParams p) {
 // 16-byte stores; all its tokens' loads are in flight together.  HBM-bound: it writes what
 // the view holds and reads a fraction of that.  Before, each code, scale and zero was a load
 // of its own behind three 64-bit divisions per thread (dequant_kernel): 16,255 tokens x 8
-// heads of K and V at 3 bits 101 -> 32 us (2.5 TB/s, scattered to their positions); 3,969
+// heads of K and V at 3 bits 101 -> 28 us (2.9 TB/s, scattered to their positions); 3,969
 // tokens x 32 heads of legacy 2-bit rows 52 -> 12.8 us (2.9 TB/s).
 namespace {
 constexpr int kDqTok = 4;
@@ -486,7 +486,8 @@ __global__ __launch_bounds__(256) void importance_finish_kernel(const Importance
 // The radix select before it made four histogram passes over 64 slots whatever the row's
 // length, with one LDS address per lane: uniform scores, 1 x 140 45 -> 7.5 us, 1 x 2,049
 // 46 -> 9.0, 1 x 16,383 49 -> 19.7, 16 x 65,536 67 -> 53, 1 x 131,071 371 -> 150; equal
-// scores (a prompt's, all new) 1 x 16,383 87 -> 11.7 us.
+// scores (a prompt's, all new) 1 x 16,383 87 -> 11.7 us.  The promotion's form holds more state:
+// past 8,192 scores it spills (38 VGPRs at 32 slots, 50 at 64; the demotion's spills none).
 namespace {
 __device__ __forceinline__ uint32_t order_key(float f) {
     uint32_t u = __builtin_bit_cast(uint32_t, f);
@@ -863,7 +864,8 @@ hipError_t stream_read_launch(const void *p, int64_t bytes, uint32_t *sink, hipS
 // count up to 16) passes the one launch at 8 query rows without pooling (6.5-8.7 us; 11-15 at
 // 16, ~0.55 a row) and at ~12 (batch, head, query) rows with it (~0.3 us a row: 10.8 us at 32,
 // 20.5 at 64); but an eager call with a workspace and a second launch costs 12.2 us of host time
-// against 10.6, so the lines lie where the one launch takes longer than that.
+// against 10.6, so the lines lie where the one launch takes longer than that.  A captured call takes
+// the same lines, though only the device's time counts there.
 static int64_t importance_q_blocks(const ImportanceParams &p, int64_t *q_per) {
     const int64_t q = p.M - p.m0, kv = p.attn_dt == AKV_DT_F32 ? 4 : 8;
     if ((p.pool > 1 ? p.B * p.H * q < kImpMinPooledRows : q < kImpMinQueries) || p.N < kv || p.n_scores == 0) return 0;

@@ -9,8 +9,8 @@
 // over a lane's channels and then across the group's lanes; the packed rows leave
 // through LDS as contiguous stores.  What bounds the kernels at sizes that fill the GPU is
 // memory.  Measured against quant_kernel, which loads single elements and gives a block one
-// wave: one block of 16,255 float16 tokens x 8 heads 42.1 ms -> 18 us of statistics (1.8
-// TB/s) + 30 us of encoding; 3,969 float32 tokens x 32 heads in groups of 128 143 -> 26 us
+// wave: one block of 16,255 float16 tokens x 8 heads 42.1 ms -> 10 us of statistics (3.3
+// TB/s) + 29 us of encoding; 3,969 float32 tokens x 32 heads in groups of 128 143 -> 26 us
 // (2.7 TB/s); 32-token float16 blocks with one outlier channel, 15,872 tokens x 128 heads
 // 2.43 -> 0.35 ms, and their channel choice (outlier_select_kernel) 1.18 -> 0.21 ms.
 //

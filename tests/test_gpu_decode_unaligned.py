@@ -1,6 +1,7 @@
-"""The LDS-streamed decode on tiers whose meta rows and weight rows start off 16 bytes: token
-counts of every residue, one and two meta groups per token (block-affine V and the legacy
-layout), several (batch, kv-head)s, both tier orders, with weights and importance."""
+"""Decode over tiers whose meta rows, outlier values and weight rows start off 16 bytes: token
+counts of every residue, one, two and four meta groups per token (block-affine V and the legacy
+layout), one and three protected channels, several (batch, kv-head)s, both tier orders, with
+weights and importance."""
 import pytest
 import torch
 

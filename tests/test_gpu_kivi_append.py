@@ -1,4 +1,4 @@
-"""The one-pass KIVI overflow: tier, working copy and views equal to quantize_rows /
+"""The one-pass KIVI overflow: tier and views equal to quantize_rows /
 dequantize_rows on the same tokens, over dtypes, layouts, widths, group sizes past head_dim
 and chunk lengths around the workgroup's tokens: bit-exact."""
 import pytest
