@@ -273,10 +273,14 @@ class KIVIFusedCache(KIVICache):
         res = (self._residual_keys[layer_idx], self._residual_values[layer_idx])
         for bits, r in ((cfg.key_bits, res[0]), (cfg.value_bits, res[1])):
             _check_shape(r.shape[3], bits, cfg.group_size)
+        n = res[0].shape[2] - cfg.residual_length  # the keys say how many tokens of both leave
+        if res[0].shape[3] != res[1].shape[3]:
+            raise ValueError("KIVIFusedCache takes keys and values of one head_dim")
+        if res[0].shape[:2] != res[1].shape[:2] or res[1].shape[2] < n:
+            raise RuntimeError("keys and values of different heads, or fewer values than the overflow's keys")
         sides, args, mv = [], [], row_moves()
         for bits, tiers, r in ((cfg.key_bits, self._quant_keys, res[0]), (cfg.value_bits, self._quant_values, res[1])):
-            B, H, n_all, D = r.shape
-            n = n_all - cfg.residual_length
+            B, H, _, D = r.shape
             x, left = r[:, :, :n], r[:, :, n:]
             tier = tiers[layer_idx] if layer_idx in tiers else self._new_tier(x, bits)
             tier.reserve(n)
@@ -294,7 +298,7 @@ class KIVIFusedCache(KIVICache):
                 mv.copy(kept, left, left.shape[2])
             else:
                 kept = left.contiguous()
-            sides.append((tier, n, view, old, kept))
+            sides.append((tier, view, old, kept))
             args.append((x, B, H, D, n, dt, nat.KiviSide(
                 x.data_ptr(), x.stride(0) * e, x.stride(1) * e, x.stride(2) * e, tier.codes.data_ptr(),
                 tier.sc.data_ptr(), tier.ze.data_ptr(), tier.sc16.data_ptr(), tier.ze16.data_ptr(),
@@ -307,17 +311,17 @@ class KIVIFusedCache(KIVICache):
             nat.check(nat.load().akv_kivi_append(
                 arr, len(g), B, H, D, n, nat.dtype_code(x.dtype), cfg.group_size,
                 nat.DT_F16 if dt == torch.float16 else nat.DT_F32, nat.stream_of(x)), "KIVI append")
-        for tier, _, view, old, _ in sides:
+        for tier, view, old, _ in sides:
             if view is not None:
                 self._fill_view(tier, view, old, tier.n)
         mv.run()
-        (kt, nk, _, _, rk), (vt, nv, _, _, rv) = sides
-        kt.n, vt.n, kt.dirty, vt.dirty = kt.n + nk, vt.n + nv, 0, 0
+        (kt, _, _, rk), (vt, _, _, rv) = sides
+        kt.n, vt.n, kt.dirty, vt.dirty = kt.n + n, vt.n + n, 0, 0
         self._quant_keys[layer_idx], self._quant_values[layer_idx] = kt, vt
         self._dequant_keys_cache[layer_idx], self._dequant_values_cache[layer_idx] = kt, vt
         self._residual_keys[layer_idx], self._residual_values[layer_idx] = rk, rv
         return tuple(torch.cat([tier.dequantize(), kept], dim=2) if view is None else view
-                     for tier, _, view, _, kept in sides)
+                     for tier, view, _, kept in sides)
 
     @staticmethod
     def _new_view(tier: _Tier, had: int, n: int, left: torch.Tensor, dt: torch.dtype, mv: RowMoves):

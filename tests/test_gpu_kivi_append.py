@@ -49,3 +49,28 @@ def test_residual_autograd_and_refusal():
     bad = KIVIFusedCache(KIVIFusedConfig(key_bits=4, value_bits=3, residual_length=4))
     with pytest.raises(NotImplementedError):
         bad.update(k.detach(), k.detach(), 0)
+
+
+def test_the_keys_say_how_many_tokens_leave():
+    """A value more than keys stays in the values' residual window; fewer values than the overflow
+    needs, other heads and another head_dim are refused, before anything changes."""
+    from akv.baselines import KIVIFusedCache, KIVIFusedConfig, dequantize_rows, quantize_rows
+    announce("KIVI overflow of unequal keys and values")
+    g = torch.Generator(device="cuda").manual_seed(2)
+    r = lambda *s: torch.randn(s, generator=g, device="cuda").half()  # noqa: E731
+    cfg = dict(key_bits=2, value_bits=4, group_size=64, residual_length=16)
+    c = KIVIFusedCache(KIVIFusedConfig(**cfg))
+    k, v = r(1, 2, 30, 64), r(1, 2, 31, 64)
+    for step, (n, nk, nv) in enumerate(((14, 30, 31), (15, 31, 32))):
+        kv = (k, v) if step == 0 else (r(1, 2, 1, 64), r(1, 2, 1, 64))
+        got = c.update(*kv, 0)
+        k, v = (k, v) if step == 0 else (torch.cat([k, kv[0]], dim=2), torch.cat([v, kv[1]], dim=2))
+        for x, view, bits, m in ((k, got[0], 2, nk), (v, got[1], 4, nv)):
+            deq = dequantize_rows(*quantize_rows(x[:, :, :n], bits, 64), bits, 64, 64).view(1, 2, n, 64)
+            assert view.shape[2] == m and torch.equal(view, torch.cat([deq, x[:, :, n:]], dim=2))
+    for k, v, err in ((r(1, 2, 30, 64), r(1, 2, 30, 128), ValueError), (r(1, 2, 30, 64), r(1, 3, 30, 64), RuntimeError),
+                      (r(1, 2, 30, 64), r(1, 2, 13, 64), RuntimeError)):
+        c = KIVIFusedCache(KIVIFusedConfig(**cfg))
+        with pytest.raises(err):
+            c.update(k, v, 0)
+        assert not c._quant_keys and c._residual_keys[0] is k and c._residual_values[0] is v
