@@ -21,8 +21,8 @@ def test_fake_tensors(protect):
         layer = AKVLayer(hot_budget=64, protect=protect)
         for n in (5, 1, 2):
             k, v = layer.update(*(torch.empty(1, 2, n, 64, dtype=torch.float16, device="cuda") for _ in range(2)))
-    assert k.shape == v.shape == (1, 2, 8, 64) and k.device.type == "cuda"
-    assert layer._hot_positions.shape == (8,) and layer._total_len == 8
+        assert k.shape == v.shape == (1, 2, 8, 64) and k.device.type == "cuda"
+        assert layer._hot_positions.shape == (8,) and layer._total_len == 8
 
 
 def test_default_device_context_is_no_observer():
