@@ -293,15 +293,17 @@ def workspace(nbytes: int, device, zero_prefix: int = 0) -> torch.Tensor:
 
 
 def quant_pack(a: QuantArgs, like: torch.Tensor, what: str) -> None:
-    """``akv_quant_pack_ws`` on the current stream of ``like``'s device, with scratch for the
-    forms that ask for some (long K blocks)."""
+    """The quantizer on the current stream of ``like``'s device, with scratch for the calls that
+    ask for some (blocks and selections past 512 tokens; shorter ones never do, and are not
+    held up by asking)."""
     lib = load()
     ref = ctypes.byref(a)
-    nbytes = lib.akv_quant_workspace_bytes(ref)
-    if nbytes < 0:
-        check(lib.akv_quant_pack(ref, None), what)
-    ws = workspace(nbytes, like.device) if nbytes > 0 else None
-    check(lib.akv_quant_pack_ws(ref, ptr(ws), nbytes if ws is not None else 0, stream_of(like)), what)
+    nbytes = lib.akv_quant_workspace_bytes(ref) if a.block_t > 512 and a.n_sel > 512 else 0
+    if nbytes > 0:
+        ws = workspace(nbytes, like.device)
+        check(lib.akv_quant_pack_ws(ref, ptr(ws), nbytes, stream_of(like)), what)
+    else:  # none needed, or arguments that this call refuses
+        check(lib.akv_quant_pack(ref, stream_of(like)), what)
 
 
 def importance_update(a: ImportanceArgs, like: torch.Tensor, what: str) -> None:

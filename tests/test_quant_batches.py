@@ -26,6 +26,13 @@ def test_the_plan_knows_the_grid():
     assert _args(1, 1024 * 65536, 1024) == 0
 
 
+@pytest.mark.parametrize("n,T,scratch", [(512, 512, False), (513, 512, False), (512, 4096, False), (513, 513, True),
+                                         (4000, 4096, True), (4000, 32, False)])
+def test_short_blocks_need_no_scratch(n, T, scratch):
+    """The binding asks for scratch past 512 tokens of a block and of the selection only."""
+    assert (_args(2, n, T) > 0) == scratch
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n_out", [0, 1])
 def test_many_sequences(n_out):
