@@ -479,6 +479,16 @@ class AKVLayer:
             return torch.arange(self._hot_keys.shape[2], device=self._hot_keys.device)
         return self._positions
 
+    @_hot_positions.setter
+    def _hot_positions(self, positions: Optional[torch.Tensor]):
+        self._positions = positions
+
+    def __setstate__(self, state: dict):
+        """Layers saved while the positions were an attribute load too."""
+        self.__dict__.update(state)
+        if "_hot_positions" in state:
+            self._positions = self.__dict__.pop("_hot_positions")
+
     @property
     def _warm_positions(self) -> Optional[torch.Tensor]:
         """(N_warm,) int64, device: the warm tokens' positions in demotion order."""

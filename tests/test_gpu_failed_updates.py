@@ -172,3 +172,25 @@ def test_layer_crop(kw):
         if not fail.hit:
             break
     assert k > 4  # the packed tier loses tokens too
+
+
+def test_a_layer_saved_with_its_positions_goes_on():
+    """Copies of a layer, in the present form and with the positions as a host attribute, go on as it does."""
+    import copy
+
+    from akv.drop_in import AKVLayer
+    announce("copied layers")
+    chunks = _chunks((90, 1, 5), 1, 2, 64, torch.float16, 12)
+    for protect in (False, True):
+        layer = AKVLayer(warm_bits=4, hot_budget=64, protect=protect)
+        layer.update(*chunks[0])
+        a, b = copy.deepcopy(layer), AKVLayer.__new__(AKVLayer)
+        state = copy.deepcopy(layer.__dict__)
+        state.pop("_positions")
+        state["_hot_positions"] = layer._hot_positions.cpu()
+        b.__setstate__(state)
+        for c in chunks[1:]:
+            want = layer.update(*c)
+            for x in (a, b):
+                assert all(torch.equal(p, q) for p, q in zip(x.update(*c), want))
+                assert torch.equal(x._hot_positions, layer._hot_positions)
